@@ -34,7 +34,8 @@ extern "C" {
 #define PXFF_ENOTIMPL -3 /* unsupported parameter (e.g. odd 2J) */
 
 /* Launch-parameter knobs (process-wide), set by the autotuner:
- *   PXFF_TUNE_Z_CHUNKS              Z rows split into this many wavefront chunks per 64-atom tile (1..256)
+ *   PXFF_TUNE_Z_CHUNKS              Z rows split into at least this many wavefront chunks per 64-atom tile
+ *                                   (1..256; the launch takes more by a rule on 2J and the atoms)
  *   PXFF_TUNE_ACCUM_WAVES_PER_CU    persistent grid of the per-centre kernels = CUs x this (1..256)
  *   PXFF_TUNE_IMAGE_WAVES_PER_BLOCK wavefronts per workgroup of the per-image adjoint kernel (1, 2, 4)
  *   PXFF_TUNE_ACCUM_LDSADD          per-centre U_tot sums: 0 = per-group LDS partials, 1 = one LDS array

@@ -1,7 +1,7 @@
 """Autotuner for the launch parameters of the hot kernels.
 
 Knobs (``pxff_tune_set``, include/pxff.h):
-  * Z-row chunks per 64-atom tile of the Z kernel (wavefronts per tile),
+  * least Z-row chunks per 64-atom tile of the Z kernel (wavefronts per tile),
   * persistent-grid size of the per-centre kernels (wavefronts per CU),
   * how the per-centre kernels sum over images (register sums reduced once
     per centre, per-group LDS partials, LDS atomic adds, or LDS partials
@@ -21,7 +21,8 @@ from . import _native as nat
 from . import so4 as dso4
 
 Z_CHUNKS, ACCUM_WAVES_PER_CU, IMAGE_WAVES_PER_BLOCK, ACCUM_LDSADD = 0, 1, 2, 3
-CANDIDATES = {Z_CHUNKS: (4, 8, 16, 24, 32, 48, 64), ACCUM_WAVES_PER_CU: (4, 8, 16, 32, 64),
+# (the Z kernel takes at least its own rule's chunks: 16 stands for the rule)
+CANDIDATES = {Z_CHUNKS: (16, 64, 112), ACCUM_WAVES_PER_CU: (4, 8, 16, 32, 64),
               IMAGE_WAVES_PER_BLOCK: (1, 2, 4), ACCUM_LDSADD: (4, 0, 1, 2, 3)}
 CACHE = os.path.join(os.path.expanduser("~"), ".cache", "pyxtal_ff_amd", "tune.json")
 

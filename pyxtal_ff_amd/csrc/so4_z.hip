@@ -3,6 +3,7 @@
 // instantiated for every (l1, l2) pair of every supported 2J.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -15,30 +16,53 @@
 
 namespace pxff {
 
-// Z-group chunk tables per (device, 2J, normalisation, nchunks)
+// Row-group chunks per 64-atom tile (one wavefront each).  A wavefront runs
+// its chunk alone, so few chunks leave one long serial chain per wavefront
+// and, below some thousand atoms, most of the chip idle; more chunks than
+// keep the wavefronts resident only add partly filled rounds.  Measured, us
+// for Z and the B row partials, at 16 / 48 / 112 chunks: 2J = 8, 1 tile 107 /
+// 39 / 29, 13 tiles 123 / 46 / 37, 27 tiles 128 / 50 / 47, 64 tiles 129 / 66 /
+// 80 (48 is the one resident round of 12 wavefronts per CU there), 512 tiles
+// 584 / 476 / 500; 2J = 6, 16 tiles 38 / 20 / 20, 64 tiles 48 / 28 / 31.  At
+// 2J = 10 the groups are four times as long: 128 chunks at every size (64
+// tiles 345 / 272 / 236, 1 tile 306 / 144 / 74).  The tuning knob can raise
+// the count, not lower it.
+constexpr int ZCH_SMALL_TILES = 24;
+static int zchunk_rule(int twol, int ntiles) {
+    if (twol >= 10) return 128;
+    return ntiles <= ZCH_SMALL_TILES ? 112 : 48;
+}
+
+// Z-group chunk tables per (device, 2J, normalisation, nchunks).  The first
+// call for a 2J builds the tables of every chunk count the rule can choose,
+// so that a later call of another size allocates nothing (it may run under
+// stream capture).
 static std::mutex g_chunk_mutex;
 static std::map<std::tuple<int, int, int>, int *> g_chunks;
-static int get_zchunks(int twol, int norm, int nch, const int **out) {
+static int get_zchunks(int twol, int norm, int nch, int nzgroups, const int **out) {
     int dev = 0;
     PXFF_HIP_CHECK(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_chunk_mutex);
-    auto key = std::make_tuple(dev, twol * 2 + (norm ? 1 : 0), nch);
-    auto it = g_chunks.find(key);
-    if (it != g_chunks.end()) {
-        *out = it->second;
-        return 0;
+    const int tab = twol * 2 + (norm ? 1 : 0);
+    auto it = g_chunks.find(std::make_tuple(dev, tab, nch));
+    if (it == g_chunks.end()) {
+        So4HostTables t;
+        if (!build_so4_tables(twol, norm, t)) {
+            set_error("unsupported 2J");
+            return PXFF_ENOTIMPL;
+        }
+        for (int n : {nch, std::min(zchunk_rule(twol, 1), nzgroups), std::min(zchunk_rule(twol, 1 << 20), nzgroups)}) {
+            const auto key = std::make_tuple(dev, tab, n);
+            if (g_chunks.count(key)) continue;
+            const std::vector<int> c = chunk_zgroups(t, n);
+            int *d = nullptr;
+            PXFF_HIP_CHECK(hipMalloc((void **)&d, c.size() * sizeof(int)));
+            PXFF_HIP_CHECK(hipMemcpy(d, c.data(), c.size() * sizeof(int), hipMemcpyHostToDevice));
+            g_chunks[key] = d;
+        }
+        it = g_chunks.find(std::make_tuple(dev, tab, nch));
     }
-    So4HostTables t;
-    if (!build_so4_tables(twol, norm, t)) {
-        set_error("unsupported 2J");
-        return PXFF_ENOTIMPL;
-    }
-    std::vector<int> c = chunk_zgroups(t, nch);
-    int *d = nullptr;
-    PXFF_HIP_CHECK(hipMalloc((void **)&d, c.size() * sizeof(int)));
-    PXFF_HIP_CHECK(hipMemcpy(d, c.data(), c.size() * sizeof(int), hipMemcpyHostToDevice));
-    g_chunks[key] = d;
-    *out = d;
+    *out = it->second;
     return 0;
 }
 
@@ -322,9 +346,9 @@ extern "C" int pxff_so4_zb(const pxff_so4_params *p, int64_t natoms, const doubl
     if ((rc = get_so4_tables(p->twol, p->normalize_u, &T))) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int ntiles = (int)((natoms + 63) / 64);
-    const int nch = std::min(tune_value(PXFF_TUNE_Z_CHUNKS), T->nzgroups);
+    const int nch = std::min(std::max(tune_value(PXFF_TUNE_Z_CHUNKS), zchunk_rule(p->twol, ntiles)), T->nzgroups);
     const int *zch = nullptr;
-    if ((rc = get_zchunks(p->twol, p->normalize_u, nch, &zch))) return rc;
+    if ((rc = get_zchunks(p->twol, p->normalize_u, nch, T->nzgroups, &zch))) return rc;
     const int grid = 8 * ((ntiles + 7) / 8) * ((nch + 3) / 4);
     // B row partials after Z in the same buffer
     double *bpart = d_b ? d_z + 2 * (size_t)ntiles * 64 * T->nz : nullptr;
