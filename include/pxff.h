@@ -474,6 +474,31 @@ int pxff_so3_deidrj_counted(const pxff_so3_params *p, int64_t cap, const int64_t
                             const int64_t *d_atom_z, const double *d_G, const double *d_rq, const double *d_lnorm,
                             const double *d_a, const double *d_radial, double *d_dedr, void *stream);
 
+/* The energy + force path on the m >= 0 half (lmax <= 6): the radial factors,
+ * weights and dE/dP are real, so C_l,-m = (-1)^m conj(C_lm) for the expansion
+ * and for A.  Half arrays are complex [natoms][nmax][(lmax+1)(lmax+2)/2],
+ * entry l(l+1)/2 + m; values equal the m >= 0 entries of the full arrays.
+ *   pxff_so3_forward_half: expansion d_ct, power spectrum d_x (as
+ *     pxff_so3_power) and the radial store d_radial (16-byte aligned, as
+ *     pxff_so3_ctot_pairs: d_img_rev, d_work, cap and d_table as there; with
+ *     d_img_rev NULL, d_work and d_table NULL too, every image's integrals are
+ *     evaluated by the quadrature).
+ *   pxff_so3_adjoint_a_half: pxff_so3_adjoint_a on half arrays.
+ *   pxff_so3_deidrj_half: pxff_so3_deidrj (d_count NULL) or
+ *     pxff_so3_deidrj_counted (nimg an image capacity) from half A and the
+ *     forward's d_radial. */
+int pxff_so3_forward_half(const pxff_so3_params *p, int64_t natoms, const int64_t *d_img_start,
+                          const int64_t *d_img_j, const double *d_img_r, const int64_t *d_img_rev,
+                          const int64_t *d_atom_z, const double *d_G, const double *d_rq, const double *d_lnorm,
+                          double *d_ct, double *d_x, double *d_radial, int64_t *d_work, int64_t cap,
+                          const double *d_table, void *stream);
+int pxff_so3_adjoint_a_half(const pxff_so3_params *p, int64_t natoms, const double *d_ct, const double *d_beta,
+                            double *d_a, void *stream);
+int pxff_so3_deidrj_half(const pxff_so3_params *p, int64_t nimg, const int64_t *d_count, const int64_t *d_img_atom,
+                         const int64_t *d_img_j, const double *d_img_r, const int64_t *d_atom_z,
+                         const double *d_lnorm, const double *d_a, const double *d_radial, double *d_dedr,
+                         void *stream);
+
 /* Plain path: dP/dr per image [nimg*ncoef*3] (then pxff_so4_rows builds the
  * reference's dxdr / rdxdr rows, whose row rules SO3.py:243-265 shares). */
 int pxff_so3_dpdr(const pxff_so3_params *p, int64_t nimg, const int64_t *d_img_atom, const int64_t *d_img_j,

@@ -109,7 +109,7 @@ __device__ inline void so3_cutoff(int id, double r, double rc, double &f, double
     switch (id) {
     case 1: {
         double s, c;
-        sincos(M_PI * r / rc, &s, &c);
+        sincospi(x, &s, &c);  // no reduction of large arguments: fewer registers than sincos(pi x)
         f = 0.5 * (c + 1.0);
         df = -0.5 * M_PI / rc * s;
         return;
@@ -811,6 +811,48 @@ __global__ __launch_bounds__(64) void so3_radial_tab_kernel(So3Args a, const int
     }
 }
 
+// The radial store from the table without the |r| order, for small lists: one
+// wavefront per image with rev(e) >= e, lane j on the functions 2j and
+// 2j + 1, both images' rows written.  Every pair reads its interval's
+// coefficients (8 KB at 6/6) through L2, which the sorted walk avoids, but
+// the three launches of the sort (24 us, its one-workgroup scan 13 of them)
+// and the serial walk of 64 pairs per wavefront are gone.  Radial store,
+// expansion and power spectrum together, direct / sorted, us: 6/6, 2.0k
+// images 13 / 48, 20k 25 / 54, 63k 52 / 65; 3/4, 10k 14 / 45, 63k 38 / 56.
+constexpr int64_t SO3_RDIRECT = 65536;  // image capacity up to which it is used
+template <int NMAX>
+__global__ __launch_bounds__(256) void so3_radial_direct_kernel(So3Args a, int64_t natoms,
+                                                                const int64_t *__restrict__ img_start,
+                                                                const double *__restrict__ img_r,
+                                                                const int64_t *__restrict__ img_rev,
+                                                                const double *__restrict__ tab, int nk, double h,
+                                                                double *__restrict__ rad) {
+    const int64_t e = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (e >= img_start[natoms]) return;  // the grid covers the image capacity
+    const int64_t re = img_rev[e];
+    if (re < e) return;
+    const double x0 = img_r[3 * e], y0 = img_r[3 * e + 1], z0 = img_r[3 * e + 2];
+    const double u = sqrt(x0 * x0 + y0 * y0 + z0 * z0) / h;
+    int k = (int)u;
+    k = k < 0 ? 0 : (k >= nk ? nk - 1 : k);
+    const double t = 2.0 * (u - k) - 1.0;
+    const int nf = (a.lmax + 1) * 2 * NMAX;
+    for (int f0 = 2 * (threadIdx.x & 63); f0 < nf; f0 += 128) {
+        const double2 *src = reinterpret_cast<const double2 *>(tab + ((size_t)k * nf + f0) * SO3_TNP);
+        double2 c[SO3_TNP];
+#pragma unroll
+        for (int q = 0; q < SO3_TNP; q++) c[q] = src[q];
+        double v0 = c[SO3_TNP / 2 - 1].y, v1 = c[SO3_TNP - 1].y;
+#pragma unroll
+        for (int q = SO3_TDEG - 1; q >= 0; q--) {
+            v0 = fma(v0, t, q & 1 ? c[q / 2].y : c[q / 2].x);
+            v1 = fma(v1, t, q & 1 ? c[SO3_TNP / 2 + q / 2].y : c[SO3_TNP / 2 + q / 2].x);
+        }
+        *reinterpret_cast<double2 *>(rad + (size_t)e * nf + f0) = make_double2(v0, v1);
+        if (re != e) *reinterpret_cast<double2 *>(rad + (size_t)re * nf + f0) = make_double2(v0, v1);
+    }
+}
+
 // The quadrature for the image pairs in |r| order, one lane per pair and
 // one wavefront per 64 pairs.  The rows are written one l at a time through
 // LDS, 2 nmax doubles of every pair's row at once, so that a store
@@ -1034,6 +1076,7 @@ __device__ __forceinline__ cd so3_zpow(cd z, int am) {
     return w;
 }
 
+// The expansion at lmax = 7 (so3_expand_kernel holds lmax <= 6):
 // ctot[i][n][l][m] = sum_e c_e,nlm = sum_e w norm_l ex fc I_nl Y_lm (SO3.py:
 // 205-226) with the radial integrals I_nl read from the radial store.  One
 // wavefront per centre (persistent), one lane per (l, m), (lmax + 1)^2 <= 64:
@@ -1152,193 +1195,435 @@ __global__ __launch_bounds__(64) void so3_ctot_lm_kernel(So3Args a, int64_t nato
     }
 }
 
-// A double moved across lanes by one DPP control (two 32-bit moves);
-// lanes of rows outside ROWMASK read 0.
-template <int CTRL, int ROWMASK = 0xf>
-__device__ inline double dpp_f64(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWMASK, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWMASK, 0xf, false);
-    return __hiloint2double(hi, lo);
+// ------------------------------------------- lanes over (l, pairs of m >= 0)
+// The radial factors, weights and dE/dP are real, so the expansion and its
+// adjoint have C_l,-m = (-1)^m conj(C_lm) exactly: the m >= 0 half carries
+// everything (sums over m are Re(m = 0) + 2 sum over m > 0).  The per-image
+// kernels below give a lane the two orders m = 2h and 2h + 1 of one l
+// (l / 2 + 1 lanes per l, 16 lanes for l <= 6), so a wavefront works on four
+// images at once, one per row of 16 lanes: each radial integral read from
+// LDS feeds two orders, and sums over the lanes are sums over one row (DPP
+// moves only).
+//
+// Y_lm = Q(t) z^m, t = cos theta = u_z, z = u_x + i u_y for the unit vector u:
+// Q = Pbar_l^m / sin^m theta is a polynomial of degree l - m, its
+// coefficients g_so3_legq[l][m][j] (of t^j) built once per device.
+constexpr int SO3_QL = 8;  // l, m < 8, degree <= 7
+__device__ double g_so3_legq[SO3_QL * SO3_QL * SO3_QL];
+
+// The lane's l and first order m0 = 2h from its place gl in the row; l = 0,
+// on = false past lmax.
+struct So3Lane {
+    int l, m0;
+    bool on0, on1;
+};
+__device__ __forceinline__ So3Lane so3_lane(int gl, int lmax) {
+    So3Lane v;
+    int l = 0, c = 0;
+    while (gl >= c + l / 2 + 1) {
+        c += l / 2 + 1;
+        l++;
+    }
+    v.on0 = l <= lmax;
+    v.l = v.on0 ? l : 0;
+    v.m0 = v.on0 ? 2 * (gl - c) : 0;
+    v.on1 = v.on0 && v.m0 + 1 <= v.l;
+    return v;
 }
 
-// Sum over the 64 lanes of a wavefront, complete in lane 63: pairs and
-// quads (quad_perm), half rows and rows (row_half_mirror, row_mirror), then
-// row 0 into row 1 and row 2 into row 3 (row_bcast:15), rows 0-1 into rows
-// 2-3 (row_bcast:31).  Vector moves only, no LDS round trips.
-__device__ inline void wave_sum3_lane63(double &a, double &b, double &c) {
-    a += dpp_f64<0xb1>(a); b += dpp_f64<0xb1>(b); c += dpp_f64<0xb1>(c);
-    a += dpp_f64<0x4e>(a); b += dpp_f64<0x4e>(b); c += dpp_f64<0x4e>(c);
-    a += dpp_f64<0x141>(a); b += dpp_f64<0x141>(b); c += dpp_f64<0x141>(c);
-    a += dpp_f64<0x140>(a); b += dpp_f64<0x140>(b); c += dpp_f64<0x140>(c);
-    a += dpp_f64<0x142, 0xa>(a); b += dpp_f64<0x142, 0xa>(b); c += dpp_f64<0x142, 0xa>(c);
-    a += dpp_f64<0x143, 0xc>(a); b += dpp_f64<0x143, 0xc>(b); c += dpp_f64<0x143, 0xc>(c);
+// Coefficients of Q of (l, m); zero if off.
+template <int NQ>
+__device__ __forceinline__ void so3_load_q(bool on, int l, int m, double (&q)[NQ]) {
+#pragma unroll
+    for (int j = 0; j < NQ; j++) q[j] = on ? g_so3_legq[(l * SO3_QL + m) * SO3_QL + j] : 0.0;
 }
 
-// Adjoint dE/dr per image, one lane per (l, m) with l <= lmax + 1
-// ((lmax + 2)^2 <= 64): flat over images, a wavefront takes 64 consecutive
-// images (their scalars staged in LDS, one lane each) and runs them one at
-// a time.  Per image every lane forms its Y_lm (rows <= lmax + 1) as
-// Q(cos theta) z^|m| (so3_legendre_poly, built once per lane) into a
-// 64-entry LDS table, from which the lanes with l <= lmax read the
-// Y_{l+-1, m'} of the covariant gradient (SO3.py:649-674; its coefficients
-// depend on (l, m) only and are held in registers).  With
-// alpha = sum_n I_nl A_nlm and beta = sum_n dI_nl A_nlm (A of the image's
-// centre, reloaded when the centre changes),
-//   dE/dr_k = sum_lm  cu rhat_k Re(conj(alpha) Y) + cv Re(conj(alpha) dY/dr_k)
-//                   + cv rhat_k Re(conj(beta) Y),
-// cu = w norm_l ex (dfc - 2 alpha R fc), cv = w norm_l ex fc: the same sums
-// as so3_image_kernel<SO3_ADJOINT> in another order, reduced over the
-// lanes with DPP moves (wave_sum3_lane63).
-// staged: t, Re z, Im z, (unused), R, w ex fc, w ex (dfc - 2 a R fc), rhat
-constexpr int SO3_ADJ_NST = 10;
+// x summed over rows r and r ^ 1 in even rows, y in odd rows (permlane16),
+// and over the lower and upper 32 lanes likewise (permlane32).
+__device__ __forceinline__ double so3_fold16(double x, double y) {
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double so3_fold32(double x, double y) {
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// Expansion, lmax <= 6: ctot[i][n][l][m] = sum_e w norm_l ex fc I_nl Y_lm
+// (SO3.py:205-226) from the radial store, and optionally the power spectrum
+// P[i][tril(a, b)][l] = Re sum_m C_a conj(C_b) (SO3.py:228, 259) of the same
+// centre while its sums are in LDS.  One workgroup of two wavefronts per
+// centre, eight images at a time (a row of 16 lanes each).  The per-image
+// scalars, powers of z and I_nl rows of up to SO3_CH images are staged in
+// LDS; the eight rows' sums are folded with lane swaps (12 + 6 of them for
+// nmax = 6) and the two wavefronts' through LDS, in a fixed order.
+// half: out is [natoms][nmax][(lmax+1)(lmax+2)/2] (m >= 0, entry l(l+1)/2 + m);
+// else the full [natoms][nmax][lmax+1][2lmax+1], entries |m| > l zero.
+// 12,000 centres of 34 images at 6/6, with P: 86 us, 273 MB of radial rows
+// fetched at 3.2 TB/s (its forerunner, one wavefront per centre with a lane
+// per (l, m) and m < 0, took 104 us and the power spectrum another 53 us).
+// Held at three wavefronts per SIMD for nmax <= 6 (210 registers unheld).
+constexpr int SO3_CH = 40;  // images per chunk (at 6/6 23 KB of LDS, seven workgroups per CU)
+constexpr int SO3_CT = 128;
 template <int NMAX>
-__global__ __launch_bounds__(64) void so3_deidrj_lm_kernel(So3Args a, int64_t nimg, const int64_t *__restrict__ img_atom,
+__global__ __launch_bounds__(SO3_CT) __attribute__((amdgpu_waves_per_eu(NMAX <= 6 ? 3 : 2))) void so3_expand_kernel(
+                                                            So3Args a, int64_t natoms, const int64_t *__restrict__ img_start,
                                                             const int64_t *__restrict__ img_j,
                                                             const double *__restrict__ img_r,
                                                             const int64_t *__restrict__ atom_z,
-                                                            const double *__restrict__ A,
-                                                            const double *__restrict__ rad, double *__restrict__ dedr,
-                                                            const int64_t *__restrict__ d_count) {
-    __shared__ double stg[SO3_ADJ_NST][64];
-    __shared__ int64_t s_at[64];
-    __shared__ cd ysh[64];
+                                                            const double *__restrict__ rad, double *__restrict__ out,
+                                                            int half, double *__restrict__ pout) {
+    constexpr int LM = 7, NHM = LM * (LM + 1) / 2;
+    __shared__ double s_t[SO3_CH], s_wf[SO3_CH];
+    __shared__ cd s_z[SO3_CH][LM];
+    __shared__ double rI[SO3_CH * LM * NMAX];  // [image][l][n]
+    __shared__ cd cs[2][NMAX * NHM];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int L = a.lmax + 1, NH = L * (L + 1) / 2;
+    const So3Lane ln = so3_lane(lane & 15, a.lmax);
+    const int64_t c = blockIdx.x;
+    const int64_t s0 = img_start[c], s1 = img_start[c + 1];
+    double v[NMAX][4];  // Re, Im of m0, Re, Im of m0 + 1
+#pragma unroll
+    for (int n = 0; n < NMAX; n++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[n][k] = 0.0;
+    for (int64_t b0 = s0; b0 < s1; b0 += SO3_CH) {
+        const int nb = (int)(s1 - b0 < SO3_CH ? s1 - b0 : SO3_CH);
+        __syncthreads();  // the previous chunk's stage has been read
+        if (wv == 0) {
+            // one lane per image (the second wavefront copies the rows
+            // meanwhile; the cutoff and the exponential are the kernel's
+            // register peak, so nothing else is live here)
+            if (lane < nb) {
+                So3Img mi;
+                load_image(a, true, b0 + lane, c, img_j, img_r, atom_z, mi);
+                s_t[lane] = mi.z / mi.R;
+                s_wf[lane] = mi.w * mi.ex * mi.fc;
+                const cd z = cmake(mi.x / mi.R, mi.y / mi.R);
+                cd p = cmake(1.0, 0.0);
+#pragma unroll
+                for (int m = 0; m < LM; m++) {
+                    s_z[lane][m] = p;
+                    p = cmul(p, z);
+                }
+            }
+        } else {
+            // the first nmax of each 2 nmax-row of the radial store
+            constexpr int RB = 14;
+            const double *rb = rad + (size_t)b0 * L * 2 * NMAX;
+            const int nri = nb * L * NMAX;
+            for (int k0 = 0; k0 < nri; k0 += 64 * RB) {
+                double t[RB];
+#pragma unroll
+                for (int u = 0; u < RB; u++) {
+                    const int k = k0 + u * 64 + lane;
+                    const int row = k / NMAX;
+                    t[u] = k < nri ? rb[(size_t)row * 2 * NMAX + (k - row * NMAX)] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < RB; u++) {
+                    const int k = k0 + u * 64 + lane;
+                    if (k < nri) rI[k] = t[u];
+                }
+            }
+        }
+        __syncthreads();
+        asm volatile("" ::: "memory");  // the lane's coefficients are loaded here, not held over the staging
+        double q0[LM], q1[LM];
+        so3_load_q(ln.on0, ln.l, ln.m0, q0);
+        so3_load_q(ln.on1, ln.l, ln.m0 + 1, q1);
+        const double lnorm = ln.on0 ? a.lnorm[ln.l] : 0.0;
+#pragma unroll 1
+        for (int b = tid >> 4; b < nb; b += SO3_CT / 16) {
+            const double t = s_t[b], wf = s_wf[b] * lnorm;
+            double p0 = q0[LM - 1], p1 = q1[LM - 1];
+#pragma unroll
+            for (int j = LM - 2; j >= 0; j--) {
+                p0 = fma(p0, t, q0[j]);
+                p1 = fma(p1, t, q1[j]);
+            }
+            const cd z0 = s_z[b][ln.m0], z1 = s_z[b][ln.m0 + 1 < LM ? ln.m0 + 1 : LM - 1];
+            p0 *= wf;
+            p1 *= wf;
+            const double y0 = p0 * z0.re, y1 = p0 * z0.im, y2 = p1 * z1.re, y3 = p1 * z1.im;
+            const double *ri = rI + (b * L + ln.l) * NMAX;
+#pragma unroll
+            for (int n = 0; n < NMAX; n++) {
+                const double in = ri[n];
+                v[n][0] = fma(in, y0, v[n][0]);
+                v[n][1] = fma(in, y1, v[n][1]);
+                v[n][2] = fma(in, y2, v[n][2]);
+                v[n][3] = fma(in, y3, v[n][3]);
+            }
+        }
+    }
+    // fold the four rows: row r then holds component r of (Re m0, Im m0,
+    // Re m1, Im m1)
+    const int row = lane >> 4, m = ln.m0 + (row >> 1);
+    const bool st = row >> 1 ? ln.on1 : ln.on0;
+#pragma unroll
+    for (int n = 0; n < NMAX; n++) {
+        const double w = so3_fold32(so3_fold16(v[n][0], v[n][1]), so3_fold16(v[n][2], v[n][3]));
+        if (st) reinterpret_cast<double *>(&cs[wv][n * NH + ln.l * (ln.l + 1) / 2 + m])[row & 1] = w;
+    }
+    __syncthreads();
+    for (int k = tid; k < NMAX * NH; k += SO3_CT) cs[0][k] = cadd(cs[0][k], cs[1][k]);
+    __syncthreads();
+    if (half) {
+        cd *oc = reinterpret_cast<cd *>(out) + (size_t)c * NMAX * NH;
+        for (int k = tid; k < NMAX * NH; k += SO3_CT) oc[k] = cs[0][k];
+    } else {
+        const int M2 = 2 * a.lmax + 1;
+        cd *oc = reinterpret_cast<cd *>(out) + (size_t)c * NMAX * L * M2;
+        for (int k = tid; k < NMAX * L * M2; k += SO3_CT) {
+            const int nl = k / M2, l = nl % L, mm = k - nl * M2 - a.lmax, am = mm < 0 ? -mm : mm;
+            cd z = cmake(0.0, 0.0);
+            if (am <= l) {
+                z = cs[0][nl / L * NH + l * (l + 1) / 2 + am];
+                if (mm < 0) z = (am & 1) ? cmake(-z.re, z.im) : cmake(z.re, -z.im);
+            }
+            oc[k] = z;
+        }
+    }
+    if (pout == nullptr) return;
+    const int nc = NMAX * (NMAX + 1) / 2 * L;
+    double *po = pout + (size_t)c * nc;
+    for (int k = tid; k < nc; k += SO3_CT) {
+        const int tri = k / L, l = k - tri * L;
+        int aa = 0;
+        while ((aa + 1) * (aa + 2) / 2 <= tri) aa++;
+        const cd *ca = cs[0] + aa * NH + l * (l + 1) / 2, *cb = cs[0] + (tri - aa * (aa + 1) / 2) * NH + l * (l + 1) / 2;
+        double s = 0.0;
+        for (int mm = 1; mm <= l; mm++) s += cdotre(ca[mm], cb[mm]);
+        po[k] = fma(2.0, s, cdotre(ca[0], cb[0]));
+    }
+}
+
+// The half-layout A[i][n][hm] = sum_n' S[n][n'][l] C[i][n'][hm] (so3_adj_a_kernel
+// on the m >= 0 entries): 0.31 of the bytes of the full layout at lmax = 6,
+// 19 us for 12,000 centres against 35 us.
+template <int NMAX>
+__global__ __launch_bounds__(256) void so3_adj_a_half_kernel(int64_t natoms, int lmax, const double *__restrict__ ct,
+                                                             const double *__restrict__ beta, double *__restrict__ A) {
+    constexpr int NTRI = NMAX * (NMAX + 1) / 2;
+    const int L = lmax + 1, NH = L * (L + 1) / 2;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= natoms * NH) return;
+    const int64_t i = t / NH;
+    const int k = (int)(t - i * NH);
+    int l = 0;
+    while ((l + 1) * (l + 2) / 2 <= k) l++;
+    const cd *c = reinterpret_cast<const cd *>(ct) + (size_t)i * NMAX * NH + k;
+    cd *o = reinterpret_cast<cd *>(A) + (size_t)i * NMAX * NH + k;
+    cd cv[NMAX];
+#pragma unroll
+    for (int np = 0; np < NMAX; np++) cv[np] = c[(size_t)np * NH];
+    const double *b = beta + (size_t)i * NTRI * L + l;
+#pragma unroll
+    for (int n = 0; n < NMAX; n++) {
+        cd s = cmake(0, 0);
+#pragma unroll
+        for (int np = 0; np < NMAX; np++) {
+            const int hi = n > np ? n : np, lo = n > np ? np : n;
+            double f = b[(hi * (hi + 1) / 2 + lo) * L];
+            if (np == n) f *= 2.0;
+            s = cadd(s, cscale(cv[np], f));
+        }
+        o[(size_t)n * NH] = s;
+    }
+}
+
+// A double moved within its row by one DPP control.
+template <int CTRL>
+__device__ __forceinline__ double so3_dpp(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Adjoint dE/dr per image, lmax <= 6, lanes over (l, pairs of m >= 0), four
+// images at a time.  With A' = norm_l (1 or 2) A, alpha = sum_n I_nl A'_nlm
+// and beta = sum_n dI_nl A'_nlm, an image's energy derivative needs
+//   S   = sum_lm Q Re(conj(cu alpha + cv beta) z^m)       (along u),
+//   G_x = sum m Q Re(conj(alpha) z^(m-1)),  G_y = sum m Q Re(conj(alpha) i z^(m-1)),
+//   G_z = sum Q' Re(conj(alpha) z^m)
+// (G: the gradient of sum Re(conj(alpha) Y) as a function of u, whose
+// tangential part over R is the gradient the reference forms from Y_{l+-1},
+// SO3.py:649-674):  dE/dr = S u + (cv / R) (G - u (u . G)),
+// cu = w ex (dfc - 2 alpha R fc), cv = w ex fc.  The four sums over a row of
+// 16 lanes take 22 moves and 5 additions (halves of the row keep two sums,
+// quads one), and go to LDS; after 32 images one lane each combines them and
+// writes dE/dr in place.  The radial rows, the kernel's main traffic, are
+// copied to LDS 8 images at a time, the next 8 in flight in registers.
+// A row of lanes takes consecutive images, so it keeps A of one centre for
+// several of them.  One batch per wavefront: in a loop over batches the
+// constants of the cutoff and the exponential are held in registers across
+// it (256 of them and one wavefront per SIMD).
+// 407k images at 6/6: 111 us, 2.5 TB/s of radial rows, two wavefronts per
+// SIMD; 5.8k images at 3/4: 11 us (its forerunner with a lane per (l, m), a Y
+// table and 64-lane sums: 215 and 56 us).
+constexpr int SO3_AB = 32;  // images per batch, SO3_AB / 4 per row of lanes
+template <int NMAX>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NMAX <= 4 ? 3 : 2))) void so3_deidrj_half_kernel(
+                                                             So3Args a, int64_t nimg, const int64_t *__restrict__ img_atom,
+                                                             const int64_t *__restrict__ img_j,
+                                                             const double *__restrict__ img_r,
+                                                             const int64_t *__restrict__ atom_z,
+                                                             const double *__restrict__ A, int half,
+                                                             const double *__restrict__ rad, double *__restrict__ dedr,
+                                                             const int64_t *__restrict__ d_count) {
+    constexpr int LM = 7, PER = SO3_AB / 4;
+    constexpr int NFM = LM * 2 * NMAX;             // doubles of a radial row (lmax = 6)
+    constexpr int NLD = (4 * NFM + 63) / 64;       // 16-byte loads per lane for 8 rows
+    __shared__ double s_u[3][SO3_AB], s_cu[SO3_AB], s_cv[SO3_AB], s_ir[SO3_AB];
+    __shared__ cd s_z[SO3_AB][LM];
+    __shared__ int64_t s_at[SO3_AB];
+    __shared__ double s_sum[SO3_AB][4];
+    __shared__ __attribute__((aligned(16))) double s_row[8 * (NFM + 2)];
     if (d_count) {
         const int64_t c = *d_count;
         nimg = c < nimg ? c : nimg;
     }
-    const int L = a.lmax + 1;
-    const int M2 = 2 * a.lmax + 1;
-    const int lane = threadIdx.x;
-    const int64_t base = (int64_t)blockIdx.x * 64;
-    if (base >= nimg) return;  // a launch over an image capacity
-    const int nb = (int)((nimg - base) < 64 ? (nimg - base) : 64);
-    int l = 0;
-    while ((l + 1) * (l + 1) <= lane) l++;
-    const int m = lane - l * l - l;
-    const bool ylane = lane < (L + 1) * (L + 1);  // rows 0..lmax+1
-    const bool act = lane < L * L;                // rows 0..lmax
-    const int am = m < 0 ? -m : m;
-    double q[SO3_QK];  // Y rows l <= lmax + 1 <= 7
-    so3_legendre_poly(l, am, ylane, q);
-    const double msg = (m < 0 && (am & 1)) ? -1.0 : 1.0, imsg = m < 0 ? -msg : msg;
-    // covariant gradient coefficients of the lane's (l, m) and the lanes of
-    // the Y values they multiply (-1: term absent)
-    const double dl = l, dm = m;
-    double gc[6] = {0, 0, 0, 0, 0, 0};
-    int gi[6] = {-1, -1, -1, -1, -1, -1};
-    auto lidx = [&](int ll, int mm) { return ll * ll + ll + mm; };
-    if (act && l > 0) {
-        gc[0] = -sqrt(((dl + 1) * (dl + 1) - dm * dm) / (2 * dl + 1) / (2 * dl + 3)) * dl;  // x0: Y(l+1, m)
-        gi[0] = lidx(l + 1, m);
-        if (am <= l - 1) {
-            gc[1] = sqrt((dl * dl - dm * dm) / (2 * dl - 1) / (2 * dl + 1)) * (dl + 1);      // x0: Y(l-1, m)
-            gi[1] = lidx(l - 1, m);
-        }
-        gc[2] = -sqrt((dl + dm + 1) * (dl + dm + 2) / 2 / (2 * dl + 1) / (2 * dl + 3)) * dl;  // xp: Y(l+1, m+1)
-        gi[2] = lidx(l + 1, m + 1);
-        if (abs(m + 1) <= l - 1) {
-            gc[3] = -sqrt((dl - dm - 1) * (dl - dm) / 2 / (2 * dl - 1) / (2 * dl + 1)) * (dl + 1);  // xp: Y(l-1, m+1)
-            gi[3] = lidx(l - 1, m + 1);
-        }
-        gc[4] = -sqrt((dl - dm + 1) * (dl - dm + 2) / 2 / (2 * dl + 1) / (2 * dl + 3)) * dl;  // xm: Y(l+1, m-1)
-        gi[4] = lidx(l + 1, m - 1);
-        if (abs(m - 1) <= l - 1) {
-            gc[5] = -sqrt((dl + dm - 1) * (dl + dm) / 2 / (2 * dl - 1) / (2 * dl + 1)) * (dl + 1);  // xm: Y(l-1, m-1)
-            gi[5] = lidx(l - 1, m - 1);
-        }
+    const int64_t b0 = (int64_t)blockIdx.x * SO3_AB;
+    if (b0 >= nimg) return;  // a launch over an image capacity
+    const int nb = (int)(nimg - b0 < SO3_AB ? nimg - b0 : SO3_AB);
+    const int lane = threadIdx.x, g = lane >> 4, gl = lane & 15;
+    const int L = a.lmax + 1, nf = L * 2 * NMAX, RS = nf + 2;
+    const So3Lane ln = so3_lane(gl, a.lmax);
+    const double sc0 = ln.on0 ? a.lnorm[ln.l] * (ln.m0 ? 2.0 : 1.0) : 0.0, sc1 = ln.on1 ? 2.0 * a.lnorm[ln.l] : 0.0;
+    const double dm0 = ln.m0, dm1 = ln.m0 + 1;
+    const int iz = ln.m0 + 1 < LM ? ln.m0 + 1 : LM - 1, ip = ln.m0 > 0 ? ln.m0 - 1 : 0;
+    const int NH = L * (L + 1) / 2, M2 = 2 * a.lmax + 1;
+    const int astep = half ? NH : L * M2, asize = NMAX * astep;
+    const int aoff = half ? ln.l * (ln.l + 1) / 2 + ln.m0 : ln.l * M2 + a.lmax + ln.m0;
+    // the lane's share of 8 radial rows: unit k of row pair s = k / nf
+    int gof[NLD], lof[NLD];
+#pragma unroll
+    for (int u = 0; u < NLD; u++) {
+        const int k = u * 64 + lane, s = k / nf, o = k - s * nf;  // o in 16-byte units over two rows
+        const bool in = k < 4 * nf;
+        const int r2 = 2 * o >= nf ? 1 : 0;
+        gof[u] = in ? s * PER * nf + 2 * o : -1;
+        lof[u] = in ? (s * 2 + r2) * RS + 2 * o - r2 * nf : 0;
     }
-    const double lnorm = act ? a.lnorm[l] : 0.0;
-    const double r2 = 1.0 / sqrt(2.0);
-    {
-        const int64_t e = base + lane;
+    double2 pre[NLD];
+    auto fetch = [&](int it) {
+        // images b0 + s PER + it, + 1 of every row s
+        const double *src = rad + (size_t)(b0 + it) * nf;
+        const int last = (nb - it) * nf;  // doubles available from src
+#pragma unroll
+        for (int u = 0; u < NLD; u++)
+            pre[u] = gof[u] >= 0 && gof[u] < last ? *reinterpret_cast<const double2 *>(src + gof[u]) : make_double2(0.0, 0.0);
+    };
+    if (lane < SO3_AB) {
+        const int64_t e = b0 + lane;
         const bool ok = lane < nb;
         So3Img mi;
         load_image(a, ok, e, ok ? img_atom[e] : 0, img_j, img_r, atom_z, mi);
-        stg[0][lane] = mi.z / mi.R;  // t = cos theta
-        stg[1][lane] = mi.x / mi.R;  // z = sin theta e^{i phi}
-        stg[2][lane] = mi.y / mi.R;
-        stg[3][lane] = 0.0;
-        stg[4][lane] = mi.R;
-        stg[5][lane] = ok ? mi.w * mi.ex * mi.fc : 0.0;
-        stg[6][lane] = ok ? mi.w * mi.ex * (mi.dfc - 2.0 * a.alpha * mi.R * mi.fc) : 0.0;
-        stg[7][lane] = mi.rh[0];
-        stg[8][lane] = mi.rh[1];
-        stg[9][lane] = mi.rh[2];
+        s_u[0][lane] = mi.rh[0];
+        s_u[1][lane] = mi.rh[1];
+        s_u[2][lane] = mi.rh[2];
+        s_cu[lane] = ok ? mi.w * mi.ex * (mi.dfc - 2.0 * a.alpha * mi.R * mi.fc) : 0.0;
+        s_cv[lane] = ok ? mi.w * mi.ex * mi.fc : 0.0;
+        s_ir[lane] = 1.0 / mi.R;
         s_at[lane] = ok ? mi.i : -1;
-    }
-    __syncthreads();
-    int64_t cur = -1;
-    double Ar[NMAX], Ai[NMAX];
+        const cd z = cmake(mi.rh[0], mi.rh[1]);
+        cd p = cmake(1.0, 0.0);
 #pragma unroll
-    for (int n = 0; n < NMAX; n++) {
-        Ar[n] = 0.0;
-        Ai[n] = 0.0;
-    }
-    for (int b = 0; b < nb; b++) {
-        const int64_t i = s_at[b];
-        if (i != cur) {  // uniform: the image's centre changed
-            cur = i;
-            if (act) {
-                const cd *ai = reinterpret_cast<const cd *>(A) + (size_t)i * NMAX * L * M2;
-#pragma unroll
-                for (int n = 0; n < NMAX; n++) {
-                    const cd v = ai[(n * L + l) * M2 + a.lmax + m];
-                    Ar[n] = v.re;
-                    Ai[n] = v.im;
-                }
-            }
+        for (int m = 0; m < LM; m++) {
+            s_z[lane][m] = p;
+            p = cmul(p, z);
         }
-        // Y_lm of every lane (rows 0..lmax+1)
-        const double pl = ylane ? so3_legendre_eval(q, stg[0][b]) : 0.0;
-        const cd em = so3_zpow(cmake(stg[1][b], stg[2][b]), am);
-        const cd y = cmake(msg * pl * em.re, imsg * pl * em.im);
-        ysh[lane] = y;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        double c0 = 0.0, c1 = 0.0, c2 = 0.0;
-        if (act) {
-            const double R = stg[4][b], iR = 1.0 / R;
-            const double cv = stg[5][b] * lnorm, cu = stg[6][b] * lnorm;
-            const double rh0 = stg[7][b], rh1 = stg[8][b], rh2 = stg[9][b];
-            cd yv[6];
+    }
+    // the lane's coefficients, A and the rows are loaded here: held over
+    // the staging above (its cutoff and exponential are the register
+    // peak) they would cost a wavefront per SIMD
+    asm volatile("" ::: "memory");
+    fetch(0);
+    double q0[LM], q1[LM];
+    so3_load_q(ln.on0, ln.l, ln.m0, q0);
+    so3_load_q(ln.on1, ln.l, ln.m0 + 1, q1);
+    int64_t cur = -1;
+    double Ar0[NMAX], Ai0[NMAX], Ar1[NMAX], Ai1[NMAX];
 #pragma unroll
-            for (int q = 0; q < 6; q++) yv[q] = gi[q] >= 0 ? ysh[gi[q]] : cmake(0.0, 0.0);
-            const cd x0 = cmake((gc[0] * yv[0].re + gc[1] * yv[1].re) * iR, (gc[0] * yv[0].im + gc[1] * yv[1].im) * iR);
-            const cd xp = cmake((gc[2] * yv[2].re + gc[3] * yv[3].re) * iR, (gc[2] * yv[2].im + gc[3] * yv[3].im) * iR);
-            const cd xm = cmake((gc[4] * yv[4].re + gc[5] * yv[5].re) * iR, (gc[4] * yv[4].im + gc[5] * yv[5].im) * iR);
-            // grad Y: (xm - xp)/sqrt2, i (xm + xp)/sqrt2, x0
-            const cd g0 = cmake((xm.re - xp.re) * r2, (xm.im - xp.im) * r2);
-            const cd g1 = cmake(-(xm.im + xp.im) * r2, (xm.re + xp.re) * r2);
-            const double *ri = rad + ((size_t)(base + b) * L + l) * 2 * NMAX;
-            double ar = 0.0, ai2 = 0.0, br = 0.0, bi = 0.0;
+    for (int n = 0; n < NMAX; n++) Ar0[n] = Ai0[n] = Ar1[n] = Ai1[n] = 0.0;
+#pragma unroll 1
+    for (int it = 0; it < PER; it++) {
+        if ((it & 1) == 0) {
+            __syncthreads();  // the previous rows have been read, the scalars are written
+#pragma unroll
+            for (int u = 0; u < NLD; u++)
+                if (gof[u] >= 0) *reinterpret_cast<double2 *>(s_row + lof[u]) = pre[u];
+            __syncthreads();
+            if (it + 2 < PER) fetch(it + 2);
+        }
+        const int b = g * PER + it;
+        const int64_t i = s_at[b];
+        if (i != cur && i >= 0) {  // the row's image belongs to another centre
+            cur = i;
+            const cd *ai = reinterpret_cast<const cd *>(A) + (size_t)i * asize + aoff;
 #pragma unroll
             for (int n = 0; n < NMAX; n++) {
-                const double In = ri[n], dIn = ri[NMAX + n];
-                ar = fma(In, Ar[n], ar);
-                ai2 = fma(In, Ai[n], ai2);
-                br = fma(dIn, Ar[n], br);
-                bi = fma(dIn, Ai[n], bi);
+                const cd x0 = ai[n * astep], x1 = ln.on1 ? ai[n * astep + 1] : x0;
+                Ar0[n] = sc0 * x0.re;
+                Ai0[n] = sc0 * x0.im;
+                Ar1[n] = sc1 * x1.re;
+                Ai1[n] = sc1 * x1.im;
             }
-            // Re(conj(alpha) z) = ar z.re + ai z.im
-            const double ray = ar * y.re + ai2 * y.im;
-            const double rby = br * y.re + bi * y.im;
-            const double s = cu * ray + cv * rby;
-            c0 = fma(s, rh0, cv * (ar * g0.re + ai2 * g0.im));
-            c1 = fma(s, rh1, cv * (ar * g1.re + ai2 * g1.im));
-            c2 = fma(s, rh2, cv * (ar * x0.re + ai2 * x0.im));
         }
-        wave_sum3_lane63(c0, c1, c2);
-        if (lane == 63) {
-            const int64_t e = base + b;
-            dedr[3 * e] = c0;
-            dedr[3 * e + 1] = c1;
-            dedr[3 * e + 2] = c2;
+        const double *ri = s_row + (g * 2 + (it & 1)) * RS + ln.l * 2 * NMAX;
+        double ar0 = 0.0, ai0 = 0.0, br0 = 0.0, bi0 = 0.0, ar1 = 0.0, ai1 = 0.0, br1 = 0.0, bi1 = 0.0;
+#pragma unroll
+        for (int n = 0; n < NMAX; n++) {
+            const double In = ri[n], dIn = ri[NMAX + n];
+            ar0 = fma(In, Ar0[n], ar0);
+            ai0 = fma(In, Ai0[n], ai0);
+            ar1 = fma(In, Ar1[n], ar1);
+            ai1 = fma(In, Ai1[n], ai1);
+            br0 = fma(dIn, Ar0[n], br0);
+            bi0 = fma(dIn, Ai0[n], bi0);
+            br1 = fma(dIn, Ar1[n], br1);
+            bi1 = fma(dIn, Ai1[n], bi1);
         }
-        // the next image rewrites the Y table
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const double t = s_u[2][b], cu = s_cu[b], cv = s_cv[b];
+        double p0 = q0[LM - 1], p1 = q1[LM - 1], d0 = 0.0, d1 = 0.0;
+#pragma unroll
+        for (int j = LM - 2; j >= 0; j--) {
+            d0 = fma(d0, t, p0);
+            d1 = fma(d1, t, p1);
+            p0 = fma(p0, t, q0[j]);
+            p1 = fma(p1, t, q1[j]);
+        }
+        const cd z0 = s_z[b][ln.m0], z1 = s_z[b][iz], zp = s_z[b][ip];
+        const double P0 = ar0 * z0.re + ai0 * z0.im, P1 = ar1 * z1.re + ai1 * z1.im;
+        const double B0 = br0 * z0.re + bi0 * z0.im, B1 = br1 * z1.re + bi1 * z1.im;
+        const double w0 = dm0 * p0, w1 = dm1 * p1;
+        double S = p0 * (cu * P0 + cv * B0) + p1 * (cu * P1 + cv * B1);
+        double Gx = w0 * (ar0 * zp.re + ai0 * zp.im) + w1 * (ar1 * z0.re + ai1 * z0.im);
+        double Gy = w0 * (ai0 * zp.re - ar0 * zp.im) + w1 * (ai1 * z0.re - ar1 * z0.im);
+        double Gz = d0 * P0 + d1 * P1;
+        // sums over the row of 16 lanes: bit 3 of the lane keeps (S, Gx)
+        // or (Gy, Gz), bit 2 one of the two, then the quad
+        const bool up = gl & 8, up2 = gl & 4;
+        const double k0 = (up ? Gy : S) + so3_dpp<0x128>(up ? S : Gy);
+        const double k1 = (up ? Gz : Gx) + so3_dpp<0x128>(up ? Gx : Gz);
+        double k = (up2 ? k1 : k0) + so3_dpp<0x141>(up2 ? k0 : k1);
+        k += so3_dpp<0x4e>(k);
+        k += so3_dpp<0xb1>(k);
+        if ((gl & 3) == 0) s_sum[b][gl >> 2] = k;
+    }
+    __syncthreads();
+    if (lane < nb) {
+        const double ux = s_u[0][lane], uy = s_u[1][lane], uz = s_u[2][lane];
+        const double S = s_sum[lane][0], Gx = s_sum[lane][1], Gy = s_sum[lane][2], Gz = s_sum[lane][3];
+        const double f = s_cv[lane] * s_ir[lane], r = S - f * (ux * Gx + uy * Gy + uz * Gz);
+        double *o = dedr + 3 * (b0 + lane);
+        o[0] = fma(f, Gx, r * ux);
+        o[1] = fma(f, Gy, r * uy);
+        o[2] = fma(f, Gz, r * uz);
     }
 }
 
@@ -1616,6 +1901,28 @@ int so3_series_init() {
         if (m > 0) pm[m] = -std::sqrt((2.0 * m + 1.0) / (2.0 * m));
         p1[m] = std::sqrt(2.0 * m + 3.0);
     }
+    // Q of (l, m) by the recurrence of ylm_row on coefficient vectors:
+    // P_m = sqrt(1/4pi) prod pmm_k, P_m+1 = p1 t P_m, P_k = lega_k (t P_k-1 -
+    // legb_k P_k-2)
+    std::vector<double> lq(SO3_QL * SO3_QL * SO3_QL, 0.0);
+    for (int m = 0; m < SO3_QL; m++) {
+        double prev[SO3_QL] = {0}, cur[SO3_QL] = {0};
+        cur[0] = std::sqrt(0.25 / M_PI);
+        for (int k = 1; k <= m; k++) cur[0] *= pm[k];
+        for (int l = m; l < SO3_QL; l++) {
+            if (l > m) {
+                const double c1 = l == m + 1 ? p1[m] : la[l * SO3_LEGD + m], c2 = l == m + 1 ? 0.0 : lb[l * SO3_LEGD + m];
+                double nx[SO3_QL];
+                for (int j = 0; j < SO3_QL; j++) nx[j] = c1 * ((j > 0 ? cur[j - 1] : 0.0) - c2 * prev[j]);
+                for (int j = 0; j < SO3_QL; j++) {
+                    prev[j] = cur[j];
+                    cur[j] = nx[j];
+                }
+            }
+            for (int j = 0; j < SO3_QL; j++) lq[(l * SO3_QL + m) * SO3_QL + j] = cur[j];
+        }
+    }
+    PXFF_HIP_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(g_so3_legq), lq.data(), lq.size() * sizeof(double)));
     PXFF_HIP_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(g_so3_lega), la.data(), la.size() * sizeof(double)));
     PXFF_HIP_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(g_so3_legb), lb.data(), lb.size() * sizeof(double)));
     PXFF_HIP_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(g_so3_pmm), pm.data(), pm.size() * sizeof(double)));
@@ -1663,7 +1970,7 @@ static int so3_ctot_impl(const pxff_so3_params *p, int64_t natoms, const int64_t
                          const int64_t *d_img_j, const double *d_img_r, const int64_t *d_img_rev,
                          const int64_t *d_atom_z, const double *d_G, const double *d_rq, const double *d_lnorm,
                          const double *d_dr, double *d_out, double *d_radial, void *stream, int64_t *d_work = nullptr,
-                         int64_t cap = 0, const double *d_table = nullptr) {
+                         int64_t cap = 0, const double *d_table = nullptr, int half = 0, double *d_x = nullptr) {
     int rc = so3_check(p);
     if (rc) return rc;
     if (natoms <= 0) return 0;
@@ -1687,7 +1994,13 @@ static int so3_ctot_impl(const pxff_so3_params *p, int64_t natoms, const int64_t
                 // with pairs, one resident round of wavefronts (2 per SIMD at
                 // 256 registers), each queueing several chunks of 64 images so
                 // that its batches of 64 qualifying images are full
-                if (d_img_rev && d_work && cap > 0) {
+                if (d_img_rev && d_table && cap > 0 && cap <= SO3_RDIRECT) {
+                    const int nk = so3_rtab_nk(p);
+                    SO3_DISPATCH_NMAX(p->nmax, if constexpr (NM <= 6) {
+                        so3_radial_direct_kernel<NM><<<div_up(cap, 4), 256, 0, s>>>(
+                            a, natoms, d_img_start, d_img_r, d_img_rev, d_table, nk, p->rcut / nk, d_radial);
+                    });
+                } else if (d_img_rev && d_work && cap > 0) {
                     // pair images sorted into |r| bins, then one image per lane
                     so3_rbin_hist_kernel<<<SO3_RBLK, SO3_RBT, 0, s>>>(natoms, d_img_start, d_img_r, d_img_rev, p->rcut,
                                                                   d_work);
@@ -1721,7 +2034,12 @@ static int so3_ctot_impl(const pxff_so3_params *p, int64_t natoms, const int64_t
             }
             PXFF_LAUNCH_CHECK();
         }
-        if (d_radial && p->lmax <= 7) {
+        if (d_radial && p->lmax <= 6) {
+            PXFF_REQUIRE(natoms <= 0x7fffffff, "too many atoms for one launch");
+            SO3_DISPATCH_NMAX(p->nmax, (so3_expand_kernel<NM><<<(unsigned)natoms, SO3_CT, 0, s>>>(
+                                           a, natoms, d_img_start, d_img_j, d_img_r, d_atom_z, d_radial, d_out, half,
+                                           d_x)));
+        } else if (d_radial && p->lmax == 7) {
             // one lane per (l, m), the n-sums in registers
             SO3_DISPATCH_NMAX(p->nmax, (so3_ctot_lm_kernel<NM><<<grid, 64, 0, s>>>(
                                            a, natoms, d_img_start, d_img_j, d_img_r, d_atom_z, d_radial, d_out)));
@@ -1756,6 +2074,22 @@ extern "C" int pxff_so3_ctot_pairs(const pxff_so3_params *p, int64_t natoms, con
                  "SO3: the radial table needs the |r| ordering workspace and nmax, lmax <= 6");
     return so3_ctot_impl(p, natoms, d_img_start, d_img_j, d_img_r, d_img_rev, d_atom_z, d_G, d_rq, d_lnorm, nullptr,
                          d_out, d_radial, stream, d_work, cap, d_table);
+}
+
+extern "C" int pxff_so3_forward_half(const pxff_so3_params *p, int64_t natoms, const int64_t *d_img_start,
+                                     const int64_t *d_img_j, const double *d_img_r, const int64_t *d_img_rev,
+                                     const int64_t *d_atom_z, const double *d_G, const double *d_rq,
+                                     const double *d_lnorm, double *d_ct, double *d_x, double *d_radial,
+                                     int64_t *d_work, int64_t cap, const double *d_table, void *stream) {
+    PXFF_REQUIRE(p != nullptr && p->lmax <= 6, "SO3: the m >= 0 layout is for lmax <= 6");
+    PXFF_REQUIRE(d_radial != nullptr && d_ct != nullptr && d_x != nullptr, "null output");
+    PXFF_REQUIRE(d_img_rev != nullptr || (d_work == nullptr && d_table == nullptr),
+                 "SO3: the |r| ordering and the radial table need the reverse images");
+    PXFF_REQUIRE(cap >= 0 && (d_work == nullptr || cap > 0), "SO3: the |r| ordering needs the image capacity");
+    PXFF_REQUIRE(d_table == nullptr || (d_work != nullptr && p->nmax <= 6),
+                 "SO3: the radial table needs the |r| ordering workspace and nmax, lmax <= 6");
+    return so3_ctot_impl(p, natoms, d_img_start, d_img_j, d_img_r, d_img_rev, d_atom_z, d_G, d_rq, d_lnorm, nullptr,
+                         d_ct, d_radial, stream, d_work, cap, d_table, 1, d_x);
 }
 
 extern "C" int pxff_so3_radial_table_size(const pxff_so3_params *p, int *nk, int64_t *len) {
@@ -1815,6 +2149,45 @@ extern "C" int pxff_so3_adjoint_a(const pxff_so3_params *p, int64_t natoms, cons
     return 0;
 }
 
+extern "C" int pxff_so3_adjoint_a_half(const pxff_so3_params *p, int64_t natoms, const double *d_ct,
+                                       const double *d_beta, double *d_a, void *stream) {
+    int rc = so3_check(p);
+    if (rc) return rc;
+    PXFF_REQUIRE(p->lmax <= 6, "SO3: the m >= 0 layout is for lmax <= 6");
+    if (natoms <= 0) return 0;
+    const int64_t nh = (int64_t)(p->lmax + 1) * (p->lmax + 2) / 2;
+    hipStream_t s = (hipStream_t)stream;
+    SO3_DISPATCH_NMAX(p->nmax, (so3_adj_a_half_kernel<NM><<<div_up(natoms * nh, 256), 256, 0, s>>>(
+                                   natoms, p->lmax, d_ct, d_beta, d_a)));
+    PXFF_LAUNCH_CHECK();
+    return 0;
+}
+
+static int so3_deidrj_rows(const So3Args &a, int64_t nimg, const int64_t *d_img_atom, const int64_t *d_img_j,
+                           const double *d_img_r, const int64_t *d_atom_z, const double *d_a, int half,
+                           const double *d_radial, double *d_dedr, hipStream_t s, const int64_t *d_count) {
+    const int64_t grid = (nimg + SO3_AB - 1) / SO3_AB;
+    PXFF_REQUIRE(grid <= 0x7fffffff, "too many images for one launch");
+    SO3_DISPATCH_NMAX(a.nmax, (so3_deidrj_half_kernel<NM><<<(unsigned)grid, 64, 0, s>>>(
+                                  a, nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_a, half, d_radial, d_dedr,
+                                  d_count)));
+    PXFF_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int pxff_so3_deidrj_half(const pxff_so3_params *p, int64_t nimg, const int64_t *d_count,
+                                    const int64_t *d_img_atom, const int64_t *d_img_j, const double *d_img_r,
+                                    const int64_t *d_atom_z, const double *d_lnorm, const double *d_a,
+                                    const double *d_radial, double *d_dedr, void *stream) {
+    int rc = so3_check(p);
+    if (rc) return rc;
+    PXFF_REQUIRE(p->lmax <= 6, "SO3: the m >= 0 layout is for lmax <= 6");
+    PXFF_REQUIRE(d_radial != nullptr && ((uintptr_t)d_radial & 15) == 0, "SO3: needs 16-byte aligned radial integrals");
+    if (nimg <= 0) return 0;
+    return so3_deidrj_rows(make_args(p, nullptr, nullptr, d_lnorm), nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_a,
+                           1, d_radial, d_dedr, (hipStream_t)stream, d_count);
+}
+
 static int so3_image_launch(const pxff_so3_params *p, int mode, int64_t nimg, const int64_t *d_img_atom,
                             const int64_t *d_img_j, const double *d_img_r, const int64_t *d_atom_z, const double *d_G,
                             const double *d_rq, const double *d_lnorm, const double *d_cin, double *d_out,
@@ -1828,11 +2201,8 @@ static int so3_image_launch(const pxff_so3_params *p, int mode, int64_t nimg, co
     PXFF_REQUIRE(lds <= 160 * 1024, "SO3: LDS need exceeds 160 KB");
     const int NG = 64 / (p->lmax + 1);
     const int grid = div_up(nimg, NG);
-    if (mode == SO3_ADJOINT && d_radial && p->lmax <= 6) {
-        // one lane per (l, m), 64 images per wavefront
-        SO3_DISPATCH_NMAX(p->nmax, (so3_deidrj_lm_kernel<NM><<<div_up(nimg, 64), 64, 0, s>>>(
-                                       a, nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_cin, d_radial, d_out,
-                                       d_count)));
+    if (mode == SO3_ADJOINT && d_radial && p->lmax <= 6 && ((uintptr_t)d_radial & 15) == 0) {
+        return so3_deidrj_rows(a, nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_cin, 0, d_radial, d_out, s, d_count);
     } else if (mode == SO3_ADJOINT) {
         SO3_DISPATCH_NMAX(p->nmax, {
             auto k = so3_image_kernel<NM, SO3_ADJOINT>;

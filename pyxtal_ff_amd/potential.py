@@ -208,6 +208,10 @@ def _fused_adjoint(nl, cfg, weights, model, species_atom, work_order=None, count
     SNAP, (atomic numbers,) for SO(3)."""
     if isinstance(cfg, dev_so3.So3Config):
         (atom_z,) = weights
+        if dev_so3.half_layout(cfg):
+            x, ct, rad = dev_so3.forward_half(nl, cfg, atom_z)
+            e_atom, beta = model.energy_grad(x, species_atom)
+            return e_atom, dev_so3.adjoint_half(nl, cfg, atom_z, ct, beta, rad, counted=counted)
         x, ct, rad = dev_so3.forward(nl, cfg, atom_z, radial=True)
         e_atom, beta = model.energy_grad(x, species_atom)
         a = dev_so3.adjoint_a(nl, cfg, ct, beta)

@@ -151,6 +151,50 @@ def forward(nl, cfg, atom_z, img_r=None, radial=False):
     return power(nl, cfg, ct), ct
 
 
+def half_layout(cfg):
+    """Whether the m >= 0 half of the expansion serves the energy + force path."""
+    return cfg.lmax <= 6
+
+
+def forward_half(nl, cfg, atom_z):
+    """(x, expansion, radial integrals) of the list's own separations, the
+    expansion as its m >= 0 half [N, nmax, (lmax+1)(lmax+2)/2] complex and
+    the power spectrum formed beside it (pxff_so3_forward_half)."""
+    p = nat.ptr
+    dev = nl.pos.device
+    cap = nl.img_capacity
+    ct = _f64(nl.natoms * cfg.nmax * (cfg.lmax + 1) * (cfg.lmax + 2), dev)
+    x = _f64(nl.natoms * cfg.ncoef, dev)
+    rad = _f64(cap * (cfg.lmax + 1) * 2 * cfg.nmax, dev)
+    work = torch.empty(RWORK + cap, dtype=torch.int64, device=dev)
+    nat.check(nat.lib().pxff_so3_forward_half(cfg.params, nl.natoms, p(nl.img_start), p(nl.img_j), p(nl.img_r),
+                                              p(nl.img_rev), p(atom_z), p(cfg.G), p(cfg.rq), p(cfg.lnorm), p(ct), p(x),
+                                              p(rad), p(work), cap, p(cfg.radial_table()), nat.stream()),
+              "pxff_so3_forward_half")
+    return x[: nl.natoms * cfg.ncoef].view(nl.natoms, cfg.ncoef), ct, rad
+
+
+def adjoint_half(nl, cfg, atom_z, ct, beta, radial, counted=False):
+    """dE/dr per image from dE/dx and forward_half's arrays: a function
+    launching the sweep.  A is formed at once; counted as in deidrj."""
+    p = nat.ptr
+    dev = nl.pos.device
+    a = torch.empty_like(ct)
+    beta = beta.contiguous()
+    nat.check(nat.lib().pxff_so3_adjoint_a_half(cfg.params, nl.natoms, p(ct), p(beta), p(a), nat.stream()),
+              "pxff_so3_adjoint_a_half")
+
+    def sweep():
+        n = nl.img_capacity if counted else nl.nimg
+        out = _f64(n * 3, dev)
+        count = nl.img_start[nl.natoms:] if counted else None
+        nat.check(nat.lib().pxff_so3_deidrj_half(cfg.params, n, p(count), p(nl.img_atom), p(nl.img_j), p(nl.img_r),
+                                                 p(atom_z), p(cfg.lnorm), p(a), p(radial), p(out), nat.stream()),
+                  "pxff_so3_deidrj_half")
+        return out[: n * 3].view(n, 3)
+    return sweep
+
+
 def adjoint_a(nl, cfg, ct, beta):
     p = nat.ptr
     a = _f64(nl.natoms * cfg.csz * 2, nl.pos.device)
