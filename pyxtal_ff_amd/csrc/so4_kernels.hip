@@ -28,6 +28,7 @@
 #include <map>
 #include <atomic>
 #include <mutex>
+#include <numeric>
 #include <tuple>
 #include <utility>
 #include <vector>
@@ -50,6 +51,162 @@ int upload(const std::vector<T> &v, T **dst) {
     return 0;
 }
 }  // namespace
+
+// Tables of the matrix-core dB/dr kernel (so4_dbdr_centre_kernel).
+static int db_tables(const So4HostTables &t, So4Dev &d) {
+    const int nw = db_waves(t.twol), tw = ((t.nb + 3) / 4 + nw - 1) / nw, nslot = nw * tw * 4;
+    // stages: runs of levels whose values share a W row
+    std::vector<int> stage(t.ldim, 0);
+    for (int l = 1; l < t.ldim; l++) stage[l] = stage[l - 1] + (db_stage_first(t.twol, l) == l ? 1 : 0);
+    const int nstage = stage[t.ldim - 1] + 1;
+    // the levels that hold a block of b
+    std::vector<unsigned> lev(nslot, 0u);
+    std::vector<int> level(t.nblk, 0);
+    for (int l = 0; l < t.ldim; l++)
+        for (int k = t.blk_level_start[l]; k < t.blk_level_start[l + 1]; k++) {
+            level[k] = l;
+            for (int q = 0; q < 3; q++)
+                if (t.blk_tb[3 * k + q] >= 0) lev[t.blk_tb[3 * k + q]] |= 1u << l;
+        }
+    // Components to the places (wavefront, tile, row): a tile costs the union
+    // of its components' levels, and the wavefronts wait for each other
+    // after every stage, so the cost is the sum over the stages of the
+    // busiest wavefront's steps (then the steps of all).  Exchanges while
+    // they do not cost more, from the components in order of their levels.
+    std::vector<int> place(nslot);
+    std::iota(place.begin(), place.end(), 0);
+    std::stable_sort(place.begin(), place.end(), [&](int a, int b) { return lev[a] > lev[b]; });
+    // deal the tiles out in turn
+    {
+        std::vector<int> p(place.size());
+        for (int k = 0; k < nw * tw; k++)
+            for (int q = 0; q < 4; q++) p[((k % nw) * tw + k / nw) * 4 + q] = place[4 * k + q];
+        place = p;
+    }
+    std::vector<int> work(nw * nstage);
+    auto wave_work = [&](int w) {
+        std::fill(work.begin() + w * nstage, work.begin() + (w + 1) * nstage, 0);
+        for (int k = 0; k < tw; k++) {
+            unsigned m = 0;
+            for (int q = 0; q < 4; q++) m |= lev[place[(w * tw + k) * 4 + q]];
+            for (int l = 0; l < t.ldim; l++)
+                if (m >> l & 1) work[w * nstage + stage[l]] += db_steps(l);
+        }
+    };
+    auto total = [&]() {
+        long peak = 0, sum = 0;
+        for (int s = 0; s < nstage; s++) {
+            int mx = 0;
+            for (int w = 0; w < nw; w++) {
+                mx = std::max(mx, work[w * nstage + s]);
+                sum += work[w * nstage + s];
+            }
+            peak += mx;
+        }
+        return peak * 4096 + sum;
+    };
+    for (int w = 0; w < nw; w++) wave_work(w);
+    uint32_t rnd = 12345u;
+    auto next = [&](int n) {
+        rnd = rnd * 1664525u + 1013904223u;
+        return (int)((rnd >> 8) % (uint32_t)n);
+    };
+    long best = total();
+    for (int it = 0; it < 60000; it++) {
+        const int i = next((int)place.size()), j = next((int)place.size());
+        if (i / 4 == j / 4 || lev[place[i]] == lev[place[j]]) continue;
+        std::swap(place[i], place[j]);
+        wave_work(i / (4 * tw));
+        wave_work(j / (4 * tw));
+        const long now = total();
+        if (now <= best) {
+            best = now;
+        } else {
+            std::swap(place[i], place[j]);
+            wave_work(i / (4 * tw));
+            wave_work(j / (4 * tw));
+        }
+    }
+    // levels of every tile, then the component of every slot (-1 none)
+    std::vector<int> tile, where(t.nb, 0);
+    for (int k = 0; k < nw * tw; k++) {
+        unsigned m = 0;
+        for (int q = 0; q < 4; q++) m |= lev[place[4 * k + q]];
+        tile.push_back((int)m);
+    }
+    for (int k = 0; k < nslot; k++) {
+        tile.push_back(place[k] < t.nb ? place[k] : -1);
+        if (place[k] < t.nb) where[place[k]] = k;
+    }
+    // LDS row of the block of every (level, slot) (the zero row without one)
+    // and its factor 2 f norm_l; Z elements in level order: their Z offset,
+    // then place in the stage's LDS rows and twice the half weight
+    const int zero = db_stage_zlds(t.twol) - db_stride(t.twol);
+    std::vector<int> row((size_t)t.ldim * nslot, zero), zmap, first;
+    std::vector<double> fac((size_t)t.ldim * nslot, 0.0);
+    int z = 0, c = 0;
+    for (int l = 0; l < t.ldim; l++) {
+        if (l == 0 || stage[l] != stage[l - 1]) {
+            first.push_back(z);
+            first.push_back(c);
+            first.push_back(l);
+        }
+        const int base = db_level_zbase(t.twol, l), st = db_level_stride(l);
+        for (int k = t.blk_level_start[l]; k < t.blk_level_start[l + 1]; k++) {
+            const int at = base + (k - t.blk_level_start[l]) * st;
+            for (int q = 0; q < 3; q++) {
+                const int b = t.blk_tb[3 * k + q];
+                if (b < 0) continue;
+                const size_t e = (size_t)l * nslot + where[b];
+                if (row[e] != zero) {
+                    set_error("two blocks of one level target one bispectrum component");
+                    return PXFF_EINVAL;
+                }
+                row[e] = at;
+                fac[e] = t.blk_tf[3 * k + q] * 2.0 * t.lnorm[l];
+            }
+            for (int loc = 0; loc < (l / 2 + 1) * (l + 1); loc++) {
+                zmap.push_back(t.blk_zoff[k] + loc);
+                zmap.push_back((at + 2 * loc) | (int)(2.0 * t.h_weight[t.hoff[l] + loc]) << 16);
+            }
+        }
+        z += (t.blk_level_start[l + 1] - t.blk_level_start[l]) * (l / 2 + 1) * (l + 1);
+        c += db_steps(l) * 16;
+    }
+    first.push_back(z);
+    first.push_back(c);
+    first.push_back(t.ldim);
+    // coefficients (C1, C2) of V_q at element k of a level (re / im of half
+    // element loc, times W's sqrt factor s): V_q[k] = C1 Z[k + off1] + C2 Z[k + off2]
+    std::vector<double> coef;
+    auto f = [](int n) {
+        double v = 1.0;
+        for (int k = 2; k <= n; k++) v *= k;
+        return v;
+    };
+    for (int l = 0; l < t.ldim; l++)
+        for (int k = 0; k < 4 * db_steps(l); k++) {
+            const int loc = k / 2, mb = loc / (l + 1), m = loc - mb * (l + 1);
+            const bool in = loc < (l / 2 + 1) * (l + 1);
+            const double s = in ? std::sqrt(f(m) * f(l - m) / (f(mb) * f(l - mb))) : 0.0;
+            const double up = in ? std::sqrt((double)((m + 1) * (l - m))) : 0.0;
+            const double dn = in ? std::sqrt((double)(m * (l - m + 1))) : 0.0;
+            const double sg = k & 1 ? -1.0 : 1.0;
+            const double cc[4][2] = {{s, 0.0}, {sg * s * (l - 2 * m), 0.0}, {s * up, -s * dn}, {sg * s * up, sg * s * dn}};
+            for (int q = 0; q < 4; q++) {
+                coef.push_back(cc[q][0]);
+                coef.push_back(cc[q][1]);
+            }
+        }
+    d.db_nstage = nstage;
+    int rc = 0;
+    if ((rc = upload(tile, &d.db_tile))) return rc;
+    if ((rc = upload(row, &d.db_row))) return rc;
+    if ((rc = upload(fac, &d.db_fac))) return rc;
+    if ((rc = upload(zmap, &d.db_zmap))) return rc;
+    if ((rc = upload(first, &d.db_stage))) return rc;
+    return upload(coef, &d.db_coef);
+}
 
 int find_so4_tables(int twol, int norm, const So4Dev **out) {
     int dev = 0;
@@ -160,6 +317,7 @@ int get_so4_tables(int twol, int norm, const So4Dev **out) {
     for (auto &q : yt) ytf.insert(ytf.end(), q.begin(), q.end());
     d.nytask = (int)yt.size();
     if ((rc = upload(ytf, &d.ytask))) return rc;
+    if ((rc = db_tables(t, d))) return rc;
     g_tabs[key] = d;
     *out = &g_tabs[key];
     return 0;
@@ -343,6 +501,19 @@ __device__ inline void sweep_rows_w(int mb, const CK &ck, F &&f) {
         }
         f(l, w, 2 * mb <= l);
     }
+}
+
+// One level of the W rows with nothing but multiplications: row mb of level l
+// is the coefficients in x of (b + a x)^mb (conj a - conj b x)^(l - mb) (the
+// inversion of row 0 of level mb is the first power), so every level
+// multiplies by one of the two factors.  w[m] is zero for m > l - 1 on entry.
+template <int TWOJ>
+__device__ __forceinline__ void row_step_w(int l, int mb, const CK &ck, cd *w) {
+    const bool up = l <= mb;
+    const cd f0 = up ? cconj(ck.cb) : ck.ca, f1 = up ? cconj(ck.ca) : cmake(-ck.cb.re, -ck.cb.im);
+#pragma unroll
+    for (int m = TWOJ; m >= 1; m--) w[m] = cmadd(f1, w[m - 1], cmul(f0, w[m]));
+    w[0] = cmul(f0, w[0]);
 }
 
 // sqrt(m! (l - m)! / (mb! (l - mb)!)), the factor of sweep_rows_w, from
@@ -1290,168 +1461,329 @@ __global__ __launch_bounds__(64) void so4_dbdr_kernel(
 }
 
 // --------------------------------------- plain dB/dr, one centre per workgroup
-// The same dB/dr per image as so4_dbdr_kernel, organised around the centre:
-// a workgroup (one wavefront) takes one centre and runs its images NG at a
-// time.  With the su(2) generators of the image (see su2_generators), the
-// derivative of a block product needs U alone:
-//   Re <dU_tot/dr_k, Z_blk> = fc (p_k A1 + Re q_k A2 + Im q_k A3) + dfc rhat_k Au,
-// A the generator sums of the image's U rows against the block's Z rows
-// (generator_dots; the middle row of an even level weighted 1 / 0.5 / 0
-// for ma < , = , > l/2).  Level by level the groups put their U half rows
-// into LDS and the wavefront stages the centre's Z blocks of the level
-// there (weights applied), read from the tile-major Z; then each lane sums
-// one (image, block) pair over all the block's rows and adds
-// 2 norm_l w f (.) to the block's (b, factor) targets (three terms of
-// compute_dbidrj, SNAP.py:1143-1257) directly in the output rows: within a
-// level each (image, b, k) receives at most one block, and the barriers
-// between levels order the additions of different levels.  LDS holds only
-// the level's U rows, its Z blocks and per-image factors; NG is chosen so
-// that it stays within 20 KB where possible (two workgroups per SIMD).
-// Workgroups are mapped to centres so that the eight centres whose Z
-// entries share a 128-byte line run on one XCD (the Z reads of the
-// tile-major layout then hit that XCD's L2).
+// dB/dr of every image of a centre on the FP64 matrix cores.  With the su(2)
+// generators of an image (su2_generators) and W the rows of sweep_rows_w,
+//   dB_b/dr_k = w [fc (p_k A1 + Re q_k A2 + Im q_k A3) + dfc rhat_k Au]_b,
+// each A_q of component b a real inner product over the half elements of
+// three levels: of W of the image with
+//   V_q = sum over the blocks targeting b (compute_dbidrj, SNAP.py:1143-1257)
+//         of 2 f norm_l (generator q applied to the block's weighted Z rows),
+// and V_q depends on the centre only.  So per centre it is a product of a
+// matrix with four rows (q) per b by a matrix with a column per image, the
+// sum running over (level, half element, re / im).  Level by level the
+// workgroup puts the images' W rows (one thread per image and row) and the
+// centre's Z blocks (half weights applied) into LDS; a wavefront forms the
+// operand V_q of its tiles of four b from two Z values and two coefficients
+// (generator, sqrt factors of W) and keeps the sums of up to 16 b and 48
+// images in registers over all levels, so the outputs are written once.
+// Rows of a 16x16x4 tile are (q, b), so that a lane ends up with all four
+// sums of its (b, image).
+// Levels go in stages, runs of levels whose values share a W row, so that the
+// workgroup meets at a barrier twice per stage and not per level.
+// A tile of four b costs the union of their levels: the b are grouped for
+// small unions (2J = 8: 440 steps of four products per 16 images against 304
+// for each b alone and 523 in index order).
+// Bound by latency, two workgroups per CU (registers): of 95k cycles of a
+// workgroup at 2J = 8 the products take 48k, the W rows and their barriers
+// 30k, the prologue 16k.  4096 atoms (115k images), 2J = 8: 620 -> 398 us;
+// 1728 atoms: 264 -> 180 us.  The
+// forerunner summed one (image, block) per lane on the vector units and added
+// to the output rows level by level (0.9 GB read and 0.9 GB written for 157 MB
+// of output).  Measured beside it (4096 atoms): eight wavefronts of half the
+// tiles 525 us, a stage per level 474 us.
+typedef double db_d4 __attribute__((ext_vector_type(4)));
 template <int TWOJ>
-__host__ __device__ constexpr int dbdr_centre_ng() {
-    constexpr int G = TWOJ / 2 + 1;
-    constexpr int NL = (TWOJ / 2 + 1) * (TWOJ + 1);
-    constexpr int fixed = zlevel_max_of(TWOJ) * 16 + (TWOJ + 1) * (TWOJ + 1) * 8;
-    constexpr int per = NL * 16 + 12 * 8;
-    constexpr int fit = (20480 - fixed) / per;
-    return fit >= 64 / G ? 64 / G : (fit >= 4 ? fit : 64 / G);
-}
+struct DbDim {
+    static constexpr int NW = db_waves(TWOJ);
+    static constexpr int T = 64 * NW;
+    static constexpr int G = TWOJ / 2 + 1;
+    static constexpr int NT = TWOJ <= 8 ? 3 : 2;  // tiles of 16 images per pass
+    static constexpr int NI = 16 * NT;
+    static constexpr int KS = db_stride(TWOJ);  // W row: the values of the longest stage
+    static constexpr int TW = ((nb_of(TWOJ) + 3) / 4 + NW - 1) / NW;  // tiles per wavefront
+    static constexpr int NSLOT = NW * TW * 4;
+    static constexpr int ZP = (db_stage_zmax(TWOJ) + T - 1) / T;       // Z elements of a stage per thread
+    static constexpr int CP = (db_steps(TWOJ) * 16 + T - 1) / T;       // coefficient pairs
+    static_assert(NI * G <= T, "one thread per (image, row)");
+    static_assert(16 * 3 * nb_of(TWOJ) <= NI * KS, "the output tile reuses the W rows");
+};
 
+struct DbArgs {
+    const int64_t *__restrict__ img_start, *__restrict__ img_j;
+    const double *__restrict__ img_r, *__restrict__ atom_w, *__restrict__ zt;
+    int nz, cutoff_id, z_atom_major, nstage;
+    const int *__restrict__ db_tile, *__restrict__ db_row;
+    const double *__restrict__ db_fac, *__restrict__ db_coef;
+    const int *__restrict__ db_zmap, *__restrict__ db_stage;
+    double rcut, rfac0;
+};
+
+// One pass: images [e0, e0 + ne), ne <= NI, of centre c.
 template <int TWOJ>
-__global__ __launch_bounds__(64) void so4_dbdr_centre_kernel(
-    int64_t natoms, const int64_t *__restrict__ img_start, const int64_t *__restrict__ img_j,
-    const double *__restrict__ img_r, const double *__restrict__ atom_w, const double *__restrict__ zt, int nz,
-    int nb, const double *rootpq_g, const double *__restrict__ lnorm, const int *__restrict__ blk_level_start,
-    const int *__restrict__ blk_zoff, const int *__restrict__ blk_tb, const double *__restrict__ blk_tf, double rcut,
-    double rfac0, int cutoff_id, int z_atom_major, double *__restrict__ dbdr) {
-    constexpr int G = TWOJ / 2 + 1;
-    constexpr int NG = dbdr_centre_ng<TWOJ>();
-    constexpr int NL = (TWOJ / 2 + 1) * (TWOJ + 1);
-    constexpr int ZLM = zlevel_max_of(TWOJ);
-    // per image: w fc p_k, w fc Re q_k, w fc Im q_k, w dfc rhat_k (k = 0..2)
-    constexpr int NSC = 12;
-    __shared__ double rpq[(TWOJ + 1) * (TWOJ + 1)];
-    __shared__ cd Ul[NG][NL];
-    __shared__ cd Zl[ZLM];
-    __shared__ double sc[NG][NSC];
-    // centre of this workgroup: swap the 3-bit fields (b / 8) % 8 and b % 8
-    // of the block index (the XCD is b % 8)
-    const int64_t bid = blockIdx.x;
-    const int64_t c = (bid & ~(int64_t)63) | ((bid & 7) << 3) | ((bid >> 3) & 7);
-    if (c >= natoms) return;
-    const int lane = threadIdx.x;
-    const int g = lane / G, mb = lane % G;
-    for (int k = lane; k < (TWOJ + 1) * (TWOJ + 1); k += 64) rpq[k] = rootpq_g[k];
-    const int64_t s0 = img_start[c], s1 = img_start[c + 1];
-    // the centre's Z entries: stride 64 in the tile-major layout, 1 in the
-    // atom-major copy
-    const cd *zc = reinterpret_cast<const cd *>(zt) + (z_atom_major ? (size_t)c * nz
-                                                                      : (size_t)(c >> 6) * nz * 64 + (c & 63));
-    const int zs = z_atom_major ? 1 : 64;
-    for (int64_t e0 = s0; e0 < s1; e0 += NG) {
-        const int ne = (int)(s1 - e0 < NG ? s1 - e0 : NG);
-        // the chunk's output rows start at zero
-        for (int k = lane; k < ne * nb * 3; k += 64) dbdr[(size_t)e0 * nb * 3 + k] = 0.0;
-        const int64_t e = e0 + g;
-        bool valid = g < ne;
-        double x = 0, yy = 0, zz = 1.0, r = 1.0, w = 0.0;
-        if (valid) {
-            x = img_r[3 * e];
-            yy = img_r[3 * e + 1];
-            zz = img_r[3 * e + 2];
-            r = sqrt(x * x + yy * yy + zz * zz);
-            w = atom_w[img_j[e]];
-            if (r < 1e-8) {  // coincident atoms contribute nothing (SNAP.py:1487)
-                valid = false;
-                x = 0;
-                yy = 0;
-                zz = 1.0;
-                r = 1.0;
-                w = 0.0;
-            }
+__device__ __forceinline__ void so4_dbdr_pass(const DbArgs &A, int64_t c, int64_t e0, int ne, double *__restrict__ dbdr) {
+    using D = DbDim<TWOJ>;
+    constexpr int T = D::T, G = D::G, NT = D::NT, NI = D::NI, KS = D::KS, TW = D::TW;
+    constexpr int NB = nb_of(TWOJ), NSLOT = D::NSLOT, ZP = D::ZP, CP = D::CP, NL = TWOJ + 1;
+    // the operand loads run up to five steps past a level's last (their
+    // values are not used): slack behind each array
+    constexpr int PAD = 5 * 4, ZLEN = db_stage_zlds(TWOJ) + PAD;
+    __shared__ __attribute__((aligned(16))) double Ul[NI * KS + PAD];
+    __shared__ __attribute__((aligned(16))) double Zl[ZLEN];
+    __shared__ double2 Cl[(db_steps(TWOJ) + 5) * 16];
+    __shared__ double s_fac[NL * NSLOT];
+    __shared__ int s_row[NL * NSLOT], s_b[NSLOT];
+    __shared__ double sc[NI][12];  // w fc p_k, w fc Re q_k, w fc Im q_k, w dfc rhat_k
+    __shared__ cd sck[NI][2];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int nt = (ne + 15) / 16;
+    const cd *zc = reinterpret_cast<const cd *>(A.zt) + (A.z_atom_major ? (size_t)c * A.nz
+                                                                          : (size_t)(c >> 6) * A.nz * 64 + (c & 63));
+    const int zs = A.z_atom_major ? 1 : 64;
+    // per stage s: {first Z element, first coefficient pair, first level}
+    __shared__ int stg[3 * (NL + 1)];
+    if (tid < 3 * (A.nstage + 1)) stg[tid] = A.db_stage[tid];
+    const int2 *zmap = reinterpret_cast<const int2 *>(A.db_zmap);
+    // the centre's Z blocks and the coefficients of a stage are loaded one
+    // stage ahead of their use, the places of its Z elements two
+    int2 mp[ZP];
+    cd zv[ZP];
+    int zp[ZP];
+    cd cv[CP];
+    auto places = [&](int s) __attribute__((always_inline)) {
+        const int z0 = stg[3 * s], z1 = stg[3 * s + 3];
+#pragma unroll
+        for (int u = 0; u < ZP; u++) mp[u] = z0 + u * T + tid < z1 ? zmap[z0 + u * T + tid] : make_int2(0, -1);
+    };
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < ZP; u++) {
+            zp[u] = mp[u].y;
+            zv[u] = zc[(size_t)mp[u].x * zs];  // (places without an element read element 0)
+        }
+        const int c0 = stg[3 * s + 1], c1 = stg[3 * s + 4];
+#pragma unroll
+        for (int u = 0; u < CP; u++) {
+            const int k = c0 + u * T + tid;
+            cv[u] = reinterpret_cast<const cd *>(A.db_coef)[k < c1 ? k : c0];
+        }
+    };
+    __syncthreads();
+    places(0);
+    // this image's record while the tables are on their way
+    double x = 0, yy = 0, zz = 1.0, wn = 0.0;
+    if (tid < ne) {
+        const int64_t e = e0 + tid;
+        x = A.img_r[3 * e];
+        yy = A.img_r[3 * e + 1];
+        zz = A.img_r[3 * e + 2];
+        wn = A.atom_w[A.img_j[e]];
+    }
+    for (int k = tid; k < NL * NSLOT; k += T) {
+        s_row[k] = A.db_row[k];
+        s_fac[k] = A.db_fac[k];
+    }
+    // levels of this wavefront's tiles, and the component of every slot
+    int tmask[TW];
+    static_for<TW>([&](auto TT) __attribute__((always_inline)) {
+        constexpr int t = decltype(TT)::value;
+        tmask[t] = __builtin_amdgcn_readfirstlane(A.db_tile[wv * TW + t]);
+    });
+    for (int k = tid; k < NSLOT; k += T) s_b[k] = A.db_tile[D::NW * TW + k];
+    for (int k = tid; k < (NI * KS + PAD) / 2; k += T) reinterpret_cast<double2 *>(Ul)[k] = make_double2(0.0, 0.0);
+    for (int k = tid; k < ZLEN / 2; k += T) reinterpret_cast<double2 *>(Zl)[k] = make_double2(0.0, 0.0);
+    for (int k = tid; k < (db_steps(TWOJ) + 5) * 16; k += T) Cl[k] = make_double2(0.0, 0.0);
+    fetch(0);
+    if (A.nstage > 1) places(1);
+    // operand roles of the lane: A row (q, b) and k', B column = image
+    const int q = (lane & 15) >> 2, bl = lane & 3, kp = lane >> 4, par = kp & 1;
+    const int sw = par ? -1 : 1;  // the other part of the same element
+    const int off1 = q == 0 ? 0 : (q == 1 ? sw : (q == 2 ? 2 : 2 + sw));
+    const int off2 = q == 2 ? -2 : (q == 3 ? sw - 2 : 0);
+    const int img = tid / G, mb = tid - img * G;  // W rows: one thread per (image, row)
+    if (tid < NI) {
+        double r = sqrt(x * x + yy * yy + zz * zz);
+        if (r < 1e-8) {  // coincident atoms contribute nothing (SNAP.py:1487)
+            x = 0;
+            yy = 0;
+            zz = 1.0;
+            r = 1.0;
+            wn = 0.0;
         }
         double fc, dfc;
-        cutoff_fdf(cutoff_id, r, rcut, fc, dfc);
+        cutoff_fdf(A.cutoff_id, r, A.rcut, fc, dfc);
         CK ck;
-        cayley_klein(x, yy, zz, r, rfac0 * M_PI * r / rcut, true, ck);
-        if (g < NG && mb == 0) {
-            double p[3];
-            cd q[3];
-            su2_generators(ck, p, q);
-            double *S = sc[g];
-            const double wf = w * fc, wd = w * dfc / r;
-            S[0] = wf * p[0];
-            S[1] = wf * p[1];
-            S[2] = wf * p[2];
-            S[3] = wf * q[0].re;
-            S[4] = wf * q[1].re;
-            S[5] = wf * q[2].re;
-            S[6] = wf * q[0].im;
-            S[7] = wf * q[1].im;
-            S[8] = wf * q[2].im;
-            S[9] = wd * x;
-            S[10] = wd * yy;
-            S[11] = wd * zz;
+        cayley_klein(x, yy, zz, r, A.rfac0 * M_PI * r / A.rcut, true, ck);
+        double p[3];
+        cd qq[3];
+        su2_generators(ck, p, qq);
+        sck[tid][0] = ck.ca;
+        sck[tid][1] = ck.cb;
+        const double wf = wn * fc, wd = wn * dfc / r;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            sc[tid][k] = wf * p[k];
+            sc[tid][3 + k] = wf * qq[k].re;
+            sc[tid][6 + k] = wf * qq[k].im;
         }
-        __syncthreads();
-        sweep_rows<TWOJ, false>(mb, rpq, ck, [&](int l, const cd *u, const cd(*du)[TWOJ + 1], bool half) {
-            (void)du;
-            if (g < NG && half) {
+        sc[tid][9] = wd * x;
+        sc[tid][10] = wd * yy;
+        sc[tid][11] = wd * zz;
+    }
+    __syncthreads();
+    db_d4 acc[TW][NT];
+#pragma unroll
+    for (int t = 0; t < TW; t++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) acc[t][n] = db_d4{0.0, 0.0, 0.0, 0.0};
+    CK ck;
+    ck.ca = img < NI ? sck[img][0] : cmake(1.0, 0.0);
+    ck.cb = img < NI ? sck[img][1] : cmake(0.0, 0.0);
+    cd w[TWOJ + 1];
+#pragma unroll
+    for (int m = 0; m <= TWOJ; m++) w[m] = cmake(m == 0 ? 1.0 : 0.0, 0.0);
+    // rolled over stages and levels: unrolled, every wavefront would run once
+    // through tens of KB of instructions
+#pragma unroll 1
+    for (int s = 0; s < A.nstage; s++) {
+        const int l0 = stg[3 * s + 2], l1 = stg[3 * s + 5];
+        if (s > 0) __syncthreads();  // the previous stage's operands have been read
+        int uo = 0;  // values of the stage's earlier levels in a W row
+#pragma unroll 1
+        for (int l = l0; l < l1; l++) {
+            if (l > 0) row_step_w<TWOJ>(l, mb, ck, w);
+            if (img < NI && 2 * mb <= l) {
+                double2 *ur = reinterpret_cast<double2 *>(Ul + img * KS + uo + 2 * mb * (l + 1));
 #pragma unroll
                 for (int m = 0; m <= TWOJ; m++)
-                    if (m <= l) Ul[g][mb * (l + 1) + m] = u[m];
+                    if (m <= l) ur[m] = make_double2(w[m].re, w[m].im);
             }
-            const int b0 = blk_level_start[l], nbl = blk_level_start[l + 1] - b0;
-            const int nloc = (l / 2 + 1) * (l + 1);
-            for (int it = lane; it < nbl * nloc; it += 64) {
-                const int bk = it / nloc, loc = it - bk * nloc;
-                const int row = loc / (l + 1), ma = loc - row * (l + 1);
-                const double wt = 2 * row < l ? 1.0 : (ma < row ? 1.0 : (ma == row ? 0.5 : 0.0));
-                const cd zv = zc[(size_t)(blk_zoff[b0 + bk] + loc) * zs];
-                Zl[it] = cmake(wt * zv.re, wt * zv.im);
-            }
-            // also orders the previous level's output additions before this
-            // level's
-            __syncthreads();
-            const double nrm2 = 2.0 * lnorm[l];
-            const int nrow = l / 2 + 1;
-            for (int it = lane; it < ne * nbl; it += 64) {
-                const int bk = it / ne, gg = it - bk * ne;
-                const int blk = b0 + bk;
-                double *o = dbdr + (size_t)(e0 + gg) * nb * 3;
-                int tb[3];
-                double tf[3];
+            uo += 4 * ((2 * (l / 2 + 1) * (l + 1) + 3) / 4);
+        }
 #pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    tb[q] = blk_tb[3 * blk + q];
-                    tf[q] = blk_tf[3 * blk + q] * nrm2;
+        for (int u = 0; u < ZP; u++) {
+            if (zp[u] < 0) continue;
+            // place in the low half, twice the half weight above
+            const double wt = 0.5 * (zp[u] >> 16);
+            *reinterpret_cast<double2 *>(Zl + (zp[u] & 0xffff)) = make_double2(wt * zv[u].re, wt * zv[u].im);
+        }
+#pragma unroll
+        for (int u = 0; u < CP; u++)
+            if (u * T + tid < 4 * uo) Cl[u * T + tid] = make_double2(cv[u].re, cv[u].im);
+        __syncthreads();
+        if (s + 1 < A.nstage) fetch(s + 1);
+        if (s + 2 < A.nstage) places(s + 2);
+        // a (tile, level) at a time, two steps per turn, the operands of the
+        // next turn on their way while the matrix cores work on this one
+        // (two register sets in turn)
+        struct Turn {
+            double2 c[2];
+            double x[2], y[2], b[2][NT];
+        };
+        static_for<TW>([&](auto TT) __attribute__((always_inline)) {
+            constexpr int t = decltype(TT)::value;
+            int ko = 0;
+#pragma unroll 1
+            for (int l = l0; l < l1; l++) {
+                const int kq = (2 * (l / 2 + 1) * (l + 1) + 3) / 4;
+                if ((tmask[t] >> l) & 1) {  // uniform
+                    const int slot = l * NSLOT + (wv * TW + t) * 4 + bl;
+                    const double *z = Zl + s_row[slot] + kp;
+                    const double fac = s_fac[slot];
+                    const double *ub = Ul + (lane & 15) * KS + kp + 4 * ko;
+                    const double2 *cb = Cl + kp * 4 + q + 16 * ko;
+                    auto load = [&](Turn &g, int kk) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            g.c[h] = cb[(kk + h) * 16];
+                            g.x[h] = z[(kk + h) * 4 + off1];
+                            g.y[h] = z[(kk + h) * 4 + off2];
+#pragma unroll
+                            for (int n = 0; n < NT; n++) g.b[h][n] = ub[n * 16 * KS + (kk + h) * 4];
+                        }
+                    };
+                    auto mul = [&](const Turn &g, int kk) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            if (kk + h >= kq) return;  // uniform
+                            const double av = fac * fma(g.c[h].x, g.x[h], g.c[h].y * g.y[h]);
+#pragma unroll
+                            for (int n = 0; n < NT; n++)
+                                if (n < nt)
+                                    acc[t][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, g.b[h][n], acc[t][n], 0, 0, 0);
+                        }
+                    };
+                    Turn g0, g1;
+                    load(g0, 0);
+#pragma unroll 1
+                    for (int kk = 0; kk < kq; kk += 4) {
+                        load(g1, kk + 2);
+                        mul(g0, kk);
+                        load(g0, kk + 4);
+                        mul(g1, kk + 2);
+                    }
                 }
-                // the targets' current values, loaded ahead of the sums so
-                // that their latency overlaps them (a block's targets are
-                // distinct b, duplicates being merged in the table, so none
-                // of these loads can see one of the stores below)
-                double old[3][3];
-#pragma unroll
-                for (int q = 0; q < 3; q++)
-#pragma unroll
-                    for (int k = 0; k < 3; k++) old[q][k] = tb[q] >= 0 ? o[3 * tb[q] + k] : 0.0;
-                double au = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-                for (int row = 0; row < nrow; row++)
-                    generator_dots<TWOJ>(l, &Ul[gg][row * (l + 1)], &Zl[bk * nloc + row * (l + 1)], au, a1, a2, a3);
-                const double *S = sc[gg];
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    const double pk = S[k] * a1 + S[3 + k] * a2 + S[6 + k] * a3 + S[9 + k] * au;
-#pragma unroll
-                    for (int q = 0; q < 3; q++)
-                        if (tb[q] >= 0) o[3 * tb[q] + k] = fma(tf[q], pk, old[q][k]);
-                }
+                ko += kq;
             }
-            __syncthreads();
         });
+    }
+    // lane (image, b): combine the four sums, collect 16 images' rows in
+    // LDS and write them out
+    double *ob = Ul;
+    static_for<NT>([&](auto NN) __attribute__((always_inline)) {
+        constexpr int n = decltype(NN)::value;
+        if (n >= nt) return;  // uniform
+        __syncthreads();
+        const double *S = sc[n * 16 + (lane & 15)];
+        static_for<TW>([&](auto TT) __attribute__((always_inline)) {
+            constexpr int t = decltype(TT)::value;
+            const int b = s_b[(wv * TW + t) * 4 + kp];
+            if (b < 0) return;
+            double *o = ob + (lane & 15) * (3 * NB) + 3 * b;
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                o[k] = S[k] * acc[t][n][1] + S[3 + k] * acc[t][n][2] + S[6 + k] * acc[t][n][3] + S[9 + k] * acc[t][n][0];
+        });
+        __syncthreads();
+        const int cnt = (ne - 16 * n < 16 ? ne - 16 * n : 16) * 3 * NB;
+        double *og = dbdr + (size_t)(e0 + 16 * n) * 3 * NB;
+        for (int k = tid; k < cnt; k += T) og[k] = ob[k];
+    });
+}
+
+// Centre of workgroup b: the 3-bit fields (b / 8) % 8 and b % 8 of the block
+// index swapped (the XCD is b % 8), so that the eight centres whose Z
+// entries share a 128-byte line run on one XCD.
+__device__ __forceinline__ int64_t so4_db_centre(int64_t b) {
+    return (b & ~(int64_t)63) | ((b & 7) << 3) | ((b >> 3) & 7);
+}
+
+// The first NI images of every centre, one workgroup each.  No loop over
+// passes here: the constants of the cutoff and of the Cayley-Klein parameters
+// are then held across it, which costs 144 spilled registers at 2J = 8
+// (725 against 540 us for 4096 atoms when the two were compared).
+template <int TWOJ>
+__global__ __launch_bounds__(DbDim<TWOJ>::T) __attribute__((amdgpu_waves_per_eu(2))) void so4_dbdr_centre_kernel(
+    DbArgs A, int64_t natoms, double *__restrict__ dbdr) {
+    constexpr int NI = DbDim<TWOJ>::NI;
+    const int64_t c = so4_db_centre(blockIdx.x);
+    if (c >= natoms) return;
+    const int64_t s0 = A.img_start[c], n = A.img_start[c + 1] - s0;
+    if (n > 0) so4_dbdr_pass<TWOJ>(A, c, s0, (int)(n < NI ? n : NI), dbdr);
+}
+
+// The images past NI of the centres that have more (none in a solid at the
+// usual cutoffs), a persistent grid over the centres.
+template <int TWOJ>
+__global__ __launch_bounds__(DbDim<TWOJ>::T) __attribute__((amdgpu_waves_per_eu(2))) void so4_dbdr_rest_kernel(
+    DbArgs A, int64_t natoms, double *__restrict__ dbdr) {
+    constexpr int NI = DbDim<TWOJ>::NI;
+    for (int64_t c = blockIdx.x; c < natoms; c += gridDim.x) {
+        const int64_t s1 = A.img_start[c + 1];
+#pragma unroll 1
+        for (int64_t e0 = A.img_start[c] + NI; e0 < s1; e0 += NI) {
+            so4_dbdr_pass<TWOJ>(A, c, e0, (int)(s1 - e0 < NI ? s1 - e0 : NI), dbdr);
+            __syncthreads();  // the next pass rewrites the LDS
+        }
     }
 }
 
@@ -2110,10 +2442,13 @@ extern "C" int pxff_so4_dbdr_centres(const pxff_so4_params *p, int64_t natoms, c
     // one workgroup per centre, rounded up to whole 64-centre tiles (the
     // centre map permutes within a tile; centres >= natoms exit)
     const unsigned grid = (unsigned)((natoms + 63) / 64 * 64);
-    PXFF_DISPATCH_TWOJ(p->twol, (so4_dbdr_centre_kernel<TJ><<<grid, 64, 0, s>>>(
-                                    natoms, d_img_start, d_img_j, d_img_r, d_atom_w, d_z, T->nz, T->nb, T->rootpq,
-                                    T->lnorm, T->blk_level_start, T->blk_zoff, T->blk_tb, T->blk_tf, p->rcut,
-                                    p->rfac0, p->cutoff_id, z_atom_major ? 1 : 0, d_dbdr)));
+    const DbArgs A{d_img_start, d_img_j,   d_img_r,   d_atom_w,  d_z,        T->nz,       p->cutoff_id,
+                   z_atom_major ? 1 : 0, T->db_nstage, T->db_tile, T->db_row, T->db_fac, T->db_coef, T->db_zmap,
+                   T->db_stage, p->rcut,   p->rfac0};
+    const unsigned rest = (unsigned)std::min<int64_t>(natoms, (int64_t)num_cus() * 4);
+    PXFF_DISPATCH_TWOJ(p->twol, (so4_dbdr_centre_kernel<TJ><<<grid, DbDim<TJ>::T, 0, s>>>(A, natoms, d_dbdr)));
+    PXFF_LAUNCH_CHECK();
+    PXFF_DISPATCH_TWOJ(p->twol, (so4_dbdr_rest_kernel<TJ><<<rest, DbDim<TJ>::T, 0, s>>>(A, natoms, d_dbdr)));
     PXFF_LAUNCH_CHECK();
     return 0;
 }

@@ -86,16 +86,6 @@ static int get_zchunks(int twol, int norm, int nch, int nzgroups, const int **ou
 // row.  Workgroup ids are mapped so that the chunks of one tile run on the
 // same XCD (workgroups are dispatched to the 8 XCDs round-robin), sharing
 // its L2.
-// Compile-time loop: f(std::integral_constant<int, 0>) ... f(<N-1>).
-template <typename F, int... I>
-__device__ inline void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ inline void static_for(F &&f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // Sign flip by XOR on the high word (m is 0 or 0x80000000).
 __device__ __forceinline__ double xsign(double x, uint32_t m) {
     return __hiloint2double(__double2hiint(x) ^ (int)m, __double2loint(x));

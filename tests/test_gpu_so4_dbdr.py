@@ -1,0 +1,35 @@
+"""The matrix-core dB/dr kernel against the per-image kernel at the edges of
+its tiles and passes: 16 images to a tile, 48 (2J = 10: 32) to the first
+pass, the rest in passes of the persistent kernel.
+
+Tolerance: both sum the same FP64 terms in another order, a few hundred per
+output, with rows of at most unit size: 1e-13 of the whole (norm), 1e-12 of
+the largest element for any single one."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# every centre of a cluster smaller than the cutoff has n - 1 images; 1 atom
+# (none) and 2 (one image) are the smallest
+@pytest.mark.parametrize("twol", [0, 2, 6, 8, 10])
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 18, 33, 34, 49, 50, 98])
+def test_dbdr_image_counts(n, twol):
+    from pyxtal_ff_amd import so4
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    rng = np.random.default_rng(100 * twol + n)
+    pos = rng.uniform(0.0, 2.6, (n, 3))
+    nl = DeviceNeighborList([pos], [np.eye(3) * 100.0], [np.zeros(3, bool)], 4.9)
+    assert nl.nimg == n * (n - 1)
+    cfg = so4.So4Config(twol, 4.9, 0.99363)
+    w = torch.rand(n, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda() + 0.5
+    _, z, _ = so4.forward(nl, cfg, w, w)
+    k = nl.nimg * cfg.nb * 3
+    ref = so4.dbdr_per_image(nl, cfg, w, z)[:k]
+    for atom_major in (False, True):
+        d = so4.dbdr(nl, cfg, w, z, atom_major=atom_major)[:k]
+        if k:
+            assert float((d - ref).norm() / ref.norm()) < 1e-13
+            assert float((d - ref).abs().max() / ref.abs().max()) < 1e-12
