@@ -362,6 +362,12 @@ int pxff_dxdr_contract_t(int64_t natoms, int nb, const int64_t *d_row_start, con
 int pxff_rdxdr_reduce(int64_t natoms, int nb, const int64_t *d_row_start, const double *d_rdxdr, double *d_out,
                       void *stream);
 
+/* Per-atom stress of the network's contraction (neuralnetwork.py:484-497):
+ * d_out [natoms*6] = -sum_b beta[i,b] rv[i,b,:] for d_beta [natoms*nb] and the
+ * per-atom Voigt rdxdr d_rv [natoms*nb*6] of pxff_rdxdr_reduce. */
+int pxff_voigt_contract(int64_t natoms, int nb, const double *d_beta, const double *d_rv, double *d_out,
+                        void *stream);
+
 /* Segmented sum over contiguous rows: out [nseg*ncol], out[s][c] = sum of
  * in[r][c] for r in [d_seg_start[s], d_seg_start[s+1]) (d_seg_start [nseg+1]
  * int64).  Per-structure energies / virials of a batch (the reference sums

@@ -73,6 +73,7 @@ _SIGS = {
     "pxff_dxdr_contract_t": ([I64, I32, P, P, P, P, P, P], I32),
     "pxff_dxdr_contract": ([I64, ctypes.c_int, P, P, P, P, P, P, P], I32),
     "pxff_rdxdr_reduce": ([I64, ctypes.c_int, P, P, P, P], I32),
+    "pxff_voigt_contract": ([I64, I32, P, P, P, P], I32),
     "pxff_so3_ctot": ([P, I64, P, P, P, P, P, P, P, P, P, P, P], I32),
     "pxff_so3_ctot_pairs": ([P, I64, P, P, P, P, P, P, P, P, P, P, P, I64, P, P], I32),
     "pxff_so3_forward_half": ([P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, P, P], I32),

@@ -1988,6 +1988,40 @@ __global__ void rdxdr_reduce_kernel(int64_t natoms, int nb, const int64_t *__res
     for (int k = 0; k < 6; k++) out[((size_t)i * nb + b) * 6 + k] = s[vo[k]];
 }
 
+// Stress of centre i in the network's contraction (neuralnetwork.py:484-497):
+// out[i, v] = -sum_b beta[i, b] rv[i, b, v] over the per-atom Voigt rdxdr.
+// Bound by reading rv once.  One wavefront per atom, 60 lanes: lane = (ten b,
+// component v), so that a lane keeps its component over the whole row and the
+// loads are contiguous; then the ten lanes of a component in a fixed order.
+// 1728 atoms, 55 components (4.6 MB): a few us, against 10.1 ms of a library
+// matrix-vector product over the flattened (atom, b) with six columns.
+__global__ __launch_bounds__(256) void voigt_contract_kernel(int64_t natoms, int nb, const double *__restrict__ beta,
+                                                              const double *__restrict__ rv,
+                                                              double *__restrict__ out) {
+    __shared__ double red[4][60];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t i = (int64_t)blockIdx.x * 4 + wv;
+    const bool in = i < natoms && lane < 60;
+    if (in) {
+        const double *be = beta + (size_t)i * nb, *r = rv + (size_t)i * nb * 6 + lane;
+        double s0 = 0.0, s1 = 0.0;
+        int b = lane / 6;
+        for (; b + 10 < nb; b += 20) {
+            s0 += be[b] * r[60 * (b / 10)];
+            s1 += be[b + 10] * r[60 * (b / 10 + 1)];
+        }
+        if (b < nb) s0 += be[b] * r[60 * (b / 10)];
+        red[wv][lane] = s0 + s1;
+    }
+    __syncthreads();
+    if (in && lane < 6) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 10; k++) s += red[wv][6 * k + lane];
+        out[6 * i + lane] = -s;
+    }
+}
+
 // ----------------------------------------------------------- tangent of B
 // dB_b = sum over the (block k, factor f) pairs targeting b of f p_k with
 // p_k = 2 Re sum_loc hw(loc) conj(dU^l[loc]) Z_k[loc] and dU = dU_tot (u_norm
@@ -2492,6 +2526,17 @@ extern "C" int pxff_rdxdr_reduce(int64_t natoms, int nb, const int64_t *d_row_st
     if (natoms <= 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     rdxdr_reduce_kernel<<<div_up(natoms * nb, 256), 256, 0, s>>>(natoms, nb, d_row_start, d_rdxdr, d_out);
+    PXFF_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int pxff_voigt_contract(int64_t natoms, int nb, const double *d_beta, const double *d_rv, double *d_out,
+                                   void *stream) {
+    if (natoms <= 0) return 0;
+    PXFF_REQUIRE(nb > 0, "nb must be > 0");
+    PXFF_REQUIRE(natoms <= 0x7fffffff, "too many atoms for one launch");
+    hipStream_t s = (hipStream_t)stream;
+    voigt_contract_kernel<<<div_up(natoms, 4), 256, 0, s>>>(natoms, nb, d_beta, d_rv, d_out);
     PXFF_LAUNCH_CHECK();
     return 0;
 }

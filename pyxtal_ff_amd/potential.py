@@ -267,7 +267,8 @@ def energy_forces_plain(nl, cfg, atom_w, site_w, model, species, stress=False):
     out = {"energy": e.detach(), "forces": -grad, "atom_energies": e_atom.detach()}
     if stress:
         rv = dev_so4.rdxdr_reduce(nl, cfg.nb, rd)  # [N, nb, 6]
-        out["stress_voigt"] = -torch.einsum("ik,ikl->l", beta, rv)
+        seg = nl.atom_start[:: len(nl.atom_start) - 1].contiguous()  # [0, N]
+        out["stress_voigt"] = _segment_total(dev_so4.voigt_contract(beta, rv), seg)
     return out
 
 

@@ -282,3 +282,14 @@ def rdxdr_reduce(nl, nb, rdxdr):
     nat.check(nat.lib().pxff_rdxdr_reduce(nl.natoms, nb, p(nl.row_start), p(rdxdr), p(out), nat.stream()),
               "pxff_rdxdr_reduce")
     return out[: nl.natoms * nb * 6].view(nl.natoms, nb, 6)
+
+
+def voigt_contract(beta, rv):
+    """Per-atom stress [N, 6] = -sum_b beta[i, b] rv[i, b, :] of the network's
+    contraction (neuralnetwork.py:484-497) over per-atom Voigt rdxdr."""
+    p = nat.ptr
+    n, nb = beta.shape
+    out = _f64(n * 6, beta.device)
+    beta, rv = beta.contiguous(), rv.contiguous()
+    nat.check(nat.lib().pxff_voigt_contract(n, nb, p(beta), p(rv), p(out), nat.stream()), "pxff_voigt_contract")
+    return out[: n * 6].view(n, 6)

@@ -92,7 +92,7 @@ def teacher_labels(desc, teacher, species, plain=True):
         (beta,) = torch.autograd.grad(e_atom.sum(), [xx])
         f = -dso4.dxdr_contract(nl, nf, beta, dx)
         rv = dso4.rdxdr_reduce(nl, nf, rd)  # [N, nf, 6]
-        s_atom = -torch.einsum("ik,ikl->il", beta, rv)
+        s_atom = dso4.voigt_contract(beta, rv)
         return (b.per_structure(e_atom.detach()), f.detach(),
                 (b.per_structure(s_atom) * EV2GPA).detach())
     from .batch import energy_forces_virial, stress_voigt
