@@ -342,6 +342,15 @@ int pxff_so4_rows(int64_t natoms, int nb, const int64_t *d_row_start, const int6
                   const int64_t *d_seq, const int64_t *d_nsite, const double *d_pos, const double *d_img_r,
                   const double *d_dbdr, const double *d_inv_vol, double *d_dxdr, double *d_rdxdr, void *stream);
 
+/* The dxdr rows of pxff_so4_rows and the per-atom Voigt rdxdr
+ * (utilities/__init__.py:226-235) in one pass, without the per-row rdxdr:
+ * d_rv [natoms*nb*6] as pxff_rdxdr_reduce over the rows gives it, with the
+ * absolute positions cancelled: 1/V sum over centre i's images of r (x) dB.
+ * NaN where 1/V is not finite. */
+int pxff_rows_voigt(int64_t natoms, int nb, const int64_t *d_row_start, const int64_t *d_row_img,
+                    const int64_t *d_nsite, const double *d_img_r, const double *d_dbdr, const double *d_inv_vol,
+                    double *d_dxdr, double *d_rv, void *stream);
+
 /* Plain path, force contraction (neuralnetwork.py:484-497, 657-677):
  * dE/dR_m = sum_{rows (i,m)} sum_b beta[i,b] dxdr[row,b,:], gathered per m
  * through the reverse-row index.  d_grad [natoms*3]. */

@@ -1788,55 +1788,119 @@ __global__ __launch_bounds__(DbDim<TWOJ>::T) __attribute__((amdgpu_waves_per_eu(
 }
 
 // -------------------------------------------------------------- row scatter
-// Reference layout rows (SNAP.py:1458-1468).  One workgroup per centre;
-// threads over the (b, k) / (b, a, c) components, looping over the centre's
-// rows in order -- no atomics, rows are owned by their centre.
-__global__ __launch_bounds__(256) void so4_rows_kernel(int64_t natoms, int nb, const int64_t *__restrict__ row_start,
+// Reference layout rows (SNAP.py:1458-1468).  One wavefront per (centre, 64
+// of the 3 nb columns (b, c)), four to a workgroup: a lane goes once through
+// the centre's images, eight loads in flight, and keeps the sums of the row
+// it is in and those over the whole centre, so dB/dr is read once for all
+// outputs; rows are owned by their centre, no atomics.  The images of a
+// centre's rows follow each other in memory, so the row ends are only
+// positions in that run: they come 64 at a time into a register and are
+// picked by lane.  Bound by memory.
+//   ROWS_DX    dxdr alone
+//   ROWS_FULL  and -bstress/V per row, bstress[nsite] += Ri (x) dB,
+//              bstress[row] -= Rj (x) dB
+//   ROWS_VOIGT and its sum over the centre's rows, in which the absolute
+//              positions cancel: 1/V sum_e r_e (x) dB, Voigt order
+// 1728 atoms, 28 images each, 55 components: dxdr and the Voigt sums 30 us
+// (130 MB read and written), before 92 us with the per-row rdxdr (a workgroup
+// per centre, two passes over its images, one load in flight) and 49 us for
+// its sum.  300 atoms, 73 images each, 126 components: dxdr and per-row rdxdr
+// 149 -> 49 us (270 MB).
+enum { ROWS_DX, ROWS_FULL, ROWS_VOIGT };
+
+template <int MODE>
+__global__ __launch_bounds__(256) void so4_rows_kernel(int64_t natoms, int nb, int nslice,
+                                                        const int64_t *__restrict__ row_start,
                                                         const int64_t *__restrict__ row_img,
-                                                        const int64_t *__restrict__ seq,
                                                         const int64_t *__restrict__ nsite,
                                                         const double *__restrict__ pos,
                                                         const double *__restrict__ img_r,
                                                         const double *__restrict__ dbdr,
                                                         const double *__restrict__ inv_vol, double *__restrict__ dxdr,
-                                                        double *__restrict__ rdxdr) {
-    const int64_t i = blockIdx.x;
+                                                        double *__restrict__ out) {
+    constexpr int U = 8;
+    const int lane = threadIdx.x & 63;
+    const int64_t unit = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t i = unit / nslice;
     if (i >= natoms) return;
+    const int nbk = nb * 3, t = (int)(unit - i * nslice) * 64 + lane;
+    const bool in = t < nbk;
+    const int tc = in ? t : nbk - 1;
+    const int b = tc / 3, c = tc - 3 * b;
     const int64_t r0 = row_start[i], r1 = row_start[i + 1], ns = nsite[i];
-    const int nbk = nb * 3;
-    for (int t = threadIdx.x; t < nbk; t += blockDim.x) {
-        double self = 0.0;
-        for (int64_t rw = r0; rw < r1; rw++) {
-            if (rw == ns) continue;
-            double v = 0.0;
-            for (int64_t e = row_img[rw]; e < row_img[rw + 1]; e++) v += dbdr[(size_t)e * nbk + t];
-            dxdr[(size_t)rw * nbk + t] = v;
+    const int64_t e0 = row_img[r0], e1 = row_img[r1];
+    double iv = 0.0, Ri[3] = {0.0, 0.0, 0.0};
+    if (MODE != ROWS_DX) iv = inv_vol[i];
+    if (MODE == ROWS_FULL)
+        for (int a = 0; a < 3; a++) Ri[a] = pos[3 * i + a];
+    double self = 0.0, v = 0.0, site[3] = {0.0, 0.0, 0.0}, w[3] = {0.0, 0.0, 0.0};
+    // ends of the rows rb .. rb + 63, relative to e0
+    int64_t rw = r0, rb = r0;
+    auto ends = [&](int64_t base) {
+        const int64_t k = base + lane;
+        return k < r1 ? (int)(row_img[k + 1] - e0) : 0x7fffffff;
+    };
+    int end = ends(rb);
+    int next = __builtin_amdgcn_readlane(end, 0);
+    const int n = (int)(e1 - e0);
+    auto close = [&]() {  // the row rw is complete
+        if (MODE == ROWS_FULL) {
+            if (rw == ns) {
+                for (int a = 0; a < 3; a++) site[a] += w[a];
+            } else if (in) {
+                for (int a = 0; a < 3; a++) out[(size_t)rw * 3 * nbk + 9 * b + 3 * a + c] = -w[a] * iv;
+            }
+            for (int a = 0; a < 3; a++) w[a] = 0.0;
+        }
+        if (rw != ns) {
+            if (in) dxdr[(size_t)rw * nbk + tc] = v;
             self -= v;
         }
-        dxdr[(size_t)ns * nbk + t] = self;
-    }
-    if (!rdxdr) return;
-    const double iv = inv_vol[i];
-    const double Ri[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-    const int nb9 = nb * 9;
-    for (int t = threadIdx.x; t < nb9; t += blockDim.x) {
-        const int b = t / 9, ac = t - b * 9, a = ac / 3, c = ac - a * 3;
-        double site = 0.0;
-        for (int64_t rw = r0; rw < r1; rw++) {
-            double v = 0.0;
-            for (int64_t e = row_img[rw]; e < row_img[rw + 1]; e++) {
-                const double db = dbdr[(size_t)e * nbk + 3 * b + c];
-                const double Rj = img_r[3 * e + a] + Ri[a];
-                site += Ri[a] * db;
-                v -= Rj * db;
-            }
-            if (rw == ns) {
-                site += v;
-            } else {
-                rdxdr[(size_t)rw * nb9 + t] = -v * iv;
-            }
+        v = 0.0;
+        rw++;
+        if (rw - rb == 64) {
+            rb = rw;
+            end = ends(rb);
         }
-        rdxdr[(size_t)ns * nb9 + t] = -site * iv;
+        next = __builtin_amdgcn_readlane(end, (int)(rw - rb));
+    };
+    const double *src = dbdr + (size_t)e0 * nbk + tc;
+    const double *rr = img_r + 3 * e0;
+    for (int e = 0; e < n; e += U) {
+        double d[U], x[U][3];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const int ek = e + k < n ? e + k : n - 1;
+            d[k] = src[(size_t)ek * nbk];
+            if (MODE != ROWS_DX)
+                for (int a = 0; a < 3; a++) x[k][a] = rr[3 * ek + a];
+        }
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            if (e + k >= n) break;  // uniform, as the row ends
+            while (e + k >= next) close();
+            v += d[k];
+            if (MODE == ROWS_VOIGT)
+                for (int a = 0; a < 3; a++) site[a] += x[k][a] * d[k];
+            if (MODE == ROWS_FULL)
+                for (int a = 0; a < 3; a++) {
+                    site[a] += Ri[a] * d[k];
+                    w[a] -= (x[k][a] + Ri[a]) * d[k];
+                }
+        }
+    }
+    while (rw < r1) close();
+    if (!in) return;
+    dxdr[(size_t)ns * nbk + tc] = self;
+    if (MODE == ROWS_FULL)
+        for (int a = 0; a < 3; a++) out[(size_t)ns * 3 * nbk + 9 * b + 3 * a + c] = -site[a] * iv;
+    if (MODE == ROWS_VOIGT) {
+        // (a, c) of the Voigt order xx yy zz xy xz yz; without a volume the
+        // rows are infinite with both signs and have no sum
+        const bool fin = fabs(iv) < __builtin_huge_val();
+        double *o = out + ((size_t)i * nb + b) * 6;
+        for (int a = 0; a < 3; a++)
+            if (a <= c) o[a == c ? a : a + c + 2] = fin ? site[a] * iv : __builtin_nan("");
     }
 }
 
@@ -2487,15 +2551,44 @@ extern "C" int pxff_so4_dbdr_centres(const pxff_so4_params *p, int64_t natoms, c
     return 0;
 }
 
+static int so4_rows_grid(int64_t natoms, int nb, int &nslice, unsigned &grid) {
+    PXFF_REQUIRE(nb > 0, "nb must be > 0");
+    nslice = (3 * nb + 63) / 64;
+    const int64_t g = (natoms * nslice + 3) / 4;
+    PXFF_REQUIRE(g <= 0x7fffffff, "too many rows for one launch");
+    grid = (unsigned)g;
+    return 0;
+}
+
 extern "C" int pxff_so4_rows(int64_t natoms, int nb, const int64_t *d_row_start, const int64_t *d_row_img,
                              const int64_t *d_seq, const int64_t *d_nsite, const double *d_pos, const double *d_img_r,
                              const double *d_dbdr, const double *d_inv_vol, double *d_dxdr, double *d_rdxdr,
                              void *stream) {
+    (void)d_seq;
     if (natoms <= 0) return 0;
-    PXFF_REQUIRE(nb > 0, "nb must be > 0");
+    int nslice = 0, rc = 0;
+    unsigned grid = 0;
+    if ((rc = so4_rows_grid(natoms, nb, nslice, grid))) return rc;
     hipStream_t s = (hipStream_t)stream;
-    so4_rows_kernel<<<(int)natoms, 256, 0, s>>>(natoms, nb, d_row_start, d_row_img, d_seq, d_nsite, d_pos, d_img_r,
-                                                 d_dbdr, d_inv_vol, d_dxdr, d_rdxdr);
+    if (d_rdxdr)
+        so4_rows_kernel<ROWS_FULL><<<grid, 256, 0, s>>>(natoms, nb, nslice, d_row_start, d_row_img, d_nsite, d_pos,
+                                                         d_img_r, d_dbdr, d_inv_vol, d_dxdr, d_rdxdr);
+    else
+        so4_rows_kernel<ROWS_DX><<<grid, 256, 0, s>>>(natoms, nb, nslice, d_row_start, d_row_img, d_nsite, d_pos,
+                                                       d_img_r, d_dbdr, d_inv_vol, d_dxdr, nullptr);
+    PXFF_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int pxff_rows_voigt(int64_t natoms, int nb, const int64_t *d_row_start, const int64_t *d_row_img,
+                               const int64_t *d_nsite, const double *d_img_r, const double *d_dbdr,
+                               const double *d_inv_vol, double *d_dxdr, double *d_rv, void *stream) {
+    if (natoms <= 0) return 0;
+    int nslice = 0, rc = 0;
+    unsigned grid = 0;
+    if ((rc = so4_rows_grid(natoms, nb, nslice, grid))) return rc;
+    so4_rows_kernel<ROWS_VOIGT><<<grid, 256, 0, (hipStream_t)stream>>>(
+        natoms, nb, nslice, d_row_start, d_row_img, d_nsite, nullptr, d_img_r, d_dbdr, d_inv_vol, d_dxdr, d_rv);
     PXFF_LAUNCH_CHECK();
     return 0;
 }

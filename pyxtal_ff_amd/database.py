@@ -31,12 +31,11 @@ def _plain_arrays(desc):
     if isinstance(desc, bt.BatchedSO3):
         x, ct, rad = dso3.forward(nl, desc.cfg, desc.state.atom_z, radial=True)
         nf = desc.cfg.ncoef
-        dx, rd = dso4.rows(nl, nf, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, ct, radial=rad), stress=True)
+        dx, rv = dso4.rows_voigt(nl, nf, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, ct, radial=rad))
     else:
         x, z, _ = dso4.forward(nl, desc.cfg, desc.atom_w, desc.site_w)
         nf = desc.cfg.nb
-        dx, rd = dso4.rows(nl, nf, dso4.dbdr(nl, desc.cfg, desc.atom_w, z), stress=True)
-    rv = dso4.rdxdr_reduce(nl, nf, rd)
+        dx, rv = dso4.rows_voigt(nl, nf, dso4.dbdr(nl, desc.cfg, desc.atom_w, z))
     return x, dx, rv
 
 

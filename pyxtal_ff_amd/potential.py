@@ -258,7 +258,10 @@ def energy_forces_plain(nl, cfg, atom_w, site_w, model, species, stress=False):
     nl.resolve()  # count settled before any kernel
     b, z, _ = dev_so4.forward(nl, cfg, atom_w, site_w)
     dbi = dev_so4.dbdr(nl, cfg, atom_w, z)
-    dx, rd = dev_so4.rows(nl, cfg.nb, dbi, stress=stress)
+    if stress:
+        dx, rv = dev_so4.rows_voigt(nl, cfg.nb, dbi)  # rv [N, nb, 6]
+    else:
+        dx, _ = dev_so4.rows(nl, cfg.nb, dbi, stress=False)
     x = b.detach().requires_grad_(True)
     e_atom = model.atom_energies(x, species)
     e = e_atom.sum()
@@ -266,7 +269,6 @@ def energy_forces_plain(nl, cfg, atom_w, site_w, model, species, stress=False):
     grad = dev_so4.dxdr_contract(nl, cfg.nb, beta, dx)
     out = {"energy": e.detach(), "forces": -grad, "atom_energies": e_atom.detach()}
     if stress:
-        rv = dev_so4.rdxdr_reduce(nl, cfg.nb, rd)  # [N, nb, 6]
         seg = nl.atom_start[:: len(nl.atom_start) - 1].contiguous()  # [0, N]
         out["stress_voigt"] = _segment_total(dev_so4.voigt_contract(beta, rv), seg)
     return out

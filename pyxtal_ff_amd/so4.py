@@ -254,6 +254,18 @@ def rows(nl, nb, dbdr_img, stress=True):
     return dx, rd
 
 
+def rows_voigt(nl, nb, dbdr_img):
+    """dxdr [nrows, nb, 3] of ``rows`` and the per-atom Voigt rdxdr [N, nb, 6]
+    that ``rdxdr_reduce`` makes of its per-row rdxdr, in one pass."""
+    p = nat.ptr
+    dev = nl.pos.device
+    dx = _f64(nl.nrows * nb * 3, dev)
+    rv = _f64(nl.natoms * nb * 6, dev)
+    nat.check(nat.lib().pxff_rows_voigt(nl.natoms, nb, p(nl.row_start), p(nl.row_img), p(nl.nsite), p(nl.img_r),
+                                        p(dbdr_img), p(nl.inv_vol), p(dx), p(rv), nat.stream()), "pxff_rows_voigt")
+    return dx[: nl.nrows * nb * 3].view(nl.nrows, nb, 3), rv[: nl.natoms * nb * 6].view(nl.natoms, nb, 6)
+
+
 def dxdr_contract(nl, nb, beta, dxdr):
     """dE/dR [N, 3] = sum over rows (i, m) of beta_i . dxdr[(i, m)]."""
     p = nat.ptr

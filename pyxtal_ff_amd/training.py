@@ -79,19 +79,17 @@ def teacher_labels(desc, teacher, species, plain=True):
     nl = b.nl.resolve()  # count settled before any kernel
     if plain and hasattr(desc, "atom_w"):
         x, z, _ = dso4.forward(nl, desc.cfg, desc.atom_w, desc.site_w)
-        dx, rd = dso4.rows(nl, desc.cfg.nb, dso4.dbdr(nl, desc.cfg, desc.atom_w, z), stress=True)
+        dx, rv = dso4.rows_voigt(nl, desc.cfg.nb, dso4.dbdr(nl, desc.cfg, desc.atom_w, z))
         nf = desc.cfg.nb
     elif plain:
         x, ct, rad = dso3.forward(nl, desc.cfg, desc.state.atom_z, radial=True)
-        dx, rd = dso4.rows(nl, desc.cfg.ncoef, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, ct, radial=rad),
-                           stress=True)
+        dx, rv = dso4.rows_voigt(nl, desc.cfg.ncoef, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, ct, radial=rad))
         nf = desc.cfg.ncoef
     if plain:
         xx = x.detach().requires_grad_(True)
         e_atom = teacher.atom_energies(xx, species)
         (beta,) = torch.autograd.grad(e_atom.sum(), [xx])
         f = -dso4.dxdr_contract(nl, nf, beta, dx)
-        rv = dso4.rdxdr_reduce(nl, nf, rd)  # [N, nf, 6]
         s_atom = dso4.voigt_contract(beta, rv)
         return (b.per_structure(e_atom.detach()), f.detach(),
                 (b.per_structure(s_atom) * EV2GPA).detach())
@@ -169,15 +167,14 @@ class ForceTrainer:
             with torch.no_grad():
                 if hasattr(desc, "atom_w"):
                     self.nf = desc.cfg.nb
-                    dx, rd = dso4.rows(nl, self.nf, dso4.dbdr(nl, desc.cfg, desc.atom_w, self.z), stress=True)
+                    dx, rv = dso4.rows_voigt(nl, self.nf, dso4.dbdr(nl, desc.cfg, desc.atom_w, self.z))
                 else:
                     from . import so3 as dso3
                     self.nf = desc.cfg.ncoef
-                    dx, rd = dso4.rows(nl, self.nf, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, self.ct,
-                                                              radial=self.rad), stress=True)
+                    dx, rv = dso4.rows_voigt(nl, self.nf, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, self.ct,
+                                                                    radial=self.rad))
                 self.dx = dx
-                self.rv = dso4.rdxdr_reduce(nl, self.nf, rd)  # [N, nf, 6], Voigt
-                del rd
+                self.rv = rv  # [N, nf, 6], Voigt
         self.n_struct = torch.as_tensor(b.counts, dtype=torch.float64, device=dev)
         self._voigt = torch.as_tensor([3 * i + j for i, j in zip(*VOIGT)], dtype=torch.int64, device=dev)
         # Adam keeps its step count on the device when the step is captured;

@@ -24,3 +24,62 @@ def test_voigt_contract(n, nb):
     # operands off the natural layout are copied first
     bt = beta.t().contiguous().cuda().t()
     assert torch.equal(so4.voigt_contract(bt, rv.cuda()).cpu(), out)
+
+
+def _list(kind):
+    import numpy as np
+    from pyxtal_ff_amd import workloads
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    rng = np.random.default_rng(7)
+    if kind == "one":  # no images
+        pos, cell, pbc, rc = np.zeros((1, 3)), np.eye(3) * 20.0, [False] * 3, 4.0
+    elif kind == "small":  # self images, several images to a row
+        pos, cell, pbc, rc = rng.uniform(0, 3.0, (3, 3)), np.eye(3) * 3.0, [True] * 3, 5.0
+    elif kind == "cluster":  # 99 rows of one image, another atom out of reach
+        pos, cell, pbc, rc = rng.uniform(0, 2.6, (100, 3)), np.eye(3) * 50.0, [False] * 3, 4.9
+        pos[57] = 25.0
+    else:
+        s = workloads.amorphous_sio2(30, 61, seed=3)
+        pos, cell, pbc, rc = s.positions, s.cell, s.pbc, 4.6
+    return DeviceNeighborList([pos], [cell], [np.asarray(pbc)], rc).resolve()
+
+
+@pytest.mark.parametrize("kind", ["one", "small", "cluster", "sio"])
+@pytest.mark.parametrize("nb", [1, 21, 22, 43, 55])  # 64 columns (b, c) to a wavefront
+def test_rows(kind, nb):
+    from pyxtal_ff_amd import so4
+    nl = _list(kind)
+    ne, nr, n = nl.nimg, nl.nrows, nl.natoms
+    g = torch.Generator().manual_seed(nb)
+    db = torch.randn((max(ne, 1), nb, 3), dtype=torch.float64, generator=g)
+    seq, r = nl.seq_array().cpu(), nl.img_r[: 3 * ne].view(-1, 3).cpu()
+    pos, iv = nl.pos.view(-1, 3).cpu(), nl.inv_vol.cpu()
+    row = nl.row_img.cpu()
+    e_row = torch.repeat_interleave(torch.arange(nr), row[1 : nr + 1] - row[:nr])
+    i = seq[e_row, 0]
+    rowsum = torch.zeros((nr, nb, 3), dtype=torch.float64).index_add_(0, e_row, db[:ne])
+    own = seq[:, 0] == seq[:, 1]
+    dx_ref = rowsum.clone()
+    dx_ref[own] = 0
+    dx_ref[own] = -torch.zeros((n, nb, 3), dtype=torch.float64).index_add_(0, seq[:, 0], dx_ref)
+    # bstress[row] -= Rj (x) dB, bstress[nsite] += Ri (x) dB
+    bs = torch.zeros((nr, nb, 3, 3), dtype=torch.float64)
+    bs.index_add_(0, e_row, -(r + pos[i])[:, None, :, None] * db[:ne, :, None, :])
+    ns = nl.nsite.cpu()
+    bs.index_add_(0, ns[i], pos[i][:, None, :, None] * db[:ne, :, None, :])
+    rd_ref = -bs * iv[seq[:, 0]][:, None, None, None]
+    rv_ref = torch.zeros((n, nb, 3, 3), dtype=torch.float64).index_add_(
+        0, i, r[:, None, :, None] * db[:ne, :, None, :]) * iv[:, None, None, None]
+    rv_ref = rv_ref.view(n, nb, 9)[:, :, [0, 4, 8, 1, 2, 5]]
+    dbd = db.cuda().contiguous()
+    dx, rd = so4.rows(nl, nb, dbd, stress=True)
+    dx1, none = so4.rows(nl, nb, dbd, stress=False)
+    dx2, rv = so4.rows_voigt(nl, nb, dbd)
+    assert none is None and torch.equal(dx, dx1) and torch.equal(dx, dx2)
+    for a, ref in ((dx, dx_ref), (rd, rd_ref), (rv, rv_ref)):
+        assert a.shape == ref.shape
+        if ref.any():
+            assert _rel(a.cpu(), ref) < 1e-13
+        else:
+            assert not a.cpu().any()
+    assert _rel(so4.rdxdr_reduce(nl, nb, rd), rv) < 1e-10 if ne else True  # the positions cancel
