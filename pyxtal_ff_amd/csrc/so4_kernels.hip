@@ -1804,8 +1804,8 @@ __global__ __launch_bounds__(DbDim<TWOJ>::T) __attribute__((amdgpu_waves_per_eu(
 // 1728 atoms, 28 images each, 55 components: dxdr and the Voigt sums 30 us
 // (130 MB read and written), before 92 us with the per-row rdxdr (a workgroup
 // per centre, two passes over its images, one load in flight) and 49 us for
-// its sum.  300 atoms, 73 images each, 126 components: dxdr and per-row rdxdr
-// 149 -> 49 us (270 MB).
+// its sum.  300 atoms, 48 images each, 147 components: dxdr and per-row rdxdr
+// 149 -> 49 us (255 MB).
 enum { ROWS_DX, ROWS_FULL, ROWS_VOIGT };
 
 template <int MODE>
