@@ -311,39 +311,66 @@ __device__ __forceinline__ void nl_fill_serial(int64_t i, const double *__restri
 }
 
 // seq rows: for centre i, ascending unique j with (i, i) inserted
-// (SNAP.py:279-296).
-__global__ void nl_rows_kernel(int64_t natoms, int64_t nimg, const int64_t *__restrict__ img_start,
-                               const int64_t *__restrict__ img_j, const int64_t *__restrict__ row_start,
-                               int64_t *__restrict__ seq, int64_t *__restrict__ row_img, int64_t *__restrict__ img_row,
-                               int64_t *__restrict__ nsite) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// (SNAP.py:279-296).  One wavefront per centre, lanes over its images 64 at a
+// time: an image's row is the number of neighbour changes up to it, counted
+// by ballot, plus one past a (i, i) row without images of its own.  Bound by
+// latency: one thread per centre, walking its images one load after the
+// other, took 22 us for 28 images (1728 atoms) and 34 us for 48 (300 atoms);
+// 3.4 us now.
+__global__ __launch_bounds__(256) void nl_rows_kernel(int64_t natoms, int64_t nimg,
+                                                      const int64_t *__restrict__ img_start,
+                                                      const int64_t *__restrict__ img_j,
+                                                      const int64_t *__restrict__ row_start, int64_t *__restrict__ seq,
+                                                      int64_t *__restrict__ row_img, int64_t *__restrict__ img_row,
+                                                      int64_t *__restrict__ nsite) {
+    const int lane = threadIdx.x & 63;
+    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= natoms) return;
-    int64_t rw = row_start[i];
-    const int64_t s0 = img_start[i], s1 = img_start[i + 1];
-    bool self_done = false;
-    int64_t a = s0;
-    while (a < s1 || !self_done) {
-        int64_t j = (a < s1) ? img_j[a] : INT64_MAX;
-        if (!self_done && i <= j) {
-            // (i, i) row: with the self images if j == i, else empty
-            seq[2 * rw] = i;
-            seq[2 * rw + 1] = i;
-            nsite[i] = rw;
-            row_img[rw] = a;
-            if (j == i) {
-                while (a < s1 && img_j[a] == i) img_row[a++] = rw;
+    const int64_t s0 = img_start[i], s1 = img_start[i + 1], r0 = row_start[i];
+    int64_t rw = r0;           // row of the next neighbour
+    int64_t prev = -1;         // neighbour before this chunk
+    int64_t own = -1, at = s1;  // the (i, i) row, and where it goes without images
+    for (int64_t a0 = s0; a0 < s1; a0 += 64) {
+        const int64_t a = a0 + lane;
+        const bool in = a < s1;
+        const int64_t j = in ? img_j[a] : INT64_MAX;
+        int64_t before = __shfl_up(j, 1);
+        if (lane == 0) before = prev;
+        const bool first = in && j != before;
+        const uint64_t firsts = __ballot(first), below = __ballot(in && j < i), self = __ballot(in && j == i);
+        const uint64_t upto = lane == 63 ? ~0ull : (1ull << (lane + 1)) - 1;
+        const int64_t past = __popcll(firsts & upto);
+        if (own < 0) {
+            const int nb = __popcll(below);
+            if (self) {
+                own = rw + __popcll(firsts & below);
+            } else if (nb < 64 && a0 + nb < s1) {  // the first larger neighbour is in this chunk
+                own = rw + __popcll(firsts & below);
+                at = a0 + nb;
             }
-            self_done = true;
-            rw++;
-            continue;
         }
-        seq[2 * rw] = i;
-        seq[2 * rw + 1] = j;
-        row_img[rw] = a;
-        while (a < s1 && img_j[a] == j) img_row[a++] = rw;
-        rw++;
+        // an own row without images shifts the larger neighbours by one
+        const int64_t row = rw + past - 1 + (at != s1 && j > i ? 1 : 0);
+        if (in) img_row[a] = row;
+        if (first) {
+            seq[2 * row] = i;
+            seq[2 * row + 1] = j;
+            row_img[row] = a;
+        }
+        rw += __popcll(firsts);
+        prev = __shfl(j, 63);
     }
-    if (i == natoms - 1) row_img[rw] = nimg;
+    const bool empty = own < 0 || at != s1;  // no images of its own
+    if (lane == 0) {
+        if (own < 0) own = rw;
+        if (empty) {
+            seq[2 * own] = i;
+            seq[2 * own + 1] = i;
+            row_img[own] = at;
+        }
+        nsite[i] = own;
+        if (i == natoms - 1) row_img[rw + (empty ? 1 : 0)] = nimg;
+    }
 }
 
 // reverse image (j, i, -T) and reverse row (j, i) by binary search in centre
@@ -1023,7 +1050,7 @@ extern "C" int pxff_nlist_rows(int64_t natoms, int64_t nimg, int64_t nrows, cons
     hipStream_t s = (hipStream_t)stream;
     nl_zero_i32_kernel<<<1, 64, 0, s>>>(d_flag, 1);
     PXFF_LAUNCH_CHECK();
-    nl_rows_kernel<<<div_up(natoms, 64), 64, 0, s>>>(natoms, nimg, d_img_start, d_img_j, d_row_start, d_seq, d_row_img,
+    nl_rows_kernel<<<div_up(natoms, 4), 256, 0, s>>>(natoms, nimg, d_img_start, d_img_j, d_row_start, d_seq, d_row_img,
                                                      d_img_row, d_nsite);
     PXFF_LAUNCH_CHECK();
     nl_row_rev_kernel<<<div_up(nrows, 256), 256, 0, s>>>(nrows, d_seq, d_row_start, d_row_rev, d_flag);

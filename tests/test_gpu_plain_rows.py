@@ -83,3 +83,35 @@ def test_rows(kind, nb):
         else:
             assert not a.cpu().any()
     assert _rel(so4.rdxdr_reduce(nl, nb, rd), rv) < 1e-10 if ne else True  # the positions cancel
+
+
+# 64 images to a pass of the wavefront: centres below, at and past one and two
+# passes; the own row first, last and in between, with images of its own and
+# without; an isolated atom
+@pytest.mark.parametrize("kind", ["one", "small", "tiny", "cluster", "sio", 64, 65, 66, 129, 130])
+def test_row_index(kind):
+    import numpy as np
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    if isinstance(kind, int):  # every atom sees the others
+        pos = np.random.default_rng(kind).uniform(0, 2.6, (kind, 3))
+        nl = DeviceNeighborList([pos], [np.eye(3) * 50.0], [np.zeros(3, bool)], 4.9).resolve()
+    elif kind == "tiny":  # one atom, all images its own, several passes
+        nl = DeviceNeighborList([np.zeros((1, 3))], [np.eye(3) * 1.5], [np.ones(3, bool)], 5.0).resolve()
+    else:
+        nl = _list(kind)
+    start, j = nl.img_start.cpu().numpy(), nl.img_j.cpu().numpy()
+    seq, row_img, img_row, nsite = [], [], [], []
+    for i in range(nl.natoms):
+        mine = j[start[i]: start[i + 1]]
+        for k in np.unique(np.append(mine, i)):
+            if k == i:
+                nsite.append(len(seq))
+            row_img.append(start[i] + np.searchsorted(mine, k))
+            img_row += [len(seq)] * int((mine == k).sum())
+            seq.append((i, k))
+    row_img.append(nl.nimg)
+    n = len(seq)
+    assert nl.nrows == n and np.array_equal(nl.seq_array().cpu().numpy(), np.array(seq))
+    assert np.array_equal(nl.row_img.cpu().numpy()[: n + 1], row_img)
+    assert np.array_equal(nl.img_row.cpu().numpy()[: nl.nimg], np.array(img_row, dtype=np.int64))
+    assert np.array_equal(nl.nsite.cpu().numpy(), nsite)
