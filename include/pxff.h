@@ -403,6 +403,14 @@ int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const int64_t *d_sp
                          const int *d_layout, const double *d_params, const double *d_dmin, const double *d_scale,
                          const double *d_x, double *d_e, double *d_beta, void *stream);
 
+/* The packed arrays of pxff_mlp_energy_grad from the parameters' own tensors,
+ * one launch per element, nothing kept: h_tensors [nelem * (2 + 2*8)] device
+ * pointers {dmin, scale, W_0, b_0, W_1, b_1, ...}, W row-major [nout][nin];
+ * d_layout [nelem * (1 + 6*8)], d_params at the offsets of h_layout, d_dmin
+ * and d_scale [nelem*nin]. */
+int pxff_mlp_pack(int nin, int nelem, const int *h_layout, const double *const *h_tensors, int *d_layout,
+                  double *d_params, double *d_dmin, double *d_scale, void *stream);
+
 /* ------------------------------------------------------------------ *
  * SO(3) power spectrum (replaces SO3.calculate / compute_cs /          *
  * compute_dcs, SO3.py:187-291, 504-694).                               *

@@ -64,6 +64,17 @@ def make_descriptor(sb, descriptor, semantics="database"):
     raise NotImplementedError(f"{t} is not implemented")
 
 
+class _Network:
+    """The network step of a calculator's fused evaluation."""
+
+    def __init__(self, calc):
+        self._c = calc
+
+    def energy_grad(self, x, _):
+        c = self._c
+        return pot.energy_and_gradient(c.model, x, c._species, c._species_atom)
+
+
 class PyXtalFFCalculator(_Base):
     implemented_properties = ["energy", "forces", "stress"]
     nolabel = True
@@ -92,6 +103,10 @@ class PyXtalFFCalculator(_Base):
             # the descriptor is built as the reference's compute_descriptor builds it
             self._desc = make_descriptor(self._sb, self.descriptor, semantics="calculator")
             self._species = pot.species_index(self._sb.symbols, self.model.elements, self.device)
+            present = [e for e, _ in self._species]
+            # every atom's network, if each atom has one
+            self._species_atom = (pot.species_atom(self._sb.symbols, present, self.device)
+                                  if set(self._sb.symbols) == set(present) else None)
             self._key = key
         else:
             pos = torch.as_tensor(np.asarray(atoms.positions, dtype=np.float64), device=self.device)
@@ -104,14 +119,18 @@ class PyXtalFFCalculator(_Base):
             _Base.calculate(self, atoms, properties, system_changes)
             atoms = self.atoms
         self._setup(atoms)
-        o = bt.energy_forces_virial(self._desc, self.model, self._species, virial=True)
-        e_atom = o["atom_energies"]
-        sv = bt.stress_voigt(o["virial"], self._sb)[0]  # eV/A^3, (xx, yy, zz, xy, xz, yz)
-        stress_ml = (sv * EV2GPA).detach().cpu().numpy()
-        self.results["energies"] = e_atom.detach().cpu().numpy()
-        self.results["energy"] = float(o["energy"][0])
+        # the kernels of the fused step, and one copy back
+        o = pot.energy_forces_fused(self._sb.nl, self._desc.state, _Network(self), None, virial=True)
+        n = len(o["atom_energies"])
+        host = torch.cat([o["energy"].view(1), o["virial"].view(9), o["atom_energies"],
+                          o["forces"].reshape(-1)]).cpu().numpy()
+        w = host[1:10].reshape(1, 3, 3)
+        sv = (-w[:, bt.VOIGT[0], bt.VOIGT[1]] * (1.0 / self._sb.volumes)[:, None])[0]  # eV/A^3, (xx, yy, zz, xy, xz, yz)
+        stress_ml = sv * EV2GPA
+        self.results["energies"] = host[10: 10 + n].copy()
+        self.results["energy"] = float(host[0])
         self.results["free_energy"] = self.results["energy"]
-        self.results["forces"] = o["forces"].detach().cpu().numpy()
+        self.results["forces"] = host[10 + n:].reshape(n, 3).copy()
         self.results["stress_ml"] = stress_ml
         self.results["energy_ml"] = self.results["energy"]
         self.results["forces_ml"] = self.results["forces"]

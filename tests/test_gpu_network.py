@@ -54,3 +54,56 @@ def test_fused_network_unknown_species_gives_nan():
     keep = torch.ones(n, dtype=torch.bool, device="cuda")
     keep[3] = False
     assert torch.isfinite(e[keep]).all() and torch.isfinite(beta[keep]).all()
+
+
+@pytest.mark.parametrize("elements,hidden,act", [(["Si"], (30, 30), "Tanh"), (["O", "Si", "C"], (24, 16, 8), "ReLU"),
+                                                 (["O", "Si"], (), "Tanh"), (["O", "Si"], (64,) * 7, "Sigmoid")])
+def test_energy_and_gradient_matches_autograd(elements, hidden, act):
+    """The parameters taken at the call, compact rows per element: atoms
+    without a network stay zero, parameters changed through .data or replaced
+    are seen, and a model the kernel cannot stand for goes through autograd
+    (a hooked layer, a subclass).  Tolerances as for the packed kernel."""
+    nin, n = 21, 77
+    rng = np.random.default_rng(len(elements))
+    symbols = list(rng.choice(elements + ["H"], size=n))
+    dr = {e: np.stack([np.full(nin, -0.1), np.full(nin, 1.2)], 1) for e in elements}
+    model = potential.NNPotential(elements, nin, hidden, seed=7, drange=dr, activation=act).cuda()
+    x = torch.as_tensor(rng.random((n, nin)), dtype=torch.float64, device="cuda")
+    species = potential.species_index(symbols, model.elements, "cuda")
+
+    def same(m):
+        e, g = potential.energy_and_gradient(m, x, species)
+        e_ref, g_ref = _torch_reference(m, x, symbols)
+        assert not e.requires_grad and not g.requires_grad
+        assert rel_err(e.cpu().numpy(), e_ref.cpu().numpy()) < 1e-13
+        assert rel_err(g.cpu().numpy(), g_ref.cpu().numpy()) < 1e-12
+        return e
+
+    assert potential._networks(model, x, species) is not None
+    e0 = same(model)
+    lin = model.models[elements[0]].layers[0]
+    lin.weight.data.mul_(1.5)  # bumps no version
+    e1 = same(model)
+    assert not torch.equal(e0, e1)
+    lin.weight = torch.nn.Parameter(0.5 * lin.weight.detach())
+    assert not torch.equal(e1, same(model))
+    h = lin.register_forward_hook(lambda mod, a, out: 2.0 * out)
+    assert potential._networks(model, x, species) is None
+    same(model)
+    h.remove()
+    covered = [s for s in symbols if s in elements]
+    keep = torch.as_tensor([k for k, s in enumerate(symbols) if s in elements], device="cuda")
+    xs = x[keep].contiguous()
+    sp = potential.species_index(covered, model.elements, "cuda")
+    at = potential.species_atom(covered, [e for e, _ in sp], "cuda")
+    a, b = potential.energy_and_gradient(model, xs, sp, at), potential.energy_and_gradient(model, xs, sp)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    with torch.no_grad():  # refused, as autograd refuses it
+        with pytest.raises(RuntimeError):
+            potential.energy_and_gradient(model, x, species)
+
+    class Other(potential.NNPotential):
+        pass
+
+    model.__class__ = Other
+    assert potential._networks(model, x, species) is None
