@@ -239,13 +239,25 @@ __global__ __launch_bounds__(64 * MLP_LW) void mlp_lds_kernel(int64_t natoms, in
 }
 
 // ---------------------------------------------------------- matrix cores
-// 16 atoms per workgroup of four wavefronts; every layer is a GEMM on the
+// 16 atoms per workgroup of eight wavefronts; every layer is a GEMM on the
 // FP64 matrix cores (v_mfma_f64_16x16x4_f64: A[i][k] in lane i + 16 k,
-// B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i % 4), element i / 4),
-// one 16-wide column tile per wavefront, activations and their derivatives
-// through LDS.  Forward, per 16-neuron tile: Z^T = W_k H_{k-1}^T (A = W_k,
-// B = H^T), H_k = act(Z + b_k); backward: G_{k-1} = (G_k W_k) * act'_{k-1}
-// (A = G_k, B = W_k), dE/dx = (G_0 W_0) * scale.
+// B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i % 4), element i / 4).
+// Forward, per 16-neuron tile: Z^T = W_k H_{k-1}^T (A = W_k, B = H^T),
+// H_k = act(Z + b_k); backward: G_{k-1} = (G_k W_k) * act'_{k-1} (A = G_k,
+// B = W_k), dE/dx = (G_0 W_0) * scale.
+// Bound by the latency of its chain (a handful of layers, each a few products
+// and one activation), not by any rate, so every step is spread over the
+// whole workgroup: the wavefronts of a tile split the sum over k (ks parts,
+// added through LDS), and then a thread has one (atom, neuron) for the
+// activation, whose tanh is the longest link of the chain.  The tile's inputs
+// and species are on their way before the element is known, those of the next
+// tile before this one is computed; the weights come a row per wavefront,
+// eight rows in flight; the layout is one register, an int per lane.
+// Four wavefronts with whole tiles and four activations to a lane, before:
+// 1000 atoms of 30 inputs 16.3 -> 13.3 us, 777 atoms of 55 inputs with two
+// elements mixed 32.6 -> 23.7, 4096 of 55 18.7 -> 14.1, 12000 of 147 65 -> 43,
+// 200000 of 55 411 -> 330; past 50000 atoms of 30 inputs, where the tanh are
+// most of the work and the call costs, 89 -> 94 us (286 -> 312 at 200000).
 // The element's weights are staged in LDS first, zero-padded, and every
 // activation row is zero past its width, so the GEMM steps need no bounds
 // tests (the K loops run over multiples of 4).  LDS rows are 2 doubles past
@@ -254,172 +266,226 @@ __global__ __launch_bounds__(64 * MLP_LW) void mlp_lds_kernel(int64_t natoms, in
 // runs the network of every element present and keeps each atom's own
 // results.
 typedef double mlp_d4 __attribute__((ext_vector_type(4)));
-constexpr int MLP_TILE = 16;
+constexpr int MLP_TILE = 16, MLP_WV = 8, MLP_T = 64 * MLP_WV;
+constexpr int MLP_XC = 3;          // 64-column groups of a tile's inputs held in registers
+constexpr int MLP_ZP = 16 * 17;    // doubles of one wavefront's partial tile
 
 __host__ __device__ inline int mlp_r16(int n) { return (n + 15) & ~15; }
 __host__ __device__ inline int mlp_r4(int n) { return (n + 3) & ~3; }
 __host__ __device__ inline int mlp_row(int n) { return ((n + 31) & ~31) + 2; }  // LDS row stride
 
-// acc = sum_k A[lane & 15][k] B[k][col], k < K (a multiple of 4):
-// a = &A[lane & 15][lane >> 4] (row-major A, k steps of 4 elements),
-// b = &B[lane >> 4][col], bstep = 4 x the row stride of B.  Four
-// accumulators take the k steps in turn (four independent MFMA chains).
-__device__ inline mlp_d4 mlp_gemm_tile(int K, const double *a, const double *b, int bstep) {
-    mlp_d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0, c2 = c0, c3 = c0;
-    const int S = K >> 2;
-    int t = 0;
-    for (; t + 4 <= S; t += 4) {
-        const double a0 = a[4 * t], a1 = a[4 * t + 4], a2 = a[4 * t + 8], a3 = a[4 * t + 12];
-        const double b0 = b[t * bstep], b1 = b[(t + 1) * bstep], b2 = b[(t + 2) * bstep], b3 = b[(t + 3) * bstep];
-        c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, c0, 0, 0, 0);
-        c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, c1, 0, 0, 0);
-        c2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, b2, c2, 0, 0, 0);
-        c3 = __builtin_amdgcn_mfma_f64_16x16x4f64(a3, b3, c3, 0, 0, 0);
-    }
-    for (; t < S; t++) c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[4 * t], b[t * bstep], c0, 0, 0, 0);
-    return (c0 + c1) + (c2 + c3);
+// Parts the k sum of a layer with t tiles is split into, with room for zp
+// partial tiles: a power of two, t * parts <= min(wavefronts, zp).
+__host__ __device__ inline int mlp_parts(int t, int zp) {
+    const int m = zp < MLP_WV ? zp : MLP_WV;
+    return t >= m ? 1 : (8 * t <= m ? 8 : (4 * t <= m ? 4 : (2 * t <= m ? 2 : 1)));
 }
 
-__global__ __launch_bounds__(256) void mlp_mfma_kernel(int64_t natoms, int nin, int nelem,
-                                                        const int64_t *__restrict__ species,
-                                                        const int *__restrict__ layout,
-                                                        const double *__restrict__ params,
-                                                        const double *__restrict__ dmin,
-                                                        const double *__restrict__ scale,
-                                                        const double *__restrict__ x, double *__restrict__ e_out,
-                                                        double *__restrict__ beta, int nlm, int hw) {
+// acc = sum over the steps t = t0, t0 + ts, ... < S of A[lane & 15][4t ..] x
+// B[4t ..][col]: a = &A[lane & 15][lane >> 4] (row-major A), b = &B[lane >>
+// 4][col], bstep = 4 x the row stride of B.  Two accumulators in turn.
+__device__ inline mlp_d4 mlp_gemm_part(int t0, int ts, int S, const double *a, const double *b, int bstep) {
+    mlp_d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0;
+    int t = t0;
+    for (; t + ts < S; t += 2 * ts) {
+        const double a0 = a[4 * t], a1 = a[4 * (t + ts)], b0 = b[t * bstep], b1 = b[(t + ts) * bstep];
+        c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, c1, 0, 0, 0);
+    }
+    if (t < S) c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[4 * t], b[t * bstep], c0, 0, 0, 0);
+    return c0 + c1;
+}
+
+// A call, not inlined: in the loops over tiles, elements and layers the
+// constants of the exponentials were otherwise held in registers throughout
+// (186 spilled).
+__device__ __attribute__((noinline)) double2 mlp_act(int act, double z) {
+    double a, da;
+    act_fdf(act, z, a, da);
+    return make_double2(a, da);
+}
+
+// nbuf: activation buffers ([16][HP] each); zpn: partial tiles.
+__global__ __launch_bounds__(MLP_T) __attribute__((amdgpu_waves_per_eu(4))) void mlp_mfma_kernel(int64_t natoms, int nin, int nelem,
+                                                         const int64_t *__restrict__ species,
+                                                         const int *__restrict__ layout,
+                                                         const double *__restrict__ params,
+                                                         const double *__restrict__ dmin,
+                                                         const double *__restrict__ scale,
+                                                         const double *__restrict__ x, double *__restrict__ e_out,
+                                                         double *__restrict__ beta, int nlm, int hw, int nbuf, int zpn) {
+    constexpr int AR = MLP_TILE / MLP_WV, RU = MLP_MAXW / MLP_WV;  // atoms and rows of W per wavefront
     extern __shared__ double sm[];
     __shared__ int s_sp[MLP_TILE];  // element of each atom; -1 no network, -2 past the end
     __shared__ int s_wo[MLP_MAXL];  // offset of layer k's padded W, then its b, in wl
     const int P0 = mlp_row(nin), HP = mlp_row(hw);
-    double *h0 = sm;                                 // [16][P0] scaled inputs, zero-padded
-    double *hact = h0 + MLP_TILE * P0;               // [nlm][16][HP] activations
-    double *hder = hact + (size_t)nlm * MLP_TILE * HP;  // [nlm][16][HP] act', then gradients
-    double *wl = hder + (size_t)nlm * MLP_TILE * HP;    // W_k [r16(nout)][row(nin)], b_k [r16(nout)]
-    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    double *h0 = sm;                                     // [16][P0] scaled inputs, zero-padded
+    double *hact = h0 + MLP_TILE * P0;                   // [nbuf][16][HP] activations of the hidden layers, in turn
+    double *hder = hact + (size_t)nbuf * MLP_TILE * HP;  // [nlm][16][HP] act', then gradients
+    double *zp = hder + (size_t)nlm * MLP_TILE * HP;     // [zpn] partial tiles
+    double *wl = zp + (size_t)zpn * MLP_ZP;              // W_k [r16(nout)][row(nin)], b_k [r16(nout)]
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int ri = lane & 15, kq = lane >> 4;
+    const int ta = tid & 15, tn = tid >> 4;  // the thread's atom and neuron in the combining steps
     // tiles [t0, t1) of this workgroup, in order: an element's weights stay
     // staged from one tile to the next (atoms come sorted by element)
     const int64_t ntiles = (natoms + MLP_TILE - 1) / MLP_TILE;
     const int64_t per = (ntiles + gridDim.x - 1) / gridDim.x;
     const int64_t t0 = (int64_t)blockIdx.x * per, t1 = t0 + per < ntiles ? t0 + per : ntiles;
     int staged = -1;  // element whose weights are in wl
+    // wavefront w loads the inputs of atoms AR w .. AR w + AR - 1
+    double xv[AR * MLP_XC];
+    int64_t spv = 0;
+    auto fetch = [&](int64_t a0) __attribute__((always_inline)) {
+        if (tid < MLP_TILE) spv = a0 + tid < natoms ? species[a0 + tid] : 0;
+#pragma unroll
+        for (int u = 0; u < AR * MLP_XC; u++) {
+            const int64_t a = a0 + AR * wv + u % AR;
+            const int c = u / AR * 64 + lane;
+            xv[u] = a < natoms && c < nin ? x[(size_t)a * nin + c] : 0.0;
+        }
+    };
+    if (t0 < t1) fetch(t0 * MLP_TILE);
+    // an element's layout in one register, an int per lane (MLP_STRIDE < 64)
+    const int lay0 = layout[lane < MLP_STRIDE ? lane : 0];
     for (int64_t tl = t0; tl < t1; tl++) {
         const int64_t a0 = tl * MLP_TILE;
         __syncthreads();  // the previous tile is done with s_sp and the scratch
         if (tid < MLP_TILE) {
-            const int64_t a = a0 + tid;
             int e = -2;
-            if (a < natoms) {
-                const int64_t sp = species[a];
-                e = (sp >= 0 && sp < nelem) ? (int)sp : -1;
-            }
+            if (a0 + tid < natoms) e = (spv >= 0 && spv < nelem) ? (int)spv : -1;
             s_sp[tid] = e;
         }
         __syncthreads();
+        const int mine = s_sp[ri];
+        bool held = true;  // xv has this tile's inputs
         for (int el = 0; el < nelem; el++) {
-            bool any = false;
-            for (int t = 0; t < MLP_TILE; t++) any = any || s_sp[t] == el;
-            if (!any) continue;  // uniform over the workgroup
-            const int *lay = layout + el * MLP_STRIDE;
-            const int nl = lay[0];
+            if (!__ballot(mine == el)) continue;  // uniform over the workgroup
+            const int layv = el == 0 ? lay0 : layout[el * MLP_STRIDE + (lane < MLP_STRIDE ? lane : 0)];
+            auto lay = [&](int k, int q) { return __builtin_amdgcn_readlane(layv, 1 + MLP_LSTRIDE * k + q); };
+            const int nl = __builtin_amdgcn_readlane(layv, 0);
             const double *dm = dmin + (size_t)el * nin, *sc = scale + (size_t)el * nin;
-            // staging: eight loads in flight per thread before their LDS stores
-            for (int q0 = tid; q0 < MLP_TILE * P0; q0 += 256 * 8) {
-                double v[8];
-    #pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const int q = q0 + 256 * u;
-                    const int t = q / P0, j = q - t * P0;
-                    const int64_t a = a0 + t;
-                    v[u] = (q < MLP_TILE * P0 && a < natoms && j < nin) ? (x[(size_t)a * nin + j] - dm[j]) * sc[j]
-                                                                         : 0.0;
-                }
-    #pragma unroll
-                for (int u = 0; u < 8; u++)
-                    if (q0 + 256 * u < MLP_TILE * P0) h0[q0 + 256 * u] = v[u];
+            double dv[MLP_XC], sv[MLP_XC];
+#pragma unroll
+            for (int u = 0; u < MLP_XC; u++) {
+                const int c = u * 64 + lane;
+                dv[u] = c < nin ? dm[c] : 0.0;
+                sv[u] = c < nin ? sc[c] : 0.0;
             }
+            if (!held) fetch(a0);
             if (el != staged) {  // uniform over the workgroup
                 staged = el;
-                int wo = 0;
-                for (int k = 0; k < nl; k++) {
-                    const int *L = lay + 1 + MLP_LSTRIDE * k;
-                    const int ni = L[0], no = L[1], R = mlp_r16(no), C = mlp_row(ni);
-                    const double *W = params + L[3], *bias = params + L[4];
-                    for (int q0 = tid; q0 < R * C + R; q0 += 256 * 8) {
-                        double v[8];
-    #pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            const int q = q0 + 256 * u;
-                            v[u] = 0.0;
-                            if (q < R * C) {
-                                const int r = q / C, c = q - r * C;
-                                if (r < no && c < ni) v[u] = W[r * ni + c];
-                            } else if (q - R * C < no) {
-                                v[u] = bias[q - R * C];
-                            }
-                        }
-    #pragma unroll
-                        for (int u = 0; u < 8; u++)
-                            if (q0 + 256 * u < R * C + R) wl[wo + q0 + 256 * u] = v[u];
+                // 64 columns of a layer at a time
+                for (int k = 0, c0 = 0, wo = 0; k < nl;) {
+                    const int ni = lay(k, 0), no = lay(k, 1), R = mlp_r16(no), C = mlp_row(ni), K = mlp_r16(ni);
+                    const double *W = params + lay(k, 3);
+                    const int c = c0 + lane;
+                    double v[RU];
+#pragma unroll
+                    for (int u = 0; u < RU; u++) {
+                        const int r = wv + MLP_WV * u;
+                        v[u] = r < no && c < ni ? W[r * ni + c] : 0.0;
                     }
-                    if (tid == 0) s_wo[k] = wo;
-                    wo += R * C + R;
+#pragma unroll
+                    for (int u = 0; u < RU; u++) {
+                        const int r = wv + MLP_WV * u;
+                        if (r < R && c < K) wl[wo + r * C + c] = v[u];
+                    }
+                    if (c0 == 0) {
+                        if (tid < R) wl[wo + R * C + tid] = tid < no ? params[lay(k, 4) + tid] : 0.0;
+                        if (tid == 0) s_wo[k] = wo;
+                    }
+                    c0 += 64;
+                    if (c0 >= K) {
+                        wo += R * (C + 1);
+                        c0 = 0;
+                        k++;
+                    }
                 }
             }
+#pragma unroll
+            for (int u = 0; u < AR * MLP_XC; u++) {
+                const int t = AR * wv + u % AR, c = u / AR * 64 + lane;
+                if (c < P0) h0[t * P0 + c] = c < nin ? (xv[u] - dv[u / AR]) * sv[u / AR] : 0.0;
+            }
+            for (int c = 64 * MLP_XC + lane; c < P0; c += 64)
+                for (int u = 0; u < AR; u++) {
+                    const int64_t a = a0 + AR * wv + u;
+                    h0[(AR * wv + u) * P0 + c] =
+                        a < natoms && c < nin ? (x[(size_t)a * nin + c] - dm[c]) * sc[c] : 0.0;
+                }
+            held = false;
             __syncthreads();
+            // the next tile's inputs, once this one's are no longer needed
+            if (tl + 1 < t1 && !__ballot(mine > el)) fetch(a0 + MLP_TILE);
             // forward
             const double *hin = h0;
             int ldi = P0;
             for (int k = 0; k < nl; k++) {
-                const int *L = lay + 1 + MLP_LSTRIDE * k;
-                const int ni = L[0], no = L[1], act = L[2], C = mlp_row(ni);
+                const int ni = lay(k, 0), no = lay(k, 1), act = lay(k, 2), C = mlp_row(ni), T = mlp_r16(no) >> 4;
                 const double *W = wl + s_wo[k], *bias = W + mlp_r16(no) * C;
-                double *ho = hact + (size_t)k * MLP_TILE * HP, *hd = hder + (size_t)k * MLP_TILE * HP;
-                for (int ct = wv; ct * 16 < no; ct += 4) {
+                double *ho = hact + (size_t)(k % (nbuf > 0 ? nbuf : 1)) * MLP_TILE * HP;
+                double *hd = hder + (size_t)k * MLP_TILE * HP;
+                const int ks = mlp_parts(T, zpn);
+                if (wv < T * ks) {
                     // D[j][i] = sum_k W[j][k] H[i][k]: A rows = neurons of the
                     // tile, B columns = atoms
-                    const mlp_d4 acc = mlp_gemm_tile(mlp_r4(ni), W + (ct * 16 + ri) * C + kq, hin + ri * ldi + kq, 4);
-    #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int j = ct * 16 + kq + 4 * r;  // neuron; the lane's atom is ri
-                        double av = 0.0, da = 0.0;          // zero past the layer width
-                        if (j < no) act_fdf(act, acc[r] + bias[j], av, da);
-                        ho[ri * HP + j] = av;
-                        hd[ri * HP + j] = da;
-                    }
+                    const int ct = wv / ks;
+                    const mlp_d4 acc = mlp_gemm_part(wv - ct * ks, ks, mlp_r4(ni) >> 2, W + (ct * 16 + ri) * C + kq,
+                                                     hin + ri * ldi + kq, 4);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) zp[wv * MLP_ZP + (kq + 4 * r) * 17 + ri] = acc[r];
+                }
+                __syncthreads();
+                for (int j = tn; j < 16 * T; j += MLP_T / 16) {
+                    const double *z = zp + (j >> 4) * ks * MLP_ZP + (j & 15) * 17 + ta;
+                    double v = bias[j];
+                    for (int p = 0; p < ks; p++) v += z[p * MLP_ZP];
+                    double2 f = mlp_act(act, v);
+                    if (j >= no) f = make_double2(0.0, 0.0);  // zero past the layer width
+                    if (k < nl - 1)
+                        ho[ta * HP + j] = f.x;
+                    else if (j == 0 && s_sp[ta] == el)
+                        e_out[a0 + ta] = f.x;
+                    hd[ta * HP + j] = f.y;
                 }
                 __syncthreads();
                 hin = ho;
                 ldi = HP;
             }
-            if (tid < MLP_TILE && s_sp[tid] == el) e_out[a0 + tid] = hin[tid * HP];
             // backward; hder of the output layer (one neuron) already is dE/dz
             for (int k = nl - 1; k >= 1; k--) {
-                const int *L = lay + 1 + MLP_LSTRIDE * k;
-                const int ni = L[0], no = L[1], C = mlp_row(ni);
+                const int ni = lay(k, 0), no = lay(k, 1), C = mlp_row(ni), T = mlp_r16(ni) >> 4, S = mlp_r4(no) >> 2;
                 const double *W = wl + s_wo[k];
                 const double *g = hder + (size_t)k * MLP_TILE * HP;
                 double *gp = hder + (size_t)(k - 1) * MLP_TILE * HP;
-                for (int ct = wv; ct * 16 < ni; ct += 4) {
-                    const int j = ct * 16 + ri;
+                const int ks = S > 1 ? mlp_parts(T, zpn) : 1;
+                if (wv < T * ks) {
                     // B[n][j] = W[n][j]
-                    const mlp_d4 acc = mlp_gemm_tile(mlp_r4(no), g + ri * HP + kq, W + kq * C + j, 4 * C);
-    #pragma unroll
-                    for (int r = 0; r < 4; r++) gp[(kq + 4 * r) * HP + j] *= acc[r];
+                    const int ct = wv / ks;
+                    const mlp_d4 acc = mlp_gemm_part(wv - ct * ks, ks, S, g + ri * HP + kq, W + kq * C + ct * 16 + ri,
+                                                     4 * C);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) zp[wv * MLP_ZP + ri * 17 + kq + 4 * r] = acc[r];
+                }
+                __syncthreads();
+                for (int j = tn; j < 16 * T; j += MLP_T / 16) {
+                    const double *z = zp + (j >> 4) * ks * MLP_ZP + (j & 15) * 17 + ta;
+                    double v = 0.0;
+                    for (int p = 0; p < ks; p++) v += z[p * MLP_ZP];
+                    gp[ta * HP + j] *= v;
                 }
                 __syncthreads();
             }
             {
-                const int *L = lay + 1;
-                const int no = L[1], C = mlp_row(nin);
+                const int S = mlp_r4(lay(0, 1)) >> 2, C = mlp_row(nin);
                 const double *W = wl + s_wo[0];
-                for (int ct = wv; ct * 16 < nin; ct += 4) {
+                for (int ct = wv; ct * 16 < nin; ct += MLP_WV) {
                     const int j = ct * 16 + ri;
-                    const mlp_d4 acc = mlp_gemm_tile(mlp_r4(no), hder + ri * HP + kq, W + kq * C + j, 4 * C);
+                    const double sj = j < nin ? sc[j] : 0.0;
+                    const mlp_d4 acc = mlp_gemm_part(0, 1, S, hder + ri * HP + kq, W + kq * C + j, 4 * C);
                     if (j < nin) {
-                        const double sj = sc[j];
-    #pragma unroll
+#pragma unroll
                         for (int r = 0; r < 4; r++) {
                             const int row = kq + 4 * r;
                             if (s_sp[row] == el) beta[(size_t)(a0 + row) * nin + j] = acc[r] * sj;
@@ -429,8 +495,9 @@ __global__ __launch_bounds__(256) void mlp_mfma_kernel(int64_t natoms, int nin, 
             }
             __syncthreads();  // the next element reuses the scratch
         }
+        if (held && tl + 1 < t1) fetch(a0 + MLP_TILE);  // no atom of the tile has a network
         // atoms without a network: NaN results
-        for (int q = tid; q < MLP_TILE * nin; q += 256) {
+        for (int q = tid; q < MLP_TILE * nin; q += MLP_T) {
             const int t = q / nin;
             if (s_sp[t] == -1) beta[(size_t)(a0 + t) * nin + (q - t * nin)] = __builtin_nan("");
         }
@@ -556,8 +623,16 @@ extern "C" int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const in
         }
         wmax = std::max(wmax, w);
     }
-    const size_t ldsm =
-        sizeof(double) * (MLP_TILE * ((size_t)mlp_row(nin) + 2 * (size_t)nlm * mlp_row(hw)) + wmax);
+    // partial tiles: one per wavefront, or as many as the widest layer has
+    // tiles where that decides whether it all fits
+    const int nbuf = std::min(2, nlm - 1);
+    auto lds_of = [&](int zpn) {
+        return sizeof(double) * (MLP_TILE * ((size_t)mlp_row(nin) + ((size_t)nbuf + nlm) * mlp_row(hw)) +
+                                 (size_t)zpn * MLP_ZP + wmax);
+    };
+    int zpn = MLP_WV;
+    if (lds_of(zpn) > 160 * 1024 - 1024) zpn = mlp_r16(hw) / 16;
+    const size_t ldsm = lds_of(zpn);
     // above 64 KB (long descriptors, e.g. SO3 6/6: 147 inputs) one workgroup
     // per CU; the kernel's static LDS (a few hundred bytes) comes on top
     if (ldsm <= 160 * 1024 - 1024) {
@@ -574,11 +649,11 @@ extern "C" int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const in
             }
         }
         // persistent: as many workgroups as the LDS keeps resident (at most
-        // 8 per CU), each over a contiguous range of 16-atom tiles
-        const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)(160 * 1024) / (int64_t)(ldsm + 1024)));
+        // 4 per CU, two by their registers), each over a contiguous range of 16-atom tiles
+        const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, (int64_t)(160 * 1024) / (int64_t)(ldsm + 1024)));
         const int64_t nwg = std::min<int64_t>(div_up(natoms, MLP_TILE), (int64_t)num_cus() * per_cu);
-        mlp_mfma_kernel<<<(unsigned)nwg, 256, ldsm, s>>>(
-            natoms, nin, nelem, d_species, d_layout, d_params, d_dmin, d_scale, d_x, d_e, d_beta, nlm, hw);
+        mlp_mfma_kernel<<<(unsigned)nwg, MLP_T, ldsm, s>>>(
+            natoms, nin, nelem, d_species, d_layout, d_params, d_dmin, d_scale, d_x, d_e, d_beta, nlm, hw, nbuf, zpn);
         PXFF_LAUNCH_CHECK();
         return 0;
     }

@@ -107,3 +107,32 @@ def test_energy_and_gradient_matches_autograd(elements, hidden, act):
 
     model.__class__ = Other
     assert potential._networks(model, x, species) is None
+
+
+# neurons around the 16-wide tiles and the splits of their sums (1 to 4 tiles),
+# inputs around the 64-column groups and past the three held in registers, the
+# deep and long ones with fewer partial tiles than wavefronts or another
+# kernel; atoms below, at and past a tile, and without a network
+@pytest.mark.parametrize("hidden,nin", [((), 1), ((1,), 3), ((16, 17), 64), ((32, 33), 65), ((48, 49), 192),
+                                        ((64, 5), 193), ((20,), 400), ((30, 30, 30, 30), 260), ((24, 24), 250)])
+@pytest.mark.parametrize("n", [1, 16, 33])
+def test_network_tile_edges(hidden, nin, n):
+    """Tolerances as above."""
+    rng = np.random.default_rng(nin)
+    model = potential.NNPotential(["Si", "O"], nin, hidden, seed=3).cuda()
+    with torch.no_grad():
+        for p in model.parameters():
+            p.add_(0.05 * torch.randn_like(p))
+    x = torch.as_tensor(rng.random((n, nin)), dtype=torch.float64, device="cuda")
+    sp = torch.as_tensor(rng.integers(0, 2, n), device="cuda")
+    symbols = [model.elements[int(k)] for k in sp.cpu()]
+    if n == 33:
+        sp[7] = -1
+        symbols[7] = "H"
+    e, beta = model.energy_grad(x, sp)
+    e_ref, g_ref = _torch_reference(model, x, symbols)
+    if n == 33:
+        assert torch.isnan(e[7]) and torch.isnan(beta[7]).all()
+        e[7], beta[7] = 0.0, 0.0
+    assert rel_err(e.cpu().numpy(), e_ref.cpu().numpy()) < 1e-13
+    assert rel_err(beta.cpu().numpy(), g_ref.cpu().numpy()) < 1e-12
