@@ -503,19 +503,6 @@ __device__ inline void sweep_rows_w(int mb, const CK &ck, F &&f) {
     }
 }
 
-// One level of the W rows with nothing but multiplications: row mb of level l
-// is the coefficients in x of (b + a x)^mb (conj a - conj b x)^(l - mb) (the
-// inversion of row 0 of level mb is the first power), so every level
-// multiplies by one of the two factors.  w[m] is zero for m > l - 1 on entry.
-template <int TWOJ>
-__device__ __forceinline__ void row_step_w(int l, int mb, const CK &ck, cd *w) {
-    const bool up = l <= mb;
-    const cd f0 = up ? cconj(ck.cb) : ck.ca, f1 = up ? cconj(ck.ca) : cmake(-ck.cb.re, -ck.cb.im);
-#pragma unroll
-    for (int m = TWOJ; m >= 1; m--) w[m] = cmadd(f1, w[m - 1], cmul(f0, w[m]));
-    w[0] = cmul(f0, w[0]);
-}
-
 // sqrt(m! (l - m)! / (mb! (l - mb)!)), the factor of sweep_rows_w, from
 // sf[k] = sqrt(k!) and isf[k] = 1 / sqrt(k!).
 __device__ inline double so4_wscale(int l, int m, int mb, const double *sf, const double *isf) {
@@ -569,6 +556,20 @@ __device__ inline void generator_dots(int l, const cd *u, const cd *y, double &a
             a3 = fma(c, t2, a3);
         }
     }
+}
+
+// One level of the W rows with nothing but multiplications: row mb of level l
+// is the coefficients in x of (b + a x)^mb (conj a - conj b x)^(l - mb) (the
+// inversion of row 0 of level mb is the first power), so every level
+// multiplies by one of the two factors.  w[m] is zero for m > l - 1 on entry.
+template <int TWOJ>
+__device__ __forceinline__ void row_step_w(int l, int mb, const CK &ck, cd *w) {
+    const bool up = l <= mb;
+    const cd f0 = up ? cconj(ck.cb) : ck.ca, f1 = up ? cconj(ck.ca) : cmake(-ck.cb.re, -ck.cb.im);
+#pragma unroll
+    for (int m = TWOJ; m >= 1; m--)
+        if (m <= l) w[m] = cmadd(f1, w[m - 1], cmul(f0, w[m]));
+    w[0] = cmul(f0, w[0]);
 }
 
 // ---------------------------------------------------------------- U_tot
@@ -1090,7 +1091,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1))) void so
 
 // U_tot from the staged per-image records (so4_stage_kernel): without the
 // cutoff and Cayley-Klein evaluation between its sweeps the kernel fits two
-// wavefronts per SIMD.
+// wavefronts per SIMD.  A wavefront per centre: for lists too short to fill
+// the chip with the wavefronts of so4_utot_group_kernel.
 template <int TWOJ>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so4_utot_staged_kernel(
     int64_t natoms, const int64_t *__restrict__ img_start, const double *__restrict__ site_w,
@@ -1098,6 +1100,136 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
     double *__restrict__ out) {
     so4_utot_body<TWOJ, false, true>(natoms, img_start, nullptr, nullptr, nullptr, site_w, nullptr, work_order,
                                      nullptr, lnorm_g, 0.0, 0.0, 1, fcut0, out, stage);
+}
+
+// The same for long lists.  G lanes (one
+// per row mb) go through images as in so4_utot_body, sums in registers, but a
+// centre gets only `split` of the wavefront's NG lane groups, and the
+// wavefront NG / split centres: with one group per centre nothing is summed
+// across lanes at all, and every centre fewer groups saves their share of the
+// LDS traffic of that sum, which took longer than the sweeps.  The groups of
+// a centre are added in halves (fixed order).  Neighbouring centres share a
+// wavefront, so their elements of the tile-major output share lines.
+// Two wavefronts per SIMD (registers: 45 complex sums at 2J = 8).
+// Against the wavefront per centre (with the staging of the records): 4096
+// atoms (28 images, 2J = 8, three groups to a centre) 36 -> 29 us, 32768 233 ->
+// 121, 110592 760 -> 396, 120000 of 32 images on average 851 -> 547; 4096 atoms
+// at 2J = 6 22 -> 20.
+template <int TWOJ>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so4_utot_group_kernel(
+    int64_t natoms, int split, const int64_t *__restrict__ img_start, const double *__restrict__ site_w,
+    const double *__restrict__ lnorm_g, double fcut0, const double *__restrict__ stage, double *__restrict__ out) {
+    constexpr int G = TWOJ / 2 + 1;
+    constexpr int NG = 64 / G;
+    constexpr int NH = nhalf_of(TWOJ);
+    constexpr int NSLOT = (TWOJ + 1) * (TWOJ + 2) / 2;  // (l, m <= l) of every level
+    constexpr int NS = so4_stage_stride<false>();
+    __shared__ cd part[NG / 2][NH];
+    __shared__ double sf[TWOJ + 1], isf[TWOJ + 1];  // sqrt(k!), 1 / sqrt(k!)
+    const int lane = threadIdx.x;
+    const int g = lane / G, mb = lane % G;
+    if (lane <= TWOJ) {
+        double f = 1.0;
+        for (int q = 2; q <= lane; q++) f *= q;
+        sf[lane] = sqrt(f);
+        isf[lane] = 1.0 / sqrt(f);
+    }
+    if (blockIdx.x == 0 && (natoms & 63)) {
+        // padding lanes of the last tile (read by the Z kernel) are zero
+        cd *last = reinterpret_cast<cd *>(out) + (size_t)(natoms >> 6) * NH * 64;
+        for (int k = lane; k < NH * 64; k += 64)
+            if ((k & 63) >= (natoms & 63)) last[k] = cmake(0.0, 0.0);
+    }
+    const int cpw = NG / split, c = g / split, p = g - c * split;
+    const int64_t i = (int64_t)blockIdx.x * cpw + c;
+    const bool mine = c < cpw && i < natoms;
+    const int64_t s = mine ? img_start[i] : 0;
+    const int n = mine ? (int)(img_start[i + 1] - s) : 0;
+    const double wself = mine ? site_w[i] : 0.0;
+    cd acc[NSLOT];
+#pragma unroll
+    for (int q = 0; q < NSLOT; q++) acc[q] = cmake(0.0, 0.0);
+    // the wavefront's longest centre bounds the loop: with a bound per lane
+    // the sums were held twice around it (140 spilled registers)
+    int most = n;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
+    most = __builtin_amdgcn_readfirstlane(most);
+#pragma unroll 1
+    for (int k0 = 0; k0 < most; k0 += split) {
+        const int k = k0 + p;
+        const bool ok = k < n;
+        const double *rec = stage + (s + (ok ? k : 0)) * NS;
+        CK ck;
+        ck.ca = cmake(1.0, 0.0);
+        ck.cb = cmake(0.0, 0.0);
+        double sc = 0.0;
+        if (ok) {
+            ck.ca = cmake(rec[0], rec[1]);
+            ck.cb = cmake(rec[2], rec[3]);
+            sc = rec[4];
+        }
+        cd w[TWOJ + 1];
+#pragma unroll
+        for (int m = 0; m <= TWOJ; m++) w[m] = cmake(m == 0 ? 1.0 : 0.0, 0.0);
+        // (the rows above the half add to sums that are not written)
+#pragma unroll
+        for (int l = 0; l <= TWOJ; l++) {
+            if (l > 0) row_step_w<TWOJ>(l, mb, ck, w);
+            const int q0 = l * (l + 1) / 2;
+#pragma unroll
+            for (int m = 0; m <= TWOJ; m++) {
+                if (m > l) continue;
+                acc[q0 + m].re = fma(sc, w[m].re, acc[q0 + m].re);
+                acc[q0 + m].im = fma(sc, w[m].im, acc[q0 + m].im);
+            }
+        }
+    }
+    // groups [half, cnt) of every centre into its groups [0, cnt - half)
+    for (int cnt = split; cnt > 1;) {
+        const int half = (cnt + 1) / 2, src = p - half;
+        __syncthreads();
+        if (c < cpw && src >= 0 && p < cnt) {
+            cd *o = part[c * (split / 2) + src];
+#pragma unroll
+            for (int l = 0; l <= TWOJ; l++)
+#pragma unroll
+                for (int m = 0; m <= l; m++)
+                    if (2 * mb <= l) o[hoff_of(l) + mb * (l + 1) + m] = acc[l * (l + 1) / 2 + m];
+        }
+        __syncthreads();
+        {
+            // no branch around the additions: the sums of both ways would be
+            // held side by side
+            const bool add = c < cpw && p + half < cnt;
+            const cd *o = part[add ? c * (split / 2) + p : 0];
+#pragma unroll
+            for (int l = 0; l <= TWOJ; l++)
+#pragma unroll
+                for (int m = 0; m <= l; m++) {
+                    const bool on = add && 2 * mb <= l;
+                    const cd v = o[on ? hoff_of(l) + mb * (l + 1) + m : 0];
+                    cd &t = acc[l * (l + 1) / 2 + m];
+                    t.re += on ? v.re : 0.0;
+                    t.im += on ? v.im : 0.0;
+                }
+        }
+        cnt = half;
+    }
+    __syncthreads();  // sf, isf
+    if (!mine || p != 0) return;
+    cd *o = reinterpret_cast<cd *>(out) + (size_t)(i >> 6) * NH * 64 + (i & 63);
+#pragma unroll
+    for (int l = 0; l <= TWOJ; l++) {
+        if (2 * mb > l) continue;
+        const double ln = lnorm_g[l];
+#pragma unroll
+        for (int m = 0; m <= l; m++) {
+            cd a = cscale(acc[l * (l + 1) / 2 + m], so4_wscale(l, m, mb, sf, isf));
+            if (m == mb) a.re += fcut0 * wself;  // addself_uarraytot
+            o[(size_t)(hoff_of(l) + mb * (l + 1) + m) * 64] = cscale(a, ln);  // ulisttot *= u_norm
+        }
+    }
 }
 
 // B (compute_bi, SNAP.py:1101-1141) from the tile-major U_tot and Z: one
@@ -2287,15 +2419,30 @@ extern "C" int pxff_so4_ui_staged(const pxff_so4_params *p, int64_t natoms, cons
     const So4Dev *T = nullptr;
     if ((rc = get_so4_tables(p->twol, p->normalize_u, &T))) return rc;
     hipStream_t s = (hipStream_t)stream;
-    const int grid = (int)std::min<int64_t>(natoms, (int64_t)num_cus() * tune_value(PXFF_TUNE_ACCUM_WAVES_PER_CU));
     const double fcut0 = cutoff_f0_host(p->cutoff_id);
     const int sgrid = (int)std::max<int64_t>(1, std::min<int64_t>(div_up(cap, 256), (int64_t)num_cus() * 8));
     so4_stage_kernel<false><<<sgrid, 256, 0, s>>>(natoms, cap, d_img_start, d_img_j, d_img_r, d_atom_w, nullptr,
                                                   p->rcut, p->rfac0, p->cutoff_id, d_stage);
     PXFF_LAUNCH_CHECK();
     PXFF_DISPATCH_TWOJ(p->twol, if constexpr (TJ <= 8) {
-        so4_utot_staged_kernel<TJ><<<grid, 64, 0, s>>>(natoms, d_img_start, d_site_w, d_work_order, T->lnorm, fcut0,
-                                                      d_stage, d_utot);
+        constexpr int NG = 64 / (TJ / 2 + 1);
+        // centres per wavefront: as many as leave a wavefront per SIMD; below
+        // four the sum over a centre's groups costs what it did (4095 atoms
+        // of 32 images, three centres to a wavefront: 39 against 38 us; 1728
+        // atoms, one: 31 against 21)
+        const int64_t want = natoms / ((int64_t)num_cus() * 4);
+        if (want >= 4) {
+            const int split = NG / (int)std::min<int64_t>(NG, want);
+            const int64_t grid = div_up(natoms, NG / split);
+            PXFF_REQUIRE(grid <= 0x7fffffff, "too many atoms for one launch");
+            so4_utot_group_kernel<TJ><<<(unsigned)grid, 64, 0, s>>>(natoms, split, d_img_start, d_site_w, T->lnorm,
+                                                                  fcut0, d_stage, d_utot);
+        } else {
+            const int grid =
+                (int)std::min<int64_t>(natoms, (int64_t)num_cus() * tune_value(PXFF_TUNE_ACCUM_WAVES_PER_CU));
+            so4_utot_staged_kernel<TJ><<<grid, 64, 0, s>>>(natoms, d_img_start, d_site_w, d_work_order, T->lnorm,
+                                                          fcut0, d_stage, d_utot);
+        }
     });
     PXFF_LAUNCH_CHECK();
     return 0;

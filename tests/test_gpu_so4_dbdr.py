@@ -33,3 +33,29 @@ def test_dbdr_image_counts(n, twol):
         if k:
             assert float((d - ref).norm() / ref.norm()) < 1e-13
             assert float((d - ref).abs().max() / ref.abs().max()) < 1e-12
+
+
+# 4096 atoms and more take the kernel with several centres per wavefront: 4, 5
+# (rounded to 6 at 2J = 8), 12 and all of a wavefront's lane groups to a centre
+@pytest.mark.parametrize("n,twol", [(4096, 8), (4097, 6), (5200, 8), (6500, 2), (12300, 8), (16500, 6), (8200, 4),
+                                    (66000, 0)])
+def test_utot_centres_per_wavefront(n, twol):
+    """U_tot of the staged records against the kernel that stages in LDS, a
+    wavefront per centre: a gas of clusters with 0 to 70 images per centre.
+    Sums of at most 70 terms in another order, 1e-14 of the norm."""
+    from pyxtal_ff_amd import so4
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    rng = np.random.default_rng(n)
+    size = rng.integers(1, 72, n)  # atoms per cluster, clusters 20 apart
+    owner = np.repeat(np.arange(n), size)[:n]
+    side = int(np.ceil((owner.max() + 1) ** (1 / 3)))
+    at = np.stack([owner % side, owner // side % side, owner // side**2], 1) * 20.0
+    pos = at + rng.uniform(0, 2.4, (n, 3))
+    nl = DeviceNeighborList([pos], [np.eye(3) * (side * 20.0 + 50.0)], [np.zeros(3, bool)], 4.3)
+    assert nl.nimg > n
+    cfg = so4.So4Config(twol, 4.3, 0.99363)
+    w = torch.rand(n, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda() + 0.5
+    a, b = so4.ui(nl, cfg, w, w), so4.ui(nl, cfg, w, w, staged=False)
+    assert float((a - b).norm() / b.norm()) < 1e-14
+    assert float((a - b).abs().max() / b.abs().max()) < 1e-13
+    assert torch.equal(a, so4.ui(nl, cfg, w, w, torch.arange(n - 1, -1, -1, device="cuda")))
