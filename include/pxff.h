@@ -297,6 +297,14 @@ int pxff_so4_tangent(const pxff_so4_params *p, int64_t natoms, const int64_t *d_
                      const double *d_img_r, const double *d_atom_w, const double *d_dr, const double *d_z,
                      double *d_dutot, double *d_db, void *stream);
 
+/* pxff_so4_tangent with room for the per-image values of its sweeps: d_stage
+ * [cap*10], images past cap (none in a list of that capacity) not counted.
+ * Long lists then take several centres per wavefront. */
+int pxff_so4_tangent_staged(const pxff_so4_params *p, int64_t natoms, const int64_t *d_img_start,
+                            const int64_t *d_img_j, const double *d_img_r, const double *d_atom_w,
+                            const double *d_dr, const double *d_z, int64_t cap, double *d_stage, double *d_dutot,
+                            double *d_db, void *stream);
+
 /* pxff_so4_tangent without the d_dutot workspace argument, allocating
  * nothing.  No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving or

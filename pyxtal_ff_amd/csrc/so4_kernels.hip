@@ -1114,8 +1114,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
 // Against the wavefront per centre (with the staging of the records): 4096
 // atoms (28 images, 2J = 8, three groups to a centre) 36 -> 29 us, 32768 233 ->
 // 121, 110592 760 -> 396, 120000 of 32 images on average 851 -> 547; 4096 atoms
-// at 2J = 6 22 -> 20.
-template <int TWOJ>
+// at 2J = 6 22 -> 20.  The tangent (with the dB sum, 2J = 8): 4096 atoms 129 ->
+// 113 us, 32768 718 -> 525, 33000 of 32 images 808 -> 670.
+template <int TWOJ, bool TANGENT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so4_utot_group_kernel(
     int64_t natoms, int split, const int64_t *__restrict__ img_start, const double *__restrict__ site_w,
     const double *__restrict__ lnorm_g, double fcut0, const double *__restrict__ stage, double *__restrict__ out) {
@@ -1123,7 +1124,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
     constexpr int NG = 64 / G;
     constexpr int NH = nhalf_of(TWOJ);
     constexpr int NSLOT = (TWOJ + 1) * (TWOJ + 2) / 2;  // (l, m <= l) of every level
-    constexpr int NS = so4_stage_stride<false>();
+    constexpr int NS = so4_stage_stride<TANGENT>();
     __shared__ cd part[NG / 2][NH];
     __shared__ double sf[TWOJ + 1], isf[TWOJ + 1];  // sqrt(k!), 1 / sqrt(k!)
     const int lane = threadIdx.x;
@@ -1145,7 +1146,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
     const bool mine = c < cpw && i < natoms;
     const int64_t s = mine ? img_start[i] : 0;
     const int n = mine ? (int)(img_start[i + 1] - s) : 0;
-    const double wself = mine ? site_w[i] : 0.0;
+    const double wself = mine && !TANGENT ? site_w[i] : 0.0;
     cd acc[NSLOT];
 #pragma unroll
     for (int q = 0; q < NSLOT; q++) acc[q] = cmake(0.0, 0.0);
@@ -1163,11 +1164,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
         CK ck;
         ck.ca = cmake(1.0, 0.0);
         ck.cb = cmake(0.0, 0.0);
-        double sc = 0.0;
+        double sc = 0.0, Qr = 0.0, Qi = 0.0, Gu = 0.0;  // TANGENT: sc is p(eta)
         if (ok) {
             ck.ca = cmake(rec[0], rec[1]);
             ck.cb = cmake(rec[2], rec[3]);
             sc = rec[4];
+            if (TANGENT) {
+                Qr = rec[5];
+                Qi = rec[6];
+                Gu = rec[7];
+            }
         }
         cd w[TWOJ + 1];
 #pragma unroll
@@ -1180,8 +1186,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
 #pragma unroll
             for (int m = 0; m <= TWOJ; m++) {
                 if (m > l) continue;
-                acc[q0 + m].re = fma(sc, w[m].re, acc[q0 + m].re);
-                acc[q0 + m].im = fma(sc, w[m].im, acc[q0 + m].im);
+                cd &a = acc[q0 + m];
+                if constexpr (!TANGENT) {
+                    a.re = fma(sc, w[m].re, a.re);
+                    a.im = fma(sc, w[m].im, a.im);
+                } else {
+                    // (U M(eta))_m on W as in so4_utot_body
+                    const double pm = sc * (double)(l - 2 * m);
+                    double re = fma(-pm, w[m].im, Gu * w[m].re);
+                    double im = fma(pm, w[m].re, Gu * w[m].im);
+                    if (m >= 1) {
+                        const double cc = (double)(l - m + 1);
+                        re = fma(cc, Qr * w[m - 1].re - Qi * w[m - 1].im, re);
+                        im = fma(cc, Qr * w[m - 1].im + Qi * w[m - 1].re, im);
+                    }
+                    if (m < l) {
+                        const double cc = (double)(m + 1);
+                        re = fma(-cc, Qr * w[m + 1].re + Qi * w[m + 1].im, re);
+                        im = fma(-cc, Qr * w[m + 1].im - Qi * w[m + 1].re, im);
+                    }
+                    a.re += re;
+                    a.im += im;
+                }
             }
         }
     }
@@ -1226,7 +1252,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
 #pragma unroll
         for (int m = 0; m <= l; m++) {
             cd a = cscale(acc[l * (l + 1) / 2 + m], so4_wscale(l, m, mb, sf, isf));
-            if (m == mb) a.re += fcut0 * wself;  // addself_uarraytot
+            if (!TANGENT && m == mb) a.re += fcut0 * wself;  // addself_uarraytot
             o[(size_t)(hoff_of(l) + mb * (l + 1) + m) * 64] = cscale(a, ln);  // ulisttot *= u_norm
         }
     }
@@ -2435,7 +2461,7 @@ extern "C" int pxff_so4_ui_staged(const pxff_so4_params *p, int64_t natoms, cons
             const int split = NG / (int)std::min<int64_t>(NG, want);
             const int64_t grid = div_up(natoms, NG / split);
             PXFF_REQUIRE(grid <= 0x7fffffff, "too many atoms for one launch");
-            so4_utot_group_kernel<TJ><<<(unsigned)grid, 64, 0, s>>>(natoms, split, d_img_start, d_site_w, T->lnorm,
+            so4_utot_group_kernel<TJ, false><<<(unsigned)grid, 64, 0, s>>>(natoms, split, d_img_start, d_site_w, T->lnorm,
                                                                   fcut0, d_stage, d_utot);
         } else {
             const int grid =
@@ -2560,7 +2586,8 @@ extern "C" int pxff_so4_forces_energy(int64_t natoms, const int64_t *d_img_start
 
 static int so4_tangent_launch(const pxff_so4_params *p, const So4Dev *T, int64_t natoms, const int64_t *d_img_start,
                               const int64_t *d_img_j, const double *d_img_r, const double *d_atom_w,
-                              const double *d_dr, const double *d_z, double *d_dutot, double *d_db, void *stream) {
+                              const double *d_dr, const double *d_z, double *d_dutot, double *d_db, void *stream, int64_t cap = 0,
+                              double *d_stage = nullptr) {
     hipStream_t s = (hipStream_t)stream;
     const int grid = (int)std::min<int64_t>(natoms, (int64_t)num_cus() * tune_value(PXFF_TUNE_ACCUM_WAVES_PER_CU));
 #define PXFF_ACCUM_TAN(MODE)                                                                      \
@@ -2571,7 +2598,22 @@ static int so4_tangent_launch(const pxff_so4_params *p, const So4Dev *T, int64_t
     // against 0.75 ms for the LDS modes on the 33.7k-atom training batch,
     // whatever mode the forward's tuning chose
     const int mode = p->twol <= 8 ? 4 : tune_value(PXFF_TUNE_ACCUM_LDSADD);
-    if (mode == 4 && p->twol <= 8) {
+    // centres per wavefront as in pxff_so4_ui_staged
+    const int64_t want = natoms / ((int64_t)num_cus() * 4);
+    if (p->twol <= 8 && d_stage != nullptr && want >= 4) {
+        const int sgrid = (int)std::max<int64_t>(1, std::min<int64_t>(div_up(cap, 256), (int64_t)num_cus() * 8));
+        so4_stage_kernel<true><<<sgrid, 256, 0, s>>>(natoms, cap, d_img_start, d_img_j, d_img_r, d_atom_w, d_dr,
+                                                     p->rcut, p->rfac0, p->cutoff_id, d_stage);
+        PXFF_LAUNCH_CHECK();
+        PXFF_DISPATCH_TWOJ(p->twol, if constexpr (TJ <= 8) {
+            constexpr int NG = 64 / (TJ / 2 + 1);
+            const int split = NG / (int)std::min<int64_t>(NG, want);
+            const int64_t ngrid = div_up(natoms, NG / split);
+            PXFF_REQUIRE(ngrid <= 0x7fffffff, "too many atoms for one launch");
+            so4_utot_group_kernel<TJ, true><<<(unsigned)ngrid, 64, 0, s>>>(natoms, split, d_img_start, nullptr,
+                                                                          T->lnorm, 0.0, d_stage, d_dutot);
+        });
+    } else if (mode == 4 && p->twol <= 8) {
         PXFF_DISPATCH_TWOJ(p->twol, if constexpr (TJ <= 8) {
             so4_utot_kernel<TJ, true><<<grid, 64, 0, s>>>(natoms, d_img_start, d_img_j, d_img_r, d_atom_w, nullptr,
                                                          d_dr, nullptr, T->rootpq, T->lnorm, p->rcut, p->rfac0,
@@ -2607,6 +2649,20 @@ extern "C" int pxff_so4_tangent(const pxff_so4_params *p, int64_t natoms, const 
     const So4Dev *T = nullptr;
     if ((rc = get_so4_tables(p->twol, p->normalize_u, &T))) return rc;
     return so4_tangent_launch(p, T, natoms, d_img_start, d_img_j, d_img_r, d_atom_w, d_dr, d_z, d_dutot, d_db, stream);
+}
+
+extern "C" int pxff_so4_tangent_staged(const pxff_so4_params *p, int64_t natoms, const int64_t *d_img_start,
+                                       const int64_t *d_img_j, const double *d_img_r, const double *d_atom_w,
+                                       const double *d_dr, const double *d_z, int64_t cap, double *d_stage,
+                                       double *d_dutot, double *d_db, void *stream) {
+    int rc = so4_check_params(p);
+    if (rc) return rc;
+    PXFF_REQUIRE(cap >= 0 && (cap == 0 || d_stage != nullptr), "stage workspace missing");
+    if (natoms <= 0) return 0;
+    const So4Dev *T = nullptr;
+    if ((rc = get_so4_tables(p->twol, p->normalize_u, &T))) return rc;
+    return so4_tangent_launch(p, T, natoms, d_img_start, d_img_j, d_img_r, d_atom_w, d_dr, d_z, d_dutot, d_db, stream,
+                              cap, d_stage);
 }
 
 // ------------------------------------------------- no-allocation tangent

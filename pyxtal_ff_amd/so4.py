@@ -181,8 +181,11 @@ def tangent(nl, cfg, atom_w, z, dr, img_r=None):
     db = _f64(nl.natoms * cfg.nb, dev)
     r = nl.img_r if img_r is None else img_r.contiguous()
     d = dr.contiguous()
-    nat.check(nat.lib().pxff_so4_tangent(cfg.params, nl.natoms, p(nl.img_start), p(nl.img_j), p(r), p(atom_w),
-                                         p(d), p(z), p(du), p(db), nat.stream()), "pxff_so4_tangent")
+    cap = min(nl.img_capacity, d.numel() // 3)
+    stage = _f64(cap * 10, dev)
+    nat.check(nat.lib().pxff_so4_tangent_staged(cfg.params, nl.natoms, p(nl.img_start), p(nl.img_j), p(r), p(atom_w),
+                                                p(d), p(z), cap, p(stage), p(du), p(db), nat.stream()),
+              "pxff_so4_tangent_staged")
     return db[: nl.natoms * cfg.nb].view(nl.natoms, cfg.nb)
 
 

@@ -59,3 +59,11 @@ def test_utot_centres_per_wavefront(n, twol):
     assert float((a - b).norm() / b.norm()) < 1e-14
     assert float((a - b).abs().max() / b.abs().max()) < 1e-13
     assert torch.equal(a, so4.ui(nl, cfg, w, w, torch.arange(n - 1, -1, -1, device="cuda")))
+    # the tangent's sums, against its wavefront per centre (within its static workspace)
+    if n * cfg.nhalf * 16 < 30e6:
+        _, z, _ = so4.forward(nl, cfg, w, w)
+        dr = torch.randn(nl.nimg * 3, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda()
+        t = so4.tangent(nl, cfg, w, z, dr)
+        ref = torch.empty_like(t)
+        so4.tangent_noalloc(nl, cfg, w, z, dr, ref)
+        assert float((t - ref).norm() / ref.norm()) < 1e-13
