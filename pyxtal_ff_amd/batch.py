@@ -61,8 +61,9 @@ class StructureBatch:
         self.volumes = np.abs(np.linalg.det(cells))
         dev = torch.device(device)
         self.device = dev
-        self.pos = torch.as_tensor(np.concatenate([a[0] for a in arrs]), dtype=torch.float64, device=dev)
-        self.builder = NeighborListBuilder(self.counts, cells, pbcs, rc, device)
+        self.builder = NeighborListBuilder(self.counts, cells, pbcs, rc, device,
+                                           _positions=np.concatenate([a[0] for a in arrs]))
+        self.pos, self.builder._positions = self.builder._positions, None
         self.nl = self.builder.build(self.pos).resolve()  # counts final before the work list is sorted
         nl = self.nl
         self.atom_struct = self.builder.atom_struct

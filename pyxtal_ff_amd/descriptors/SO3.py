@@ -9,7 +9,7 @@ import torch
 
 from .. import so3 as dev_so3
 from .. import so4 as dev_so4
-from ..neighbors import DeviceNeighborList
+from ..neighbors import DeviceNeighborList, to_host
 from ..structure import as_arrays
 from ._so4_base import prefix_count
 
@@ -177,7 +177,7 @@ class SO3:
         if self.derivative:
             dp = dev_so3.dpdr(nl, cfg, z, ct, radial=rad)
             dx, rd = dev_so4.rows(nl, cfg.ncoef, dp, stress=self.stress)
-            nr = int(nl.row_start[k].item())
+            nr = nl.nrows if k == n else int(nl.row_start[k].item())
             out["dxdr"] = dx[:nr]
             out["elements"] = list(symbols)
             out["seq"] = nl.seq_array()[:nr]
@@ -185,8 +185,7 @@ class SO3:
         else:
             out.update({"dxdr": None, "rdxdr": None, "elements": list(symbols)})
         if as_numpy:
-            for key in ("x", "dxdr", "rdxdr", "seq"):
-                if isinstance(out.get(key), torch.Tensor):
-                    out[key] = out[key].cpu().numpy()
+            keys = [key for key in ("x", "dxdr", "rdxdr", "seq") if isinstance(out.get(key), torch.Tensor)]
+            out.update(zip(keys, to_host(*[out[key] for key in keys])))
         self.clear_memory()
         return out

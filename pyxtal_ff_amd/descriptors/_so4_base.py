@@ -10,7 +10,7 @@ import numpy as np
 import torch
 
 from .. import so4 as dev_so4
-from ..neighbors import DeviceNeighborList
+from ..neighbors import DeviceNeighborList, to_device, to_host
 from ..structure import as_arrays
 
 CUTOFF_NAMES = ("cosine", "tanh", "poly1", "poly2", "poly3", "poly4", "exp")
@@ -43,14 +43,13 @@ def run_so4(atoms, twol, rcut, rfac0, cutoff_id, normalize_u, derivative, stress
     nl = DeviceNeighborList([pos], [cell], [pbc], rcut).resolve()
     cfg = dev_so4.So4Config(twol, rcut, rfac0, cutoff_id, normalize_u)
     d = nl.pos.device
-    aw = torch.as_tensor(np.asarray(atom_w, dtype=np.float64), device=d)
-    sw = torch.as_tensor(np.asarray(site_w, dtype=np.float64), device=d)
+    aw, sw = to_device(d, np.asarray(atom_w, dtype=np.float64), np.asarray(site_w, dtype=np.float64))
     b, z, _ = dev_so4.forward(nl, cfg, aw, sw)
     out = {"x": b[:k]}
     if derivative:
         dbi = dev_so4.dbdr(nl, cfg, aw, z)
         dx, rd = dev_so4.rows(nl, cfg.nb, dbi, stress=stress)
-        nr = int(nl.row_start[k].item())
+        nr = nl.nrows if k == n else int(nl.row_start[k].item())
         out["dxdr"] = dx[:nr]
         out["seq"] = nl.seq_array()[:nr]
         out["rdxdr"] = rd[:nr] if stress else None
@@ -64,7 +63,6 @@ def run_so4(atoms, twol, rcut, rfac0, cutoff_id, normalize_u, derivative, stress
             out["rdxdr"] = None
     out["elements"] = list(symbols)[:n]
     if as_numpy:
-        for key in ("x", "dxdr", "rdxdr", "seq"):
-            if key in out and isinstance(out[key], torch.Tensor):
-                out[key] = out[key].cpu().numpy()
+        keys = [key for key in ("x", "dxdr", "rdxdr", "seq") if isinstance(out.get(key), torch.Tensor)]
+        out.update(zip(keys, to_host(*[out[key] for key in keys])))
     return out

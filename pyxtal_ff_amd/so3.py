@@ -14,6 +14,7 @@ import numpy as np
 import torch
 
 from . import _native as nat
+from .neighbors import to_device
 
 CUTOFF_IDS = {"cosine": 1, "tanh": 2, "poly1": 3, "poly2": 4, "poly3": 5, "poly4": 6, "exp": 7, "unity": 8}
 RWORK = 256 * 64 + 1  # |r| bins x chunks + count: the fixed part of pxff_so3_ctot_pairs' workspace
@@ -68,9 +69,7 @@ class So3Config:
         self.csz = self.nmax * (self.lmax + 1) * (2 * self.lmax + 1)
         G, Q, ln = radial_tables(self.nmax, self.lmax, self.rcut, self.alpha)
         dev = torch.device(device)
-        self.G = torch.as_tensor(np.ascontiguousarray(G), dtype=torch.float64, device=dev)
-        self.rq = torch.as_tensor(Q, dtype=torch.float64, device=dev)
-        self.lnorm = torch.as_tensor(ln, dtype=torch.float64, device=dev)
+        self.G, self.rq, self.lnorm = to_device(dev, *(np.asarray(a, dtype=np.float64) for a in (G, Q, ln)))
         self._p = nat.So3Params(self.nmax, self.lmax, self.rcut, self.alpha, self.cutoff_id, self.nq,
                                 int(self.weight_on))
         self._table = None

@@ -216,3 +216,29 @@ def test_isolated_atom_closed_form(oracle_mod, cutoff):
     assert np.allclose(d["x"][0], fc0 ** 3 * (idxb[:, 2] + 1.0), rtol=1e-13, atol=0)
     assert d["seq"].tolist() == [[0, 0]]
     assert not d["dxdr"].any() and not d["rdxdr"].any()
+
+
+def test_grids_of_all_structures_equal_those_of_each():
+    """The bin grids of a batch, computed together, against one by one."""
+    import numpy as np
+    import pytest
+    from pyxtal_ff_amd.neighbors import _geometries, _geometry
+    rng = np.random.default_rng(3)
+    cells = rng.normal(size=(40, 3, 3)) + np.eye(3) * rng.uniform(2, 40, (40, 1, 1))
+    pbcs = np.ones((40, 3), dtype=bool)
+    pbcs[5] = [True, False, True]
+    pbcs[9] = False
+    cells[9] = 0.0
+    cells[11] = np.eye(3) * 9.8  # the plane spacing is a multiple of the cutoff
+    for rc in (0.3, 4.9, 60.0):
+        inv, geom = _geometries(cells, pbcs, rc)
+        for s in range(40):
+            i1, g1 = _geometry(cells[s], pbcs[s], rc)
+            assert np.array_equal(inv[s], i1.reshape(9)) and np.array_equal(geom[s], g1)
+    assert _geometries(np.zeros((0, 3, 3)), np.zeros((0, 3), bool), 4.0)[1].shape == (0, 8)
+    cells[0, 0, 0] = np.nan
+    with pytest.raises(ValueError):
+        _geometries(cells, pbcs, 4.9)
+    cells[0] = 0.0
+    with pytest.raises(np.linalg.LinAlgError):
+        _geometries(cells, pbcs, 4.9)
