@@ -289,6 +289,14 @@ int pxff_so4_forces_energy(int64_t natoms, const int64_t *d_img_start, const int
                            const double *d_img_r, const double *d_dedr, double *d_forces, double *d_virial,
                            const double *d_e_atom, int64_t n_e, double *d_energy, void *stream);
 
+/* Transpose of the force gather and of the per-structure virials (the double
+ * backward of force training): d_out [nimg*3] = gf_i - gf_j + gw_s^T r_e for
+ * image e of centre i (structure s = d_atom_struct[i]) with neighbour j;
+ * d_gf [natoms*3] = gradient of the forces, d_gw [nstruct*9] = gradient of
+ * W_s = sum_e r_e (x) dE/dr_e. */
+int pxff_image_grad(int64_t nimg, const int64_t *d_img_atom, const int64_t *d_img_j, const int64_t *d_atom_struct,
+                    const double *d_img_r, const double *d_gf, const double *d_gw, double *d_out, void *stream);
+
 /* Forward-mode (tangent) of B along per-image displacements dr_e
  * [nimg*3]: dB [natoms*nb] = sum_e dB/dr_e . dr_e.  Used by the double
  * backward of the adjoint (force-matched training).  d_z is the tile-major Z

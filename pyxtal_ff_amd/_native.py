@@ -66,6 +66,7 @@ _SIGS = {
     "pxff_so4_gather": ([I64, P, P, P, P, P, P, P], I32),
     "pxff_so4_forces": ([I64, P, P, P, P, P, P, P], I32),
     "pxff_so4_forces_energy": ([I64, P, P, P, P, P, P, P, I64, P, P], I32),
+    "pxff_image_grad": ([I64, P, P, P, P, P, P, P, P], I32),
     "pxff_so4_tangent": ([P, I64, P, P, P, P, P, P, P, P, P], I32),
     "pxff_so4_tangent_staged": ([P, I64, P, P, P, P, P, P, I64, P, P, P, P], I32),
     "pxff_so4_tangent_noalloc": ([P, I64, P, P, P, P, P, P, P, P], I32),

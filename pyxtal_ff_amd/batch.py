@@ -47,6 +47,41 @@ def segment_sum(v, seg, row_seg):
     return SegmentSum.apply(v, seg, row_seg)
 
 
+class ForcesVirials(torch.autograd.Function):
+    """Forces [N, 3] and per-structure virials W_s = sum_e r_e (x) dE/dr_e
+    [S, 3, 3] of a StructureBatch from dE/dr per image: the gather kernel with
+    its per-centre virials, then one sum per structure."""
+
+    @staticmethod
+    def forward(ctx, dedr, r, batch, nl):
+        ctx.batch, ctx.nl = batch, nl
+        ctx.save_for_backward(r)
+        f, vir = dev_so4.gather(nl, dedr, virial=True, img_r=r, forces=True)
+        return f, segment_sum(vir.reshape(-1, 9), batch.atom_seg, batch.atom_struct).view(batch.nstruct, 3, 3)
+
+    @staticmethod
+    def backward(ctx, gf, gw):
+        (r,) = ctx.saved_tensors
+        return _ForcesVirialsT.apply(gf, gw, r, ctx.batch, ctx.nl), None, None, None
+
+
+class _ForcesVirialsT(torch.autograd.Function):
+    """The transpose of ForcesVirials (``pxff_image_grad``), linear in the two
+    gradients; its backward is ForcesVirials again."""
+
+    @staticmethod
+    def forward(ctx, gf, gw, r, batch, nl):
+        ctx.batch, ctx.nl = batch, nl
+        ctx.save_for_backward(r)
+        return dev_so4.image_grad(nl, batch.atom_struct, r, gf, gw)
+
+    @staticmethod
+    def backward(ctx, g):
+        (r,) = ctx.saved_tensors
+        f, w = ForcesVirials.apply(g, r, ctx.batch, ctx.nl)
+        return f, w, None, None, None
+
+
 class StructureBatch:
     """Concatenated atoms of a list of Atoms-like structures on the GPU."""
 
@@ -163,10 +198,10 @@ def energy_forces_virial(desc, model, species, virial=True, create_graph=False):
     (dedr,) = torch.autograd.grad(e_struct.sum(), [r], create_graph=create_graph)
     out = {"energy": e_struct, "x": x, "atom_energies": e_atom.detach()}
     if create_graph:
-        out["forces"] = -adjoint._Gather.apply(dedr, nl)
         if virial:
-            w = (r.detach().unsqueeze(2) * dedr.unsqueeze(1)).reshape(k, 9)
-            out["virial"] = b.per_structure_images(w).view(b.nstruct, 3, 3)
+            out["forces"], out["virial"] = ForcesVirials.apply(dedr, r.detach(), b, nl)
+        else:
+            out["forces"] = -adjoint._Gather.apply(dedr, nl)
         return out
     if virial:
         g, vir = dev_so4.gather(nl, dedr, virial=True, img_r=r.detach())

@@ -156,6 +156,20 @@ def gather(nl, dedr, virial=False, img_r=None, forces=False):
     return (g, vir[: nl.natoms * 9].view(nl.natoms, 3, 3)) if virial else g
 
 
+def image_grad(nl, atom_struct, r, gf, gw):
+    """Gradient [nimg, 3] of dE/dr from those of the forces [N, 3] and of the
+    per-structure virials [S, 3, 3] (``pxff_image_grad``)."""
+    p = nat.ptr
+    k = r.shape[0]
+    if k > nl.nimg or gf.shape != (nl.natoms, 3):
+        raise ValueError("r and the force gradient must belong to the list")
+    r, gf, gw = r.contiguous(), gf.contiguous(), gw.contiguous()
+    out = _f64(k * 3, r.device)
+    nat.check(nat.lib().pxff_image_grad(k, p(nl.img_atom), p(nl.img_j), p(atom_struct), p(r), p(gf), p(gw), p(out),
+                                        nat.stream()), "pxff_image_grad")
+    return out[: k * 3].view(k, 3)
+
+
 def forces_energy(nl, dedr, e_atom, virial=False):
     """The forces -dE/dR [N, 3] (as ``gather(..., forces=True)``), the
     total energy [1] = sum of e_atom (as the one-segment ``pxff_segment_sum``)

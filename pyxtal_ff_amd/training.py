@@ -26,7 +26,7 @@ per-structure values (one per structure) go through torch reductions.
 import torch
 
 from . import adjoint
-from .batch import VOIGT
+from .batch import VOIGT, ForcesVirials
 
 EV2GPA = 160.21766208  # neuralnetwork.py: eV2GPa
 
@@ -194,7 +194,6 @@ class ForceTrainer:
         """Per-structure energies [S], forces [N, 3] and Voigt stress [S, 6]
         (GPa), differentiable in the network parameters."""
         b = self.batch
-        nl = b.nl
         x = self.x.requires_grad_(True)
         e_atom = self.model.atom_energies(x, self.species)
         # per-structure buckets first: no multi-block sum over atoms (graph capture)
@@ -205,9 +204,7 @@ class ForceTrainer:
             s_atom = -(beta.unsqueeze(2) * self.rv).sum(1)
             return b.per_structure(e_atom), forces, b.per_structure(s_atom) * EV2GPA
         dedr = self._dedr(beta.contiguous())
-        forces = -adjoint._Gather.apply(dedr, nl)
-        w = self.r.unsqueeze(2) * dedr.unsqueeze(1)  # r_e (x) dE/dr_e
-        W = b.per_structure_images(w.reshape(-1, 9)).view(b.nstruct, 3, 3)
+        forces, W = ForcesVirials.apply(dedr, self.r, b, b.nl)
         # Voigt components by a device index (no host-to-device copy in a captured step)
         S = -W.view(b.nstruct, 9).index_select(1, self._voigt) * b.inv_vol_struct[:, None]
         return b.per_structure(e_atom), forces, S * EV2GPA
