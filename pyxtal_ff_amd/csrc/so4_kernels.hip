@@ -2262,59 +2262,59 @@ __global__ __launch_bounds__(256) void voigt_contract_kernel(int64_t natoms, int
 // ----------------------------------------------------------- tangent of B
 // dB_b = sum over the (block k, factor f) pairs targeting b of f p_k with
 // p_k = 2 Re sum_loc hw(loc) conj(dU^l[loc]) Z_k[loc] and dU = dU_tot (u_norm
-// already applied by the accumulation kernel).  One workgroup of 16
-// wavefronts per 64-atom tile, one atom per lane: dU and Z are both
-// tile-major, so every load is a coalesced 1 KB row; the wavefronts split
-// the blocks (p_k into LDS; four partial sums per block keep four loads and
-// FMA chains in flight), then the components b.  The sixteen wavefronts of
-// a tile keep enough of Z in flight that the kernel runs at the rate Z
-// streams from memory.
-constexpr int TANB_THREADS = 1024;
-__global__ __launch_bounds__(TANB_THREADS) void so4_tangent_b_kernel(int64_t natoms, int nhalf, int nz, int nb, int nblk,
-                                                             int ldim, const double *__restrict__ dutile,
-                                                             const double *__restrict__ z,
-                                                             const double *__restrict__ h_weight,
-                                                             const int *__restrict__ hoff,
-                                                             const int *__restrict__ blk_level_start,
-                                                             const int *__restrict__ blk_zoff,
-                                                             const int *__restrict__ b_src,
-                                                             const double *__restrict__ b_srcf,
-                                                             double *__restrict__ db) {
-    extern __shared__ double pk[];  // [nblk][64]
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t tile = blockIdx.x;
+// already applied by the accumulation kernel).  A wavefront takes one b of a
+// 64-atom tile, one atom per lane: it sums the (at most three) blocks of b,
+// which no other b has, so every Z element is read once.  dU and Z are both
+// tile-major, every load is a coalesced 1 KB row, four sums per block and
+// eight rows of each in flight.  Bound by the Z stream.  The workgroups of a
+// tile have the same index modulo 8, so that one XCD's L2 serves the tile's
+// dU to all of them and gathers the 8-byte stores of its dB rows; the larger
+// b, with the longer blocks, start first.  33,722 atoms (2J = 8, 1.29 GB of Z):
+// 306 us, 4.2 TB/s; a workgroup per tile with the blocks' sums in LDS took 356,
+// its 534 workgroups being a round of 512 and a rest.
+constexpr int TANB_WAVES = 4;
+constexpr int TANB_XCDS = 8;
+__global__ __launch_bounds__(TANB_WAVES * 64) void so4_tangent_b_kernel(
+    int64_t natoms, int nhalf, int nz, int nb, int ldim, const double *__restrict__ dutile,
+    const double *__restrict__ z, const double *__restrict__ h_weight, const int *__restrict__ hoff,
+    const int *__restrict__ blk_level_start, const int *__restrict__ blk_zoff, const int *__restrict__ b_src,
+    const double *__restrict__ b_srcf, double *__restrict__ db) {
+    const int tg = (nb + TANB_WAVES - 1) / TANB_WAVES;
+    const int64_t q = blockIdx.x / TANB_XCDS;
+    const int64_t tile = q / tg * TANB_XCDS + blockIdx.x % TANB_XCDS;
+    const int b = nb - 1 - __builtin_amdgcn_readfirstlane((int)(q % tg) * TANB_WAVES + (threadIdx.x >> 6));
+    if (tile * 64 >= natoms || b < 0) return;  // whole wavefront
+    const int lane = threadIdx.x & 63;
     const cd *dut = reinterpret_cast<const cd *>(dutile) + (size_t)tile * nhalf * 64 + lane;
     const cd *zt = reinterpret_cast<const cd *>(z) + (size_t)tile * nz * 64 + lane;
-    const int nw = blockDim.x >> 6;
-    for (int k = wv; k < nblk; k += nw) {
+    double acc = 0.0;
+    for (int s = 0; s < 3; s++) {
+        const int k = b_src[3 * b + s];
+        if (k < 0) continue;
         int l = 0;
         while (l + 1 < ldim && k >= blk_level_start[l + 1]) l++;
         const int nloc = (l / 2 + 1) * (l + 1);
-        const int z0 = blk_zoff[k], h0 = hoff[l];
-        double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
+        const cd *u = dut + (size_t)hoff[l] * 64, *v = zt + (size_t)blk_zoff[k] * 64;
+        const double *hw = h_weight + hoff[l];
+        double p[4] = {0.0, 0.0, 0.0, 0.0};
         int t = 0;
-        for (; t + 4 <= nloc; t += 4) {
-            p0 += h_weight[h0 + t] * cdotre(dut[(size_t)(h0 + t) * 64], zt[(size_t)(z0 + t) * 64]);
-            p1 += h_weight[h0 + t + 1] * cdotre(dut[(size_t)(h0 + t + 1) * 64], zt[(size_t)(z0 + t + 1) * 64]);
-            p2 += h_weight[h0 + t + 2] * cdotre(dut[(size_t)(h0 + t + 2) * 64], zt[(size_t)(z0 + t + 2) * 64]);
-            p3 += h_weight[h0 + t + 3] * cdotre(dut[(size_t)(h0 + t + 3) * 64], zt[(size_t)(z0 + t + 3) * 64]);
-        }
-        for (; t < nloc; t++)
-            p0 += h_weight[h0 + t] * cdotre(dut[(size_t)(h0 + t) * 64], zt[(size_t)(z0 + t) * 64]);
-        pk[k * 64 + lane] = 2.0 * ((p0 + p1) + (p2 + p3));
-    }
-    __syncthreads();
-    const int64_t i = tile * 64 + lane;
-    if (i >= natoms) return;
-    for (int b = wv; b < nb; b += nw) {
-        double acc = 0.0;
+        for (; t + 8 <= nloc; t += 8) {
+            cd uu[8], vv[8];
 #pragma unroll
-        for (int t = 0; t < 3; t++) {
-            const int k = b_src[3 * b + t];
-            if (k >= 0) acc += b_srcf[3 * b + t] * pk[k * 64 + lane];
+            for (int c = 0; c < 8; c++) vv[c] = v[(size_t)(t + c) * 64], uu[c] = u[(size_t)(t + c) * 64];
+#pragma unroll
+            for (int c = 0; c < 8; c++) p[c & 3] += hw[t + c] * cdotre(uu[c], vv[c]);
         }
-        db[(size_t)i * nb + b] = acc;
+        if (t + 4 <= nloc) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) p[c] += hw[t + c] * cdotre(u[(size_t)(t + c) * 64], v[(size_t)(t + c) * 64]);
+            t += 4;
+        }
+        for (; t < nloc; t++) p[0] += hw[t] * cdotre(u[(size_t)t * 64], v[(size_t)t * 64]);
+        acc += b_srcf[3 * b + s] * (2.0 * ((p[0] + p[1]) + (p[2] + p[3])));
     }
+    const int64_t i = tile * 64 + lane;
+    if (i < natoms) db[(size_t)i * nb + b] = acc;
 }
 
 // Atom-major copy of the tile-major Z: za[i][e] = Z[i/64][e][i%64].  A
@@ -2629,13 +2629,11 @@ static int so4_tangent_launch(const pxff_so4_params *p, const So4Dev *T, int64_t
     }
 #undef PXFF_ACCUM_TAN
     PXFF_LAUNCH_CHECK();
-    const size_t lds = sizeof(double) * 64 * (size_t)T->nblk;
-    if (lds > 65536)
-        PXFF_HIP_CHECK(hipFuncSetAttribute((const void *)so4_tangent_b_kernel,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    so4_tangent_b_kernel<<<(unsigned)div_up(natoms, 64), TANB_THREADS, lds, s>>>(
-        natoms, T->nhalf, T->nz, T->nb, T->nblk, p->twol + 1, d_dutot, d_z, T->h_weight, T->hoff,
-        T->blk_level_start, T->blk_zoff, T->b_src, T->b_srcf, d_db);
+    const int64_t tgrid = div_up(div_up(natoms, 64), TANB_XCDS) * (int64_t)TANB_XCDS * div_up(T->nb, TANB_WAVES);
+    PXFF_REQUIRE(tgrid <= 0x7fffffff, "too many atoms for one launch");
+    so4_tangent_b_kernel<<<(unsigned)tgrid, TANB_WAVES * 64, 0, s>>>(
+        natoms, T->nhalf, T->nz, T->nb, p->twol + 1, d_dutot, d_z, T->h_weight, T->hoff, T->blk_level_start,
+        T->blk_zoff, T->b_src, T->b_srcf, d_db);
     PXFF_LAUNCH_CHECK();
     return 0;
 }

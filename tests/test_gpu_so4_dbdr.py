@@ -67,3 +67,26 @@ def test_utot_centres_per_wavefront(n, twol):
         ref = torch.empty_like(t)
         so4.tangent_noalloc(nl, cfg, w, z, dr, ref)
         assert float((t - ref).norm() / ref.norm()) < 1e-13
+
+
+# one atom, the edges of a 64-atom tile, more tiles than XCDs, a last tile of one atom
+@pytest.mark.parametrize("n,twol", [(1, 8), (2, 0), (63, 2), (64, 8), (65, 10), (513, 4), (577, 6)])
+def test_tangent_b_against_dbdr(n, twol):
+    """dB along displacements against the sum over images of dB/dr (sums of
+    at most a few thousand FP64 terms: 1e-12 of the norm)."""
+    from pyxtal_ff_amd import so4
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    rng = np.random.default_rng(n + twol)
+    side = int(np.ceil(n ** (1 / 3)))
+    at = np.stack(np.unravel_index(np.arange(n), (side,) * 3), 1) * 2.3
+    pos = at + rng.uniform(0, 0.4, (n, 3))
+    nl = DeviceNeighborList([pos], [np.eye(3) * (side * 2.3 + 50.0)], [np.zeros(3, bool)], 4.3)
+    cfg = so4.So4Config(twol, 4.3, 0.99363)
+    g = torch.Generator().manual_seed(n)
+    w = torch.rand(n, dtype=torch.float64, generator=g).cuda() + 0.5
+    dr = torch.randn(nl.nimg, 3, dtype=torch.float64, generator=g).cuda()
+    _, z, _ = so4.forward(nl, cfg, w, w)
+    db = so4.tangent(nl, cfg, w, z, dr).view(-1)[: n * cfg.nb].view(n, cfg.nb)
+    per_image = so4.dbdr(nl, cfg, w, z)[: nl.nimg * cfg.nb * 3].view(nl.nimg, cfg.nb, 3)
+    ref = torch.zeros_like(db).index_add(0, nl.img_atom[: nl.nimg], (per_image * dr[:, None, :]).sum(2))
+    assert float((db - ref).norm()) <= 1e-12 * max(float(ref.norm()), 1e-300)
