@@ -124,6 +124,17 @@ int pxff_nlist_count_slots(const double *d_pos, int64_t natoms, const int64_t *d
                            int32_t *d_bin_atoms, int64_t *d_img_count, int slot, int64_t *d_slot_j,
                            int32_t *d_slot_T, double *d_slot_r, int64_t *d_row_count, void *stream);
 
+/* pxff_nlist_count_slots with room for the atoms in bin order, which large
+ * lists are counted from (same output): d_bin_pos [natoms*3] double,
+ * d_bin_tag [natoms*4] int32, 16-byte aligned. */
+int pxff_nlist_count_binned(const double *d_pos, int64_t natoms, const int64_t *d_atom_struct,
+                            const int64_t *d_atom_start, const double *d_cells, const double *d_inv_cells,
+                            const int32_t *d_pbc, const int32_t *d_geom, int64_t nbins_total, double rc,
+                            int32_t *d_bin_count, int32_t *d_bin_start, int32_t *d_atom_bin, int32_t *d_wrap,
+                            int32_t *d_bin_atoms, int64_t *d_img_count, int slot, int64_t *d_slot_j,
+                            int32_t *d_slot_T, double *d_slot_r, int64_t *d_row_count, double *d_bin_pos,
+                            int32_t *d_bin_tag, void *stream);
+
 /* Phase 2: fill images (sorted per centre by (j, T)) and count seq rows.
  *   d_img_start [natoms+1] int64 = exclusive scan of d_img_count.
  *   Outputs: d_img_atom [nimg] int64 (centre), d_img_j [nimg] int64,

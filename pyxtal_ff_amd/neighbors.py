@@ -177,7 +177,9 @@ class NeighborListBuilder:
         self._ws = dict(bin_count=torch.empty(nb, **i32), bin_start=torch.empty(nb + 1, **i32),
                         atom_bin=torch.empty(max(n, 1), **i32), wrap=torch.empty(max(n, 1) * 3, **i32),
                         bin_atoms=torch.empty(max(n, 1), **i32), slot_j=torch.empty(sl, **i64),
-                        slot_T=torch.empty(sl * 3, **i32), slot_r=torch.empty(sl * 3, dtype=torch.float64, device=dev))
+                        slot_T=torch.empty(sl * 3, **i32), slot_r=torch.empty(sl * 3, dtype=torch.float64, device=dev),
+                        bin_pos=torch.empty(max(n, 1) * 3, dtype=torch.float64, device=dev),
+                        bin_tag=torch.empty(max(n, 1) * 4, **i32))
 
         # image capacity of the next build: the arrays are sized before the
         # image count is known on the host (no synchronisation in build);
@@ -251,12 +253,12 @@ class DeviceNeighborList:
         ws = self.builder._ws
         p = nat.ptr
         self._row_count = torch.empty(max(self.natoms, 1), dtype=torch.int64, device=self.pos.device)
-        nat.check(nat.lib().pxff_nlist_count_slots(
+        nat.check(nat.lib().pxff_nlist_count_binned(
             p(self.pos), self.natoms, p(self.atom_struct), p(self.atom_start), p(self.cells), p(self.inv_cells),
             p(self.pbc), p(self.geom), max(self.builder.nbins, 1), self.rc, p(ws["bin_count"]), p(ws["bin_start"]),
             p(ws["atom_bin"]), p(ws["wrap"]), p(ws["bin_atoms"]), p(self._img_count), self.builder.SLOT,
-            p(ws["slot_j"]), p(ws["slot_T"]), p(ws["slot_r"]), p(self._row_count), nat.stream()),
-            "pxff_nlist_count_slots")
+            p(ws["slot_j"]), p(ws["slot_T"]), p(ws["slot_r"]), p(self._row_count), p(ws["bin_pos"]),
+            p(ws["bin_tag"]), nat.stream()), "pxff_nlist_count_binned")
 
     def _fill(self, cap):
         """Scan (clamped to cap), fill and reverse phases into arrays of cap
