@@ -92,7 +92,8 @@ def _geometries(cells, pbcs, rc):
 def to_device(device, *arrays):
     """The arrays as device tensors, by one host-to-device copy (each copy
     costs about 16 us of host time whatever its size); the tensors are parts
-    of one allocation, 256 bytes apart."""
+    of one allocation, 256 bytes apart, each with a version counter of its own
+    (writing into one leaves what autograd saved of the others valid)."""
     arrays = [np.ascontiguousarray(a) for a in arrays]
     at = [0]
     for a in arrays:
@@ -101,7 +102,7 @@ def to_device(device, *arrays):
     for a, o in zip(arrays, at):
         buf[o: o + a.nbytes] = a.reshape(-1).view(np.uint8)
     d = torch.as_tensor(buf, device=device)
-    return [d[o: o + a.nbytes].view(getattr(torch, a.dtype.name)).view(a.shape) for a, o in zip(arrays, at)]
+    return [d[o: o + a.nbytes].view(getattr(torch, a.dtype.name)).view(a.shape).data for a, o in zip(arrays, at)]
 
 
 # bytes of page-locked memory that one to_host call may take, and from where on

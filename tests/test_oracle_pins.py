@@ -242,3 +242,16 @@ def test_grids_of_all_structures_equal_those_of_each():
     cells[0] = 0.0
     with pytest.raises(np.linalg.LinAlgError):
         _geometries(cells, pbcs, 4.9)
+
+
+def test_parts_of_one_copy_are_independent_for_autograd():
+    """Positions written in place between a forward and its backward leave an
+    index from the same copy usable."""
+    import torch
+    from pyxtal_ff_amd.neighbors import to_device
+    pos, index = to_device(torch.device("cpu"), np.zeros((3, 3)), np.array([0, 0, 1], dtype=np.int64))
+    v = torch.ones(2, dtype=torch.float64, requires_grad=True)
+    e = v.index_select(0, index).sum()
+    pos.add_(1.0)
+    e.backward()
+    assert v.grad.tolist() == [2.0, 1.0]
