@@ -322,6 +322,39 @@ __global__ __launch_bounds__(256) void so4_brow_sum_kernel(int64_t natoms, int n
     bout[(size_t)i * nb + b] = 2.0 * s;
 }
 
+// The same sums, a workgroup per 64-atom tile with its sixteen wavefronts on
+// the components; the tile's B goes through LDS and out as one contiguous run
+// (above, every 8-byte store of a wavefront is in another row of B, and the
+// workgroups that fill a row's lines run far apart).  For lists with enough
+// tiles to occupy the chip; us, per component / per tile, 2J = 8: 64 tiles
+// 5.1 / 6.3, 125 8.6 / 8.8, 275 21.6 / 13.9, 512 34.4 / 22.3, 1000 70 / 47,
+// 1728 128 / 83.
+constexpr int BROW_TILES = 192;  // tiles from which it is used
+constexpr int BROW_THREADS = 1024;
+__global__ __launch_bounds__(BROW_THREADS) void so4_brow_tile_kernel(int64_t natoms, int nb, int nbrow,
+                                                                     const int *__restrict__ b_brow0,
+                                                                     const int *__restrict__ b_level,
+                                                                     const double *__restrict__ bpart,
+                                                                     double *__restrict__ bout) {
+    extern __shared__ double sb[];  // [64][nb]
+    const int lane = threadIdx.x & 63;
+    const int64_t tile = blockIdx.x;
+    const double *pt = bpart + (size_t)tile * nbrow * 64 + lane;
+    for (int b = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); b < nb; b += BROW_THREADS / 64) {
+        const int r0 = b_brow0[b];
+        const int nr = b_level[b] / 2 + 1;
+        double s = 0.0;
+#pragma unroll 4
+        for (int r = 0; r < nr; r++) s += pt[(size_t)(r0 + r) * 64];
+        sb[lane * nb + b] = 2.0 * s;
+    }
+    __syncthreads();
+    const int64_t left = natoms - tile * 64;
+    const int n = (left < 64 ? (int)left : 64) * nb;
+    double *out = bout + (size_t)tile * 64 * nb;
+    for (int k = threadIdx.x; k < n; k += BROW_THREADS) out[k] = sb[k];
+}
+
 }  // namespace pxff
 
 // =================================================================== C ABI
@@ -347,8 +380,14 @@ extern "C" int pxff_so4_zb(const pxff_so4_params *p, int64_t natoms, const doubl
                                                                            T->nbrow)));
     PXFF_LAUNCH_CHECK();
     if (d_b) {
-        const dim3 gb((unsigned)ntiles, (unsigned)div_up(T->nb, 4));
-        so4_brow_sum_kernel<<<gb, 256, 0, s>>>(natoms, T->nb, T->nbrow, T->b_brow0, T->b_level, bpart, d_b);
+        if (ntiles >= BROW_TILES) {
+            const size_t lds = sizeof(double) * 64 * (size_t)T->nb;  // at most 46.6 KB (2J = 10)
+            so4_brow_tile_kernel<<<(unsigned)ntiles, BROW_THREADS, lds, s>>>(natoms, T->nb, T->nbrow, T->b_brow0,
+                                                                            T->b_level, bpart, d_b);
+        } else {
+            const dim3 gb((unsigned)ntiles, (unsigned)div_up(T->nb, 4));
+            so4_brow_sum_kernel<<<gb, 256, 0, s>>>(natoms, T->nb, T->nbrow, T->b_brow0, T->b_level, bpart, d_b);
+        }
         PXFF_LAUNCH_CHECK();
     }
     return 0;

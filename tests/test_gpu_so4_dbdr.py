@@ -90,3 +90,22 @@ def test_tangent_b_against_dbdr(n, twol):
     per_image = so4.dbdr(nl, cfg, w, z)[: nl.nimg * cfg.nb * 3].view(nl.nimg, cfg.nb, 3)
     ref = torch.zeros_like(db).index_add(0, nl.img_atom[: nl.nimg], (per_image * dr[:, None, :]).sum(2))
     assert float((db - ref).norm()) <= 1e-12 * max(float(ref.norm()), 1e-300)
+
+
+# the last list summed per component, the first per tile (its last tile one atom), and past it
+@pytest.mark.parametrize("n,twol", [(12224, 4), (12225, 0), (12225, 10), (12288, 2), (12351, 8)])
+def test_b_row_sums(n, twol):
+    """B summed from the Z kernel's row partials against B from U_tot and Z
+    (a few dozen FP64 terms in another order: 1e-13 of the norm)."""
+    from pyxtal_ff_amd import so4
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    rng = np.random.default_rng(n + twol)
+    side = int(np.ceil(n ** (1 / 3)))
+    pos = np.stack(np.unravel_index(np.arange(n), (side,) * 3), 1) * 2.6 + rng.uniform(0, 0.4, (n, 3))
+    nl = DeviceNeighborList([pos], [np.eye(3) * (side * 2.6 + 50.0)], [np.zeros(3, bool)], 3.5)
+    cfg = so4.So4Config(twol, 3.5, 0.99363)
+    w = torch.rand(n, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda() + 0.5
+    b, z, u = so4.forward(nl, cfg, w, w)
+    ref = so4.bi(nl, cfg, u, z)
+    assert float((b - ref).norm() / ref.norm()) < 1e-13
+    assert float((b[-1] - ref[-1]).norm() / ref[-1].norm()) < 1e-13
