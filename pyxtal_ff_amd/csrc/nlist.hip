@@ -516,9 +516,18 @@ __global__ void nl_row_rev_kernel(int64_t nrows, const int64_t *__restrict__ seq
 constexpr int NL_KMAX = 128;  // 7 KB of LDS per centre: many resident wavefronts
 
 struct NlHit {
-    int64_t j;
-    int32_t T[4];
+    int32_t j, T[3];
     double r[3];
+};
+// LDS of a wavefront beside its hits: the stencil's prefixes and bins while it
+// enumerates, the sort keys after that
+struct NlShared {
+    union {
+        struct {
+            int pref[64], info[256];
+        };
+        uint64_t keys[NL_KMAX];
+    };
 };
 
 constexpr int NL_U = 4;  // candidate rounds per step, their loads in flight together
@@ -663,7 +672,7 @@ __device__ __forceinline__ int nl_wave_enumerate(int64_t i, int lane, const doub
                     const int rank = count + (int)__popcll(mask & ((1ull << lane) - 1ull));
                     if (rank < NL_KMAX) {
                         NlHit &h = hits[rank];
-                        h.j = j[u];
+                        h.j = (int32_t)j[u];
                         h.T[0] = T0;
                         h.T[1] = T1;
                         h.T[2] = T2;
@@ -828,10 +837,10 @@ __global__ __launch_bounds__(64) void nl_fill_wave_kernel(
     const int32_t *__restrict__ bin_atoms, const int64_t *__restrict__ img_start, int64_t *__restrict__ img_atom,
     int64_t *__restrict__ img_j, int32_t *__restrict__ img_T, double *__restrict__ img_r,
     int64_t *__restrict__ row_count) {
-    __shared__ int s_pref[64];
-    __shared__ int s_info[256];
+    __shared__ NlShared sh;
     __shared__ NlHit hits[NL_KMAX];
-    __shared__ uint64_t keys[NL_KMAX];
+    int *s_pref = sh.pref, *s_info = sh.info;
+    uint64_t *keys = sh.keys;
     const int64_t i = blockIdx.x;
     if (i >= natoms) return;
     nl_fill_centre(i, threadIdx.x, pos, atom_struct, cells, pbc, geom, rc2, bin_start, atom_bin, wrap, bin_atoms,
@@ -844,18 +853,23 @@ __global__ __launch_bounds__(64) void nl_fill_wave_kernel(
 // (slot_j / slot_T / slot_r at [i * slot, i * slot + count)) together with
 // its seq-row count; nl_fill_slots_kernel then copies the slots into place
 // after the scan, so those centres are enumerated once per build.
+// Wavefronts in flight hide its chains: with 6.4 KB of LDS per centre (8.4
+// with wider hits and keys of their own) and, in bin order, six wavefronts per
+// SIMD (five without the bound) binning and count of 133,621 atoms in 1024
+// cells take 307 us, before 340, of 60,000 atoms 145, before 158.  By index
+// six are slower (12,000 atoms 52 -> 54 us).
 template <bool BINNED>
-__global__ __launch_bounds__(64) void nl_count_slots_kernel(
+__global__ __launch_bounds__(64, BINNED ? 6 : 1) void nl_count_slots_kernel(
     int64_t natoms, const double *__restrict__ pos, const int64_t *__restrict__ atom_struct,
     const double *__restrict__ cells, const int32_t *__restrict__ pbc, const int32_t *__restrict__ geom, double rc2,
     const int32_t *__restrict__ bin_start, const int32_t *__restrict__ atom_bin, const int32_t *__restrict__ wrap,
     const int32_t *__restrict__ bin_atoms, int64_t *__restrict__ img_count, int slot, int64_t *__restrict__ slot_j,
     int32_t *__restrict__ slot_T, double *__restrict__ slot_r, int64_t *__restrict__ row_count,
     const double *__restrict__ bpos, const int4 *__restrict__ btag) {
-    __shared__ int s_pref[64];
-    __shared__ int s_info[256];
+    __shared__ NlShared sh;
     __shared__ NlHit hits[NL_KMAX];
-    __shared__ uint64_t keys[NL_KMAX];
+    int *s_pref = sh.pref, *s_info = sh.info;
+    uint64_t *keys = sh.keys;
     const int lane = threadIdx.x;
     const int64_t i = blockIdx.x;
     if (i >= natoms) return;  // uniform for the whole workgroup
@@ -888,10 +902,10 @@ __global__ __launch_bounds__(64) void nl_fill_slots_kernel(
     int slot, const int64_t *__restrict__ slot_j, const int32_t *__restrict__ slot_T,
     const double *__restrict__ slot_r, int64_t *__restrict__ img_atom, int64_t *__restrict__ img_j,
     int32_t *__restrict__ img_T, double *__restrict__ img_r, int64_t *__restrict__ row_count) {
-    __shared__ int s_pref[64];
-    __shared__ int s_info[256];
+    __shared__ NlShared sh;
     __shared__ NlHit hits[NL_KMAX];
-    __shared__ uint64_t keys[NL_KMAX];
+    int *s_pref = sh.pref, *s_info = sh.info;
+    uint64_t *keys = sh.keys;
     const int lane = threadIdx.x;
     const int64_t i = blockIdx.x;
     if (i >= natoms) return;
@@ -1049,7 +1063,7 @@ extern "C" int pxff_nlist_count(const double *d_pos, int64_t natoms, const int64
 // copies cost a launch (3 us), and below some thousand atoms the latency of a
 // few wavefronts per SIMD hides the lookups.  Binning and count, by index /
 // binned, us: silicon 1000 atoms 15.5 / 19, 4096 19.5 / 21.4; silica 5000
-// atoms 32 / 29.4, 8000 39.7 / 34.5, 12,000 54 / 45, 60,000 190 / 158.
+// atoms 32 / 29.4, 8000 39.7 / 34.5, 12,000 52 / 43, 60,000 187 / 145.
 constexpr int64_t NL_BINNED_ATOMS = 8000;
 
 static int nl_count_slots(const double *d_pos, int64_t natoms, const int64_t *d_atom_struct,
