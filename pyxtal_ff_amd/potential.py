@@ -369,8 +369,12 @@ def energy_forces_plain(nl, cfg, atom_w, site_w, model, species, stress=False):
     grad = dev_so4.dxdr_contract(nl, cfg.nb, beta, dx)
     out = {"energy": e_atom.sum(), "forces": -grad, "atom_energies": e_atom}
     if stress:
-        seg = nl.atom_start[:: len(nl.atom_start) - 1].contiguous()  # [0, N]
-        out["stress_voigt"] = _segment_total(dev_so4.voigt_contract(beta, rv), seg)
+        s_atom = dev_so4.voigt_contract(beta, rv)
+        if nl.natoms:
+            seg = nl.atom_start[:: len(nl.atom_start) - 1].contiguous()  # [0, N]
+            out["stress_voigt"] = _segment_total(s_atom, seg)
+        else:  # a list without structures has no segment
+            out["stress_voigt"] = s_atom.sum(0)
     return out
 
 

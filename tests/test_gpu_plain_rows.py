@@ -115,3 +115,22 @@ def test_row_index(kind):
     assert np.array_equal(nl.row_img.cpu().numpy()[: n + 1], row_img)
     assert np.array_equal(nl.img_row.cpu().numpy()[: nl.nimg], np.array(img_row, dtype=np.int64))
     assert np.array_equal(nl.nsite.cpu().numpy(), nsite)
+
+
+@pytest.mark.parametrize("stress", [False, True])
+@pytest.mark.parametrize("structures", [0, 1, 2])
+def test_plain_path_without_atoms(structures, stress):
+    """Energy, forces and stress of lists of no atoms: zeros, no error."""
+    import numpy as np
+    from pyxtal_ff_amd import potential, so4
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    nl = DeviceNeighborList([np.zeros((0, 3))] * structures, np.tile(np.eye(3) * 9.0, (structures, 1, 1)),
+                            np.ones((structures, 3), dtype=bool), 4.9)
+    cfg = so4.So4Config(4, 4.9, 0.99363)
+    w = torch.ones(0, dtype=torch.float64, device="cuda")
+    model = potential.NNPotential(["Si"], cfg.nb).cuda()
+    species = [("Si", torch.zeros(0, dtype=torch.int64, device="cuda"))]
+    out = potential.energy_forces_plain(nl, cfg, w, w, model, species, stress=stress)
+    assert float(out["energy"]) == 0.0 and out["forces"].shape == (0, 3) and out["atom_energies"].shape == (0,)
+    if stress:
+        assert torch.equal(out["stress_voigt"].cpu(), torch.zeros(6, dtype=torch.float64))
