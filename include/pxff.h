@@ -317,8 +317,10 @@ int pxff_so4_tangent(const pxff_so4_params *p, int64_t natoms, const int64_t *d_
                      double *d_dutot, double *d_db, void *stream);
 
 /* pxff_so4_tangent with room for the per-image values of its sweeps: d_stage
- * [cap*10], images past cap (none in a list of that capacity) not counted.
- * Long lists then take several centres per wavefront. */
+ * [cap*10]; cap must be at least the image count.  Long lists then take
+ * several centres per wavefront; there a record past cap is neither written
+ * nor read, and its image is missing from the sums.  Short lists, 2J = 10 and
+ * a null d_stage (cap = 0) use no records and sum every image. */
 int pxff_so4_tangent_staged(const pxff_so4_params *p, int64_t natoms, const int64_t *d_img_start,
                             const int64_t *d_img_j, const double *d_img_r, const double *d_atom_w,
                             const double *d_dr, const double *d_z, int64_t cap, double *d_stage, double *d_dutot,

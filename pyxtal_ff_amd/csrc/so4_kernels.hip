@@ -1119,7 +1119,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
 template <int TWOJ, bool TANGENT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so4_utot_group_kernel(
     int64_t natoms, int split, const int64_t *__restrict__ img_start, const double *__restrict__ site_w,
-    const double *__restrict__ lnorm_g, double fcut0, const double *__restrict__ stage, double *__restrict__ out) {
+    const double *__restrict__ lnorm_g, double fcut0, int64_t cap, const double *__restrict__ stage,
+    double *__restrict__ out) {
     constexpr int G = TWOJ / 2 + 1;
     constexpr int NG = 64 / G;
     constexpr int NH = nhalf_of(TWOJ);
@@ -1144,8 +1145,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void so
     const int cpw = NG / split, c = g / split, p = g - c * split;
     const int64_t i = (int64_t)blockIdx.x * cpw + c;
     const bool mine = c < cpw && i < natoms;
-    const int64_t s = mine ? img_start[i] : 0;
-    const int n = mine ? (int)(img_start[i + 1] - s) : 0;
+    // images past the cap staged records have none
+    const int64_t s = mine ? img_start[i] : 0, s1 = mine ? min(img_start[i + 1], cap) : 0;
+    const int n = s1 > s ? (int)(s1 - s) : 0;
     const double wself = mine && !TANGENT ? site_w[i] : 0.0;
     cd acc[NSLOT];
 #pragma unroll
@@ -2487,8 +2489,8 @@ extern "C" int pxff_so4_ui_staged(const pxff_so4_params *p, int64_t natoms, cons
             const int split = NG / (int)std::min<int64_t>(NG, want);
             const int64_t grid = div_up(natoms, NG / split);
             PXFF_REQUIRE(grid <= 0x7fffffff, "too many atoms for one launch");
-            so4_utot_group_kernel<TJ, false><<<(unsigned)grid, 64, 0, s>>>(natoms, split, d_img_start, d_site_w, T->lnorm,
-                                                                  fcut0, d_stage, d_utot);
+            so4_utot_group_kernel<TJ, false><<<(unsigned)grid, 64, 0, s>>>(natoms, split, d_img_start, d_site_w,
+                                                                           T->lnorm, fcut0, cap, d_stage, d_utot);
         } else {
             const int grid =
                 (int)std::min<int64_t>(natoms, (int64_t)num_cus() * tune_value(PXFF_TUNE_ACCUM_WAVES_PER_CU));
@@ -2637,7 +2639,7 @@ static int so4_tangent_launch(const pxff_so4_params *p, const So4Dev *T, int64_t
             const int64_t ngrid = div_up(natoms, NG / split);
             PXFF_REQUIRE(ngrid <= 0x7fffffff, "too many atoms for one launch");
             so4_utot_group_kernel<TJ, true><<<(unsigned)ngrid, 64, 0, s>>>(natoms, split, d_img_start, nullptr,
-                                                                          T->lnorm, 0.0, d_stage, d_dutot);
+                                                                          T->lnorm, 0.0, cap, d_stage, d_dutot);
         });
     } else if (mode == 4 && p->twol <= 8) {
         PXFF_DISPATCH_TWOJ(p->twol, if constexpr (TJ <= 8) {

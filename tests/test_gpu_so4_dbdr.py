@@ -109,3 +109,35 @@ def test_b_row_sums(n, twol):
     ref = so4.bi(nl, cfg, u, z)
     assert float((b - ref).norm() / ref.norm()) < 1e-13
     assert float((b[-1] - ref[-1]).norm() / ref[-1].norm()) < 1e-13
+
+
+# five, four and one lane groups to a centre; a cap of no, one, some and all images
+@pytest.mark.parametrize("n", [4096, 6001, 13000])
+@pytest.mark.parametrize("part", [0.0, 1e-9, 0.37, 1.0])
+def test_staged_tangent_stays_within_its_records(n, part):
+    """pxff_so4_tangent_staged with room for `cap` records writes and reads
+    none past them: the images after that add nothing, as with zero
+    displacements (the sums only lose zeros: the same bits)."""
+    from pyxtal_ff_amd import _native as nat, so4
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    rng = np.random.default_rng(n)
+    side = int(np.ceil((n / 4) ** (1 / 3)))
+    owner = np.arange(n) // 4
+    at = np.stack([owner % side, owner // side % side, owner // side**2], 1) * 20.0
+    pos = at + rng.uniform(0, 2.4, (n, 3))
+    nl = DeviceNeighborList([pos], [np.eye(3) * (side * 20.0 + 50.0)], [np.zeros(3, bool)], 4.3)
+    ne = nl.nimg
+    cfg = so4.So4Config(4, 4.3, 0.99363)
+    w = torch.rand(n, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda() + 0.5
+    _, z, _ = so4.forward(nl, cfg, w, w)
+    dr = torch.randn(ne * 3, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda()
+    cap = int(np.ceil(part * ne))
+    stage = torch.full((ne * 10,), float("nan"), dtype=torch.float64, device="cuda")
+    du = torch.empty(2 * cfg.nhalf * 64 * ((n + 63) // 64), dtype=torch.float64, device="cuda")
+    db = torch.empty((n, cfg.nb), dtype=torch.float64, device="cuda")
+    p = nat.ptr
+    nat.check(nat.lib().pxff_so4_tangent_staged(cfg.params, n, p(nl.img_start), p(nl.img_j), p(nl.img_r), p(w), p(dr),
+                                                p(z), cap, p(stage), p(du), p(db), nat.stream()), "tangent")
+    assert bool(stage[cap * 10:].isnan().all())
+    dr[3 * cap:] = 0.0
+    assert torch.equal(db, so4.tangent(nl, cfg, w, z, dr))
