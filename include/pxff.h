@@ -510,7 +510,9 @@ int pxff_so3_adjoint_a(const pxff_so3_params *p, int64_t natoms, const double *d
                        double *d_a, void *stream);
 
 /* Adjoint: dE/dr per image [nimg*3] (angular part and expansion recomputed
- * per image; radial integrals from d_radial when not NULL, else recomputed). */
+ * per image; radial integrals from d_radial when not NULL, else recomputed).
+ * d_a is any full array [natoms][nmax][lmax+1][2lmax+1]; it need not have the
+ * symmetry of the expansion. */
 int pxff_so3_deidrj(const pxff_so3_params *p, int64_t nimg, const int64_t *d_img_atom, const int64_t *d_img_j,
                     const double *d_img_r, const int64_t *d_atom_z, const double *d_G, const double *d_rq,
                     const double *d_lnorm, const double *d_a, const double *d_radial, double *d_dedr,

@@ -1502,17 +1502,23 @@ __device__ __forceinline__ double so3_dpp(double v) {
 // several of them.  One batch per wavefront: in a loop over batches the
 // constants of the cutoff and the exponential are held in registers across
 // it (256 of them and one wavefront per SIMD).
-// 407k images at 6/6: 111 us, 2.5 TB/s of radial rows, two wavefronts per
-// SIMD; 5.8k images at 3/4: 11 us (its forerunner with a lane per (l, m), a Y
+// 407k images at 6/6: 101 us, 2.7 TB/s of radial rows, two wavefronts per
+// SIMD (120 with a branch around the loads of the second order); 5.8k images
+// at 3/4: 11 us (its forerunner with a lane per (l, m), a Y
 // table and 64-lane sums: 215 and 56 us).
+// HALF: A is the m >= 0 half and stands for a full A with the symmetry of the
+// expansion.  Else A is full and any: only A_m + (-1)^m conj(A_-m) enters the
+// sums (A_0's real part), which a lane forms as it loads its orders, without
+// branches around the loads (407k images at 6/6: 104 us, 166 with them).  For
+// an A with the symmetry that is 2 A_m exactly, the same bits.
 constexpr int SO3_AB = 32;  // images per batch, SO3_AB / 4 per row of lanes
-template <int NMAX>
+template <int NMAX, bool HALF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NMAX <= 4 ? 3 : 2))) void so3_deidrj_half_kernel(
                                                              So3Args a, int64_t nimg, const int64_t *__restrict__ img_atom,
                                                              const int64_t *__restrict__ img_j,
                                                              const double *__restrict__ img_r,
                                                              const int64_t *__restrict__ atom_z,
-                                                             const double *__restrict__ A, int half,
+                                                             const double *__restrict__ A,
                                                              const double *__restrict__ rad, double *__restrict__ dedr,
                                                              const int64_t *__restrict__ d_count) {
     constexpr int LM = 7, PER = SO3_AB / 4;
@@ -1533,12 +1539,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NMAX <= 4 ? 
     const int lane = threadIdx.x, g = lane >> 4, gl = lane & 15;
     const int L = a.lmax + 1, nf = L * 2 * NMAX, RS = nf + 2;
     const So3Lane ln = so3_lane(gl, a.lmax);
-    const double sc0 = ln.on0 ? a.lnorm[ln.l] * (ln.m0 ? 2.0 : 1.0) : 0.0, sc1 = ln.on1 ? 2.0 * a.lnorm[ln.l] : 0.0;
+    const double two = HALF ? 2.0 : 1.0;
+    const double sc0 = ln.on0 ? a.lnorm[ln.l] * (ln.m0 ? two : 1.0) : 0.0, sc1 = ln.on1 ? two * a.lnorm[ln.l] : 0.0;
+    const int on1 = ln.on1 ? 1 : 0;
+    const double two0 = ln.m0 > 0 ? 1.0 : 0.0;  // A_0 counts once
     const double dm0 = ln.m0, dm1 = ln.m0 + 1;
     const int iz = ln.m0 + 1 < LM ? ln.m0 + 1 : LM - 1, ip = ln.m0 > 0 ? ln.m0 - 1 : 0;
     const int NH = L * (L + 1) / 2, M2 = 2 * a.lmax + 1;
-    const int astep = half ? NH : L * M2, asize = NMAX * astep;
-    const int aoff = half ? ln.l * (ln.l + 1) / 2 + ln.m0 : ln.l * M2 + a.lmax + ln.m0;
+    const int astep = HALF ? NH : L * M2, asize = NMAX * astep;
+    const int aoff = HALF ? ln.l * (ln.l + 1) / 2 + ln.m0 : ln.l * M2 + a.lmax + ln.m0;
     // the lane's share of 8 radial rows: unit k of row pair s = k / nf
     int gof[NLD], lof[NLD];
 #pragma unroll
@@ -1607,7 +1616,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NMAX <= 4 ? 
             const cd *ai = reinterpret_cast<const cd *>(A) + (size_t)i * asize + aoff;
 #pragma unroll
             for (int n = 0; n < NMAX; n++) {
-                const cd x0 = ai[n * astep], x1 = ln.on1 ? ai[n * astep + 1] : x0;
+                cd x0 = ai[n * astep], x1 = ai[n * astep + on1];
+                if (!HALF) {  // orders -m0 (even) and -m0 - 1 (odd); no branch around the loads
+                    const cd y0 = ai[n * astep - 2 * ln.m0], y1 = ai[n * astep - (2 * ln.m0 + 1) * on1];
+                    x0 = cmake(fma(two0, y0.re, x0.re), fma(-two0, y0.im, x0.im));
+                    x1 = cmake(x1.re - y1.re, x1.im + y1.im);
+                }
                 Ar0[n] = sc0 * x0.re;
                 Ai0[n] = sc0 * x0.im;
                 Ar1[n] = sc1 * x1.re;
@@ -2208,9 +2222,15 @@ static int so3_deidrj_rows(const So3Args &a, int64_t nimg, const int64_t *d_img_
                            const double *d_radial, double *d_dedr, hipStream_t s, const int64_t *d_count) {
     const int64_t grid = (nimg + SO3_AB - 1) / SO3_AB;
     PXFF_REQUIRE(grid <= 0x7fffffff, "too many images for one launch");
-    SO3_DISPATCH_NMAX(a.nmax, (so3_deidrj_half_kernel<NM><<<(unsigned)grid, 64, 0, s>>>(
-                                  a, nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_a, half, d_radial, d_dedr,
-                                  d_count)));
+    if (half) {
+        SO3_DISPATCH_NMAX(a.nmax, (so3_deidrj_half_kernel<NM, true><<<(unsigned)grid, 64, 0, s>>>(
+                                      a, nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_a, d_radial, d_dedr,
+                                      d_count)));
+    } else {
+        SO3_DISPATCH_NMAX(a.nmax, (so3_deidrj_half_kernel<NM, false><<<(unsigned)grid, 64, 0, s>>>(
+                                      a, nimg, d_img_atom, d_img_j, d_img_r, d_atom_z, d_a, d_radial, d_dedr,
+                                      d_count)));
+    }
     PXFF_LAUNCH_CHECK();
     return 0;
 }

@@ -71,3 +71,27 @@ def test_so3_direct_radial_store_equals_sorted(nmax, lmax):
         _, rad = d3.ctot(nl, cfg, z, radial=True)
         rows.append(rad[: nl.nimg * (lmax + 1) * 2 * nmax].clone())
     assert torch.equal(rows[0], rows[1])
+
+
+@pytest.mark.parametrize("nmax,lmax", [(1, 0), (2, 1), (3, 4), (8, 5), (6, 6)])
+def test_so3_adjoint_of_any_a(nmax, lmax):
+    """dE/dr from a full A without the symmetry of the expansion: the same
+    with the stored radial integrals as with recomputed ones, at every
+    alignment of the store."""
+    from pyxtal_ff_amd import so3 as d3
+    from pyxtal_ff_amd import workloads
+    from pyxtal_ff_amd.neighbors import DeviceNeighborList
+    s = workloads.amorphous_sio2(11, 22, seed=nmax)
+    nl = DeviceNeighborList([s.positions], [s.cell], [s.pbc], 4.6).resolve()
+    n = nl.natoms
+    cfg = d3.So3Config(nmax, lmax, 4.6, 2.0)
+    z = torch.as_tensor(s.numbers, device="cuda")
+    _, rad = d3.ctot(nl, cfg, z, radial=True)
+    a = torch.randn(n * cfg.csz * 2, dtype=torch.float64, generator=torch.Generator().manual_seed(lmax)).cuda()
+    ref = d3.deidrj(nl, cfg, z, a)
+    off = torch.empty(rad.numel() + 1, dtype=torch.float64, device="cuda")[1:]
+    off.copy_(rad)
+    assert _rel(d3.deidrj(nl, cfg, z, a, radial=off), ref) < 1e-11
+    assert _rel(d3.deidrj(nl, cfg, z, a, radial=rad), ref) < 1e-11
+    counted = d3.deidrj(nl, cfg, z, a, radial=rad, counted=True)
+    assert _rel(counted[: nl.nimg], ref) < 1e-11
