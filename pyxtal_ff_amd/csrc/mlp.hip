@@ -4,8 +4,8 @@
 // (pyxtal_ff/models/neuralnetwork.py:80-200: nn.Linear layers with one
 // activation each, descriptors scaled by the element's drange,
 // neuralnetwork.py:938-1029) evaluated forward, then backward to dE/dx.
-// Three kernels, by what fits in LDS: 16-atom tiles on the FP64 matrix
-// cores (mlp_mfma_kernel, scratch and one element's weights within 160 KB);
+// By what fits in LDS: 16-atom tiles on the FP64 matrix cores (mlp_mfma_kernel
+// and mlp_mfma4_kernel, scratch and one element's weights within 160 KB);
 // else one wavefront per atom with lane n holding neuron n of a layer
 // (widths <= 64), the weights of every element in LDS (mlp_lds_kernel) or
 // streamed from L2 (mlp_energy_grad_kernel).
@@ -253,11 +253,10 @@ __global__ __launch_bounds__(64 * MLP_LW) void mlp_lds_kernel(int64_t natoms, in
 // and species are on their way before the element is known, those of the next
 // tile before this one is computed; the weights come a row per wavefront,
 // eight rows in flight; the layout is one register, an int per lane.
-// Four wavefronts with whole tiles and four activations to a lane, before:
-// 1000 atoms of 30 inputs 16.3 -> 13.3 us, 777 atoms of 55 inputs with two
-// elements mixed 32.6 -> 23.7, 4096 of 55 18.7 -> 14.1, 12000 of 147 65 -> 43,
-// 200000 of 55 411 -> 330; past 50000 atoms of 30 inputs, where the tanh are
-// most of the work and the call costs, 89 -> 94 us (286 -> 312 at 200000).
+// Four wavefronts with whole tiles and four activations to a lane
+// (mlp_mfma4_kernel): 1000 atoms of 30 inputs 16.3 -> 13.3 us, 777 atoms of 55
+// inputs with two elements mixed 32.6 -> 23.7, 4096 of 55 18.7 -> 14.1, 12000
+// of 147 65 -> 43, 200000 of 55 411 -> 330.
 // The element's weights are staged in LDS first, zero-padded, and every
 // activation row is zero past its width, so the GEMM steps need no bounds
 // tests (the K loops run over multiples of 4).  LDS rows are 2 doubles past
@@ -505,6 +504,189 @@ __global__ __launch_bounds__(MLP_T) __attribute__((amdgpu_waves_per_eu(4))) void
     }
 }
 
+// The same with four wavefronts to a tile, whole 16-neuron tiles per wavefront
+// and four activations to a lane, for many tiles of short inputs and narrow
+// layers: its chain through a tile is longer, but three workgroups share a CU
+// where the registers of the eight-wavefront kernel leave room for two, and
+// the tanh of many tiles are then spread better (rule at mlp_four_waves).
+// acc = sum_k A[lane & 15][k] B[k][col], k < K (a multiple of 4):
+// a = &A[lane & 15][lane >> 4] (row-major A, k steps of 4 elements),
+// b = &B[lane >> 4][col], bstep = 4 x the row stride of B.  Four
+// accumulators take the k steps in turn (four independent MFMA chains).
+__device__ inline mlp_d4 mlp_gemm_tile(int K, const double *a, const double *b, int bstep) {
+    mlp_d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0, c2 = c0, c3 = c0;
+    const int S = K >> 2;
+    int t = 0;
+    for (; t + 4 <= S; t += 4) {
+        const double a0 = a[4 * t], a1 = a[4 * t + 4], a2 = a[4 * t + 8], a3 = a[4 * t + 12];
+        const double b0 = b[t * bstep], b1 = b[(t + 1) * bstep], b2 = b[(t + 2) * bstep], b3 = b[(t + 3) * bstep];
+        c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, c1, 0, 0, 0);
+        c2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, b2, c2, 0, 0, 0);
+        c3 = __builtin_amdgcn_mfma_f64_16x16x4f64(a3, b3, c3, 0, 0, 0);
+    }
+    for (; t < S; t++) c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[4 * t], b[t * bstep], c0, 0, 0, 0);
+    return (c0 + c1) + (c2 + c3);
+}
+
+__global__ __launch_bounds__(256) void mlp_mfma4_kernel(int64_t natoms, int nin, int nelem,
+                                                        const int64_t *__restrict__ species,
+                                                        const int *__restrict__ layout,
+                                                        const double *__restrict__ params,
+                                                        const double *__restrict__ dmin,
+                                                        const double *__restrict__ scale,
+                                                        const double *__restrict__ x, double *__restrict__ e_out,
+                                                        double *__restrict__ beta, int nlm, int hw) {
+    extern __shared__ double sm[];
+    __shared__ int s_sp[MLP_TILE];  // element of each atom; -1 no network, -2 past the end
+    __shared__ int s_wo[MLP_MAXL];  // offset of layer k's padded W, then its b, in wl
+    const int P0 = mlp_row(nin), HP = mlp_row(hw);
+    double *h0 = sm;                                 // [16][P0] scaled inputs, zero-padded
+    double *hact = h0 + MLP_TILE * P0;               // [nlm][16][HP] activations
+    double *hder = hact + (size_t)nlm * MLP_TILE * HP;  // [nlm][16][HP] act', then gradients
+    double *wl = hder + (size_t)nlm * MLP_TILE * HP;    // W_k [r16(nout)][row(nin)], b_k [r16(nout)]
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    const int ri = lane & 15, kq = lane >> 4;
+    // tiles [t0, t1) of this workgroup, in order: an element's weights stay
+    // staged from one tile to the next (atoms come sorted by element)
+    const int64_t ntiles = (natoms + MLP_TILE - 1) / MLP_TILE;
+    const int64_t per = (ntiles + gridDim.x - 1) / gridDim.x;
+    const int64_t t0 = (int64_t)blockIdx.x * per, t1 = t0 + per < ntiles ? t0 + per : ntiles;
+    int staged = -1;  // element whose weights are in wl
+    for (int64_t tl = t0; tl < t1; tl++) {
+        const int64_t a0 = tl * MLP_TILE;
+        __syncthreads();  // the previous tile is done with s_sp and the scratch
+        if (tid < MLP_TILE) {
+            const int64_t a = a0 + tid;
+            int e = -2;
+            if (a < natoms) {
+                const int64_t sp = species[a];
+                e = (sp >= 0 && sp < nelem) ? (int)sp : -1;
+            }
+            s_sp[tid] = e;
+        }
+        __syncthreads();
+        for (int el = 0; el < nelem; el++) {
+            bool any = false;
+            for (int t = 0; t < MLP_TILE; t++) any = any || s_sp[t] == el;
+            if (!any) continue;  // uniform over the workgroup
+            const int *lay = layout + el * MLP_STRIDE;
+            const int nl = lay[0];
+            const double *dm = dmin + (size_t)el * nin, *sc = scale + (size_t)el * nin;
+            // staging: eight loads in flight per thread before their LDS stores
+            for (int q0 = tid; q0 < MLP_TILE * P0; q0 += 256 * 8) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int q = q0 + 256 * u;
+                    const int t = q / P0, j = q - t * P0;
+                    const int64_t a = a0 + t;
+                    v[u] = (q < MLP_TILE * P0 && a < natoms && j < nin) ? (x[(size_t)a * nin + j] - dm[j]) * sc[j]
+                                                                         : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (q0 + 256 * u < MLP_TILE * P0) h0[q0 + 256 * u] = v[u];
+            }
+            if (el != staged) {  // uniform over the workgroup
+                staged = el;
+                int wo = 0;
+                for (int k = 0; k < nl; k++) {
+                    const int *L = lay + 1 + MLP_LSTRIDE * k;
+                    const int ni = L[0], no = L[1], R = mlp_r16(no), C = mlp_row(ni);
+                    const double *W = params + L[3], *bias = params + L[4];
+                    for (int q0 = tid; q0 < R * C + R; q0 += 256 * 8) {
+                        double v[8];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) {
+                            const int q = q0 + 256 * u;
+                            v[u] = 0.0;
+                            if (q < R * C) {
+                                const int r = q / C, c = q - r * C;
+                                if (r < no && c < ni) v[u] = W[r * ni + c];
+                            } else if (q - R * C < no) {
+                                v[u] = bias[q - R * C];
+                            }
+                        }
+#pragma unroll
+                        for (int u = 0; u < 8; u++)
+                            if (q0 + 256 * u < R * C + R) wl[wo + q0 + 256 * u] = v[u];
+                    }
+                    if (tid == 0) s_wo[k] = wo;
+                    wo += R * C + R;
+                }
+            }
+            __syncthreads();
+            // forward
+            const double *hin = h0;
+            int ldi = P0;
+            for (int k = 0; k < nl; k++) {
+                const int *L = lay + 1 + MLP_LSTRIDE * k;
+                const int ni = L[0], no = L[1], act = L[2], C = mlp_row(ni);
+                const double *W = wl + s_wo[k], *bias = W + mlp_r16(no) * C;
+                double *ho = hact + (size_t)k * MLP_TILE * HP, *hd = hder + (size_t)k * MLP_TILE * HP;
+                for (int ct = wv; ct * 16 < no; ct += 4) {
+                    // D[j][i] = sum_k W[j][k] H[i][k]: A rows = neurons of the
+                    // tile, B columns = atoms
+                    const mlp_d4 acc = mlp_gemm_tile(mlp_r4(ni), W + (ct * 16 + ri) * C + kq, hin + ri * ldi + kq, 4);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int j = ct * 16 + kq + 4 * r;  // neuron; the lane's atom is ri
+                        double av = 0.0, da = 0.0;          // zero past the layer width
+                        if (j < no) act_fdf(act, acc[r] + bias[j], av, da);
+                        ho[ri * HP + j] = av;
+                        hd[ri * HP + j] = da;
+                    }
+                }
+                __syncthreads();
+                hin = ho;
+                ldi = HP;
+            }
+            if (tid < MLP_TILE && s_sp[tid] == el) e_out[a0 + tid] = hin[tid * HP];
+            // backward; hder of the output layer (one neuron) already is dE/dz
+            for (int k = nl - 1; k >= 1; k--) {
+                const int *L = lay + 1 + MLP_LSTRIDE * k;
+                const int ni = L[0], no = L[1], C = mlp_row(ni);
+                const double *W = wl + s_wo[k];
+                const double *g = hder + (size_t)k * MLP_TILE * HP;
+                double *gp = hder + (size_t)(k - 1) * MLP_TILE * HP;
+                for (int ct = wv; ct * 16 < ni; ct += 4) {
+                    const int j = ct * 16 + ri;
+                    // B[n][j] = W[n][j]
+                    const mlp_d4 acc = mlp_gemm_tile(mlp_r4(no), g + ri * HP + kq, W + kq * C + j, 4 * C);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) gp[(kq + 4 * r) * HP + j] *= acc[r];
+                }
+                __syncthreads();
+            }
+            {
+                const int *L = lay + 1;
+                const int no = L[1], C = mlp_row(nin);
+                const double *W = wl + s_wo[0];
+                for (int ct = wv; ct * 16 < nin; ct += 4) {
+                    const int j = ct * 16 + ri;
+                    const mlp_d4 acc = mlp_gemm_tile(mlp_r4(no), hder + ri * HP + kq, W + kq * C + j, 4 * C);
+                    if (j < nin) {
+                        const double sj = sc[j];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const int row = kq + 4 * r;
+                            if (s_sp[row] == el) beta[(size_t)(a0 + row) * nin + j] = acc[r] * sj;
+                        }
+                    }
+                }
+            }
+            __syncthreads();  // the next element reuses the scratch
+        }
+        // atoms without a network: NaN results
+        for (int q = tid; q < MLP_TILE * nin; q += 256) {
+            const int t = q / nin;
+            if (s_sp[t] == -1) beta[(size_t)(a0 + t) * nin + (q - t * nin)] = __builtin_nan("");
+        }
+        if (tid < MLP_TILE && s_sp[tid] == -1) e_out[a0 + tid] = __builtin_nan("");
+    }
+}
+
 // One element's parameters from their own tensors into the packed arrays
 // (layout row, W, b, W^T, dmin, scale): one launch instead of a transpose per
 // layer, a concatenation and a copy of the layout, so that a call can take the
@@ -554,6 +736,45 @@ static int mlp_check_layout(int nin, int nelem, const int *h_layout) {
         PXFF_REQUIRE(prev == 1, "the last layer must have one output (the atomic energy)");
     }
     return 0;
+}
+
+// Dynamic LDS of the matrix-core kernels: what a CU has, less their static LDS.
+constexpr size_t MLP_LDS_MAX = 160 * 1024 - 1024;
+
+// Workgroups of lds bytes that a CU's LDS keeps resident, at most `most`.
+static int64_t mlp_resident(size_t lds, int64_t most) {
+    return std::max<int64_t>(1, std::min<int64_t>(most, (int64_t)(160 * 1024) / (int64_t)(lds + 1024)));
+}
+
+// Raise a kernel's dynamic LDS limit to lds; set is the limit so far.  Under a
+// lock, so that concurrent callers never lower it below what another relies on.
+static int mlp_raise_lds(const void *kernel, int lds, std::atomic<int> &set) {
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lock(mu);
+    if (lds > set.load(std::memory_order_relaxed)) {
+        PXFF_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        set.store(lds, std::memory_order_relaxed);
+    }
+    return 0;
+}
+
+// Four wavefronts to a tile (mlp_mfma4_kernel, lds4 bytes) or eight
+// (mlp_mfma_kernel, lds8 bytes; at most two of its workgroups fit the
+// registers of a CU): by the rounds that the tiles take, a round of the four
+// being 1 + (LDS row of the inputs) / 150 of one of the eight (1.2 to 32
+// inputs, 1.4 to 64, 1.7 to 96; past three workgroups per CU more of the four
+// only slow each other).  Over 1 to 3 layers of 16 to 64, 14 to 91 inputs and 2000 to
+// 200000 atoms the choice is at most 5 % slower than the better of the two.
+// Where one of them does not fit, the other.  Measured, us, eight / four, two
+// elements, layers of 30, 30: 30 inputs, 2000 atoms 23 / 29, 8192 23 / 29,
+// 8300 32 / 29, 12000 32 / 26, 16000 39 / 46, 20000 47 / 41, 60000 104 / 90,
+// 136000 208 / 201, 200000 307 / 285; with the elements mixed 12000 61 / 44;
+// 91 inputs, 8300 38 / 42, 16000 64 / 60, 32000 114 / 104.  Layers of 16, 16
+// and 30 inputs, 12000 28 / 20, 200000 259 / 223.
+static bool mlp_four_waves(int64_t ntiles, int nin, size_t lds8, size_t lds4) {
+    if (lds4 > MLP_LDS_MAX || lds8 > MLP_LDS_MAX) return lds4 <= MLP_LDS_MAX;
+    const int64_t n4 = num_cus() * mlp_resident(lds4, 3), n8 = num_cus() * mlp_resident(lds8, 2);
+    return (ntiles + n4 - 1) / n4 * (150 + mlp_row(nin)) <= (ntiles + n8 - 1) / n8 * 150;
 }
 
 }  // namespace pxff
@@ -631,27 +852,32 @@ extern "C" int pxff_mlp_energy_grad(int64_t natoms, int nin, int nelem, const in
                                  (size_t)zpn * MLP_ZP + wmax);
     };
     int zpn = MLP_WV;
-    if (lds_of(zpn) > 160 * 1024 - 1024) zpn = mlp_r16(hw) / 16;
+    if (lds_of(zpn) > MLP_LDS_MAX) zpn = mlp_r16(hw) / 16;
     const size_t ldsm = lds_of(zpn);
+    const size_t lds4 =
+        sizeof(double) * (MLP_TILE * ((size_t)mlp_row(nin) + 2 * (size_t)nlm * mlp_row(hw)) + wmax);
+    const int64_t ntiles = div_up(natoms, MLP_TILE);
+    if (mlp_four_waves(ntiles, nin, ldsm, lds4)) {
+        static std::atomic<int> dyn_max{65536};
+        int rc4 = mlp_raise_lds((const void *)mlp_mfma4_kernel, (int)lds4, dyn_max);
+        if (rc4) return rc4;
+        // persistent: as many workgroups as the LDS keeps resident (at most
+        // 8 per CU), each over a contiguous range of 16-atom tiles
+        const int64_t nwg = std::min<int64_t>(ntiles, (int64_t)num_cus() * mlp_resident(lds4, 8));
+        mlp_mfma4_kernel<<<(unsigned)nwg, 256, lds4, s>>>(natoms, nin, nelem, d_species, d_layout, d_params, d_dmin,
+                                                          d_scale, d_x, d_e, d_beta, nlm, hw);
+        PXFF_LAUNCH_CHECK();
+        return 0;
+    }
     // above 64 KB (long descriptors, e.g. SO3 6/6: 147 inputs) one workgroup
     // per CU; the kernel's static LDS (a few hundred bytes) comes on top
-    if (ldsm <= 160 * 1024 - 1024) {
-        // dynamic LDS limit set so far; raised under a lock so that
-        // concurrent callers never lower it below what another relies on
-        static std::mutex mfma_attr_mu;
-        static int mfma_dyn_max = 65536;
-        {
-            std::lock_guard<std::mutex> lock(mfma_attr_mu);
-            if ((int)ldsm > mfma_dyn_max) {
-                PXFF_HIP_CHECK(hipFuncSetAttribute((const void *)mlp_mfma_kernel,
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsm));
-                mfma_dyn_max = (int)ldsm;
-            }
-        }
+    if (ldsm <= MLP_LDS_MAX) {
+        static std::atomic<int> dyn_max{65536};
+        int rc8 = mlp_raise_lds((const void *)mlp_mfma_kernel, (int)ldsm, dyn_max);
+        if (rc8) return rc8;
         // persistent: as many workgroups as the LDS keeps resident (at most
         // 4 per CU, two by their registers), each over a contiguous range of 16-atom tiles
-        const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, (int64_t)(160 * 1024) / (int64_t)(ldsm + 1024)));
-        const int64_t nwg = std::min<int64_t>(div_up(natoms, MLP_TILE), (int64_t)num_cus() * per_cu);
+        const int64_t nwg = std::min<int64_t>(ntiles, (int64_t)num_cus() * mlp_resident(ldsm, 4));
         mlp_mfma_kernel<<<(unsigned)nwg, MLP_T, ldsm, s>>>(
             natoms, nin, nelem, d_species, d_layout, d_params, d_dmin, d_scale, d_x, d_e, d_beta, nlm, hw, nbuf, zpn);
         PXFF_LAUNCH_CHECK();

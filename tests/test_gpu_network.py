@@ -136,3 +136,27 @@ def test_network_tile_edges(hidden, nin, n):
         e[7], beta[7] = 0.0, 0.0
     assert rel_err(e.cpu().numpy(), e_ref.cpu().numpy()) < 1e-13
     assert rel_err(beta.cpu().numpy(), g_ref.cpu().numpy()) < 1e-12
+
+
+# more 16-atom tiles than the chip holds at once in eight-wavefront workgroups
+# (512 on 256 CUs): tiles of four wavefronts for short inputs and narrow layers
+@pytest.mark.parametrize("n,nin,hidden,act", [(8193, 30, (30, 30), "Tanh"), (12001, 14, (16,), "Softplus"),
+                                              (12288, 31, (17, 5), "ELU"), (24007, 5, (), "Tanh"),
+                                              (8209, 91, (30, 30), "Sigmoid"), (16384, 91, (30, 30), "Tanh")])
+def test_fused_network_many_tiles(n, nin, hidden, act):
+    """Elements mixed within the tiles and sorted, an atom without a network,
+    a last tile of one atom; tolerances as for few tiles."""
+    rng = np.random.default_rng(n)
+    model = potential.NNPotential(["O", "Si", "C"], nin, hidden, seed=7, activation=act).cuda()
+    x = torch.as_tensor(rng.random((n, nin)), dtype=torch.float64, device="cuda")
+    symbols = rng.choice(["O", "Si", "C"], size=n, p=[0.5, 0.4, 0.1])
+    for order in (np.arange(n), np.argsort(symbols, kind="stable")):
+        sy = list(symbols[order])
+        e_ref, g_ref = _torch_reference(model, x, sy)
+        sp = potential.species_atom(sy, model.elements, "cuda")
+        sp[n // 2] = -1
+        e, beta = model.energy_grad(x, sp)
+        assert torch.isnan(e[n // 2]) and torch.isnan(beta[n // 2]).all()
+        e[n // 2], beta[n // 2] = e_ref[n // 2], g_ref[n // 2]
+        assert rel_err(e.cpu().numpy(), e_ref.cpu().numpy()) < 1e-13
+        assert rel_err(beta.cpu().numpy(), g_ref.cpu().numpy()) < 1e-12
