@@ -61,18 +61,18 @@ static int db_tables(const So4HostTables &t, So4Dev &d) {
     const int nstage = stage[t.ldim - 1] + 1;
     // the levels that hold a block of b
     std::vector<unsigned> lev(nslot, 0u);
-    std::vector<int> level(t.nblk, 0);
     for (int l = 0; l < t.ldim; l++)
-        for (int k = t.blk_level_start[l]; k < t.blk_level_start[l + 1]; k++) {
-            level[k] = l;
+        for (int k = t.blk_level_start[l]; k < t.blk_level_start[l + 1]; k++)
             for (int q = 0; q < 3; q++)
                 if (t.blk_tb[3 * k + q] >= 0) lev[t.blk_tb[3 * k + q]] |= 1u << l;
-        }
     // Components to the places (wavefront, tile, row): a tile costs the union
     // of its components' levels, and the wavefronts wait for each other
     // after every stage, so the cost is the sum over the stages of the
     // busiest wavefront's steps (then the steps of all).  Exchanges while
     // they do not cost more, from the components in order of their levels.
+    // On the host at the first call of a 2J: the steps of every union are
+    // tabulated, and an exchange changes the work of its two tiles only (2J =
+    // 6 / 8 / 10: 0.2 / 1 / 2 ms, 4 / 8 / 10 with every exchange summed anew).
     std::vector<int> place(nslot);
     std::iota(place.begin(), place.end(), 0);
     std::stable_sort(place.begin(), place.end(), [&](int a, int b) { return lev[a] > lev[b]; });
@@ -83,49 +83,78 @@ static int db_tables(const So4HostTables &t, So4Dev &d) {
             for (int q = 0; q < 4; q++) p[((k % nw) * tw + k / nw) * 4 + q] = place[4 * k + q];
         place = p;
     }
-    std::vector<int> work(nw * nstage);
-    auto wave_work = [&](int w) {
-        std::fill(work.begin() + w * nstage, work.begin() + (w + 1) * nstage, 0);
-        for (int k = 0; k < tw; k++) {
-            unsigned m = 0;
-            for (int q = 0; q < 4; q++) m |= lev[place[(w * tw + k) * 4 + q]];
-            for (int l = 0; l < t.ldim; l++)
-                if (m >> l & 1) work[w * nstage + stage[l]] += db_steps(l);
-        }
-    };
-    auto total = [&]() {
-        long peak = 0, sum = 0;
+    // steps[m][s]: of the levels of the set m in stage s
+    std::vector<int> steps((size_t)nstage << t.ldim, 0);
+    for (unsigned m = 1; m < 1u << t.ldim; m++) {
+        const int l = __builtin_ctz(m);
+        for (int s = 0; s < nstage; s++) steps[m * nstage + s] = steps[(m & (m - 1)) * nstage + s];
+        steps[m * nstage + stage[l]] += db_steps(l);
+    }
+    std::vector<unsigned> at(nslot), uni(nw * tw, 0u);  // levels of a place's component, of a tile
+    for (int k = 0; k < nslot; k++) {
+        at[k] = lev[place[k]];
+        uni[k / 4] |= at[k];
+    }
+    std::vector<int> work(8 * nstage, 0);  // [stage][wavefront], the last four unused below 2J = 10
+    long sum = 0;
+    for (int k = 0; k < nw * tw; k++)
         for (int s = 0; s < nstage; s++) {
-            int mx = 0;
-            for (int w = 0; w < nw; w++) {
-                mx = std::max(mx, work[w * nstage + s]);
-                sum += work[w * nstage + s];
-            }
-            peak += mx;
+            work[8 * s + k / tw] += steps[uni[k] * nstage + s];
+            sum += steps[uni[k] * nstage + s];
         }
-        return peak * 4096 + sum;
+    auto peak = [&]() {
+        long p = 0;
+        for (int s = 0; s < nstage; s++) {
+            const int *w = &work[8 * s];
+            p += std::max(std::max(std::max(w[0], w[1]), std::max(w[2], w[3])),
+                          std::max(std::max(w[4], w[5]), std::max(w[6], w[7])));
+        }
+        return p;
     };
-    for (int w = 0; w < nw; w++) wave_work(w);
     uint32_t rnd = 12345u;
     auto next = [&](int n) {
         rnd = rnd * 1664525u + 1013904223u;
         return (int)((rnd >> 8) % (uint32_t)n);
     };
-    long best = total();
-    for (int it = 0; it < 60000; it++) {
-        const int i = next((int)place.size()), j = next((int)place.size());
-        if (i / 4 == j / 4 || lev[place[i]] == lev[place[j]]) continue;
-        std::swap(place[i], place[j]);
-        wave_work(i / (4 * tw));
-        wave_work(j / (4 * tw));
-        const long now = total();
-        if (now <= best) {
-            best = now;
-        } else {
+    auto others = [&](int k) {  // levels of the other three places of k's tile
+        const int b = k & ~3;
+        return at[b + ((k + 1) & 3)] | at[b + ((k + 2) & 3)] | at[b + ((k + 3) & 3)];
+    };
+    long best = peak() * 4096 + sum;
+    // 2J = 8: the last gain is at 30,000 of 32,768; 2J = 10: 40,000 come within 1e-4 of twice as many
+    const int trials = std::min(8 * nslot * nslot, 40000);
+    for (int it = 0; it < trials; it++) {
+        const int i = next(nslot), j = next(nslot), a = i / 4, b = j / 4;
+        if (a == b || at[i] == at[j]) continue;
+        const unsigned ma = others(i) | at[j], mb = others(j) | at[i];
+        if (ma == uni[a] && mb == uni[b]) {  // costs what it did
+            std::swap(at[i], at[j]);
             std::swap(place[i], place[j]);
-            wave_work(i / (4 * tw));
-            wave_work(j / (4 * tw));
+            continue;
         }
+        const int *na = &steps[ma * nstage], *oa = &steps[uni[a] * nstage];
+        const int *nb = &steps[mb * nstage], *ob = &steps[uni[b] * nstage];
+        int *wa = &work[a / tw], *wb = &work[b / tw];
+        long d = 0;
+        for (int s = 0; s < nstage; s++) {
+            wa[8 * s] += na[s] - oa[s];
+            wb[8 * s] += nb[s] - ob[s];
+            d += (na[s] - oa[s]) + (nb[s] - ob[s]);
+        }
+        const long now = peak() * 4096 + sum + d;
+        if (now > best) {
+            for (int s = 0; s < nstage; s++) {
+                wa[8 * s] -= na[s] - oa[s];
+                wb[8 * s] -= nb[s] - ob[s];
+            }
+            continue;
+        }
+        best = now;
+        sum += d;
+        uni[a] = ma;
+        uni[b] = mb;
+        std::swap(at[i], at[j]);
+        std::swap(place[i], place[j]);
     }
     // levels of every tile, then the component of every slot (-1 none)
     std::vector<int> tile, where(t.nb, 0);
