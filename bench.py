@@ -14,6 +14,7 @@ Prints one JSON line (see the keys below).  ``--gpus N`` with N > 1 exits:
 only one GPU's share of the work is measured.
 """
 import argparse
+import gc
 import json
 import os
 import sys
@@ -154,6 +155,31 @@ def gpu_time_ms(fn, reps=5):
     return a.elapsed_time(b) / reps
 
 
+def timed_steps(fn, steps, warmup=1, on_start=None):
+    """(seconds per step, last result, {median, max} host ms per step) of
+    ``steps`` calls after ``warmup`` untimed ones, the GPU waited for on both
+    sides.  A full garbage collection of a process with torch loaded takes 20
+    to 90 ms, several times a timed window of a few steps, and comes with
+    whatever was allocated before (tuning, other workloads): it is due ahead
+    of the warm-up here.  The host time of the slowest step tells a stall from
+    a slow path."""
+    import torch
+    gc.collect()
+    for _ in range(warmup):
+        fn()
+    torch.cuda.synchronize()
+    if on_start:
+        on_start()
+    marks = [time.perf_counter()]
+    for _ in range(steps):
+        out = fn()
+        marks.append(time.perf_counter())
+    torch.cuda.synchronize()
+    t = (time.perf_counter() - marks[0]) / steps
+    host = np.diff(marks) * 1e3
+    return t, out, {"median": float(np.median(host)), "max": float(host.max())}
+
+
 def isolated_kernel_ms(dso4, potential, model, species_atom, nl, cfg, w, reps=5):
     """Mean duration of each pxff kernel of both paths, from reps
     back-to-back launches between two HIP events on the launch stream
@@ -251,18 +277,6 @@ def run_gpu(steps, warmup):
     ktimes = isolated_kernel_ms(dso4, potential, model, species_atom, nl, cfg, w)
     dom = max((k for k in ADJ_KERNELS if k in ktimes), key=ktimes.get)
 
-    def timed(fn, k, wu, on_start=None):
-        for _ in range(wu):
-            fn()
-        torch.cuda.synchronize()
-        if on_start:
-            on_start()
-        t0 = time.perf_counter()
-        for _ in range(k):
-            out = fn()
-        torch.cuda.synchronize()
-        return (time.perf_counter() - t0) / k, out
-
     # timed adjoint steps; HIP events on the launch stream bracket the
     # dominant kernel's launches inside the timed region
     td = Timers()
@@ -271,17 +285,17 @@ def run_gpu(steps, warmup):
     # step calls zb: the Z kernel and the short B row-partial sum)
     name = {"network": "energy_grad", "z": "zb"}.get(dom, dom)
     td.wrap(owner, [name])
-    t_adj, out_a = timed(step_adjoint, steps, warmup, on_start=td.acc.clear)
+    t_adj, out_a, host_adj = timed_steps(step_adjoint, steps, warmup, on_start=td.acc.clear)
     dom_ms = td.summary()[name]
     td.unwrap(owner, [name])
     # the same E+F step captured once as a HIP graph and replayed; every
     # replay waits for its image count (the capacity check), as an MD
     # driver would before using the forces
     gstep = potential.FusedEFGraph(builder, cfg, (w, w), model, species_atom, pos_dev)
-    t_graph, out_gr = timed(gstep, steps, warmup)
+    t_graph, out_gr, _ = timed_steps(gstep, steps, warmup)
     out_gr = {k: v.clone() for k, v in out_gr.items()}
-    t_pl, out_p = timed(step_plain, max(1, steps), max(1, warmup))
-    t_ag, out_g = timed(step_adjoint_autograd, max(1, steps), max(1, warmup))
+    t_pl, out_p, host_pl = timed_steps(step_plain, max(1, steps), max(1, warmup))
+    t_ag, out_g, _ = timed_steps(step_adjoint_autograd, max(1, steps), max(1, warmup))
     ferr = float(torch.linalg.norm(out_a["forces"] - out_p["forces"]) / torch.linalg.norm(out_p["forces"]))
     ferr_ag = float(torch.linalg.norm(out_g["forces"] - out_a["forces"]) / torch.linalg.norm(out_a["forces"]))
     ferr_graph = float((out_gr["forces"] - out_a["forces"]).abs().max())
@@ -296,7 +310,7 @@ def run_gpu(steps, warmup):
         tnl.append(time.perf_counter() - t0)
     kmean = nl.nimg / n
     return dict(n=n, t_adj=t_adj, t_graph=t_graph, ferr_graph=ferr_graph, t_plain=t_pl, t_autograd=t_ag, ferr=ferr,
-                ferr_autograd=ferr_ag, ktimes=ktimes,
+                ferr_autograd=ferr_ag, host_adj=host_adj, host_plain=host_pl, ktimes=ktimes,
                 dom=dom, dom_ms=dom_ms,
                 t_nlist=float(np.median(tnl)), nimg=nl.nimg, nrows=nl.nrows, kmean=kmean, tuned=tuned)
 
@@ -318,13 +332,7 @@ def run_batched(steps=3):
         b.nl = b.builder.build(b.pos)
         d.state.nl = b.nl
         return bt.energy_forces_virial(d, model, sp)
-    step()
-    torch.cuda.synchronize()
-    t0 = time.perf_counter()
-    for _ in range(steps):
-        step()
-    torch.cuda.synchronize()
-    t = (time.perf_counter() - t0) / steps
+    t = timed_steps(step, steps)[0]
     return {"structures": b.nstruct, "atoms": b.natoms, "images": b.nl.nimg, "ms_per_step": t * 1e3,
             "atom_env_per_s": b.natoms / t}
 
@@ -354,14 +362,14 @@ def run_training(steps=10):
         if mode.startswith("materialized"):
             out["dxdr_rows"] = int(tr.dx.shape[0])
             out["dxdr_bytes"] = int(tr.dx.numel() * 8)
-        l0 = float(tr.step())
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(steps):
-            tr.step()
-        torch.cuda.synchronize()
-        out[mode + "_ms_per_step"] = (time.perf_counter() - t0) / steps * 1e3
-        out[mode + "_loss_first_last"] = [l0, float(tr.step())]
+        first = []
+
+        def step():
+            loss = tr.step()
+            if not first:  # the warm-up step
+                first.append(float(loss))
+        out[mode + "_ms_per_step"] = timed_steps(step, steps)[0] * 1e3
+        out[mode + "_loss_first_last"] = [first[0], float(tr.step())]
         del tr
     return out
 
@@ -443,19 +451,10 @@ def run_so3_sio2(steps=5):
         d.state.nl = b.nl
         return bt.energy_forces_virial(d, model, sp, virial=False)
 
-    def timed(fn, k):
-        fn()
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(k):
-            out = fn()
-        torch.cuda.synchronize()
-        return (time.perf_counter() - t0) / k, out
-
-    t_fused, o_f = timed(fused, steps)
+    t_fused, o_f, _ = timed_steps(fused, steps)
     g = potential.FusedEFGraph(builder, cfg, (z,), model, spa, pos)
-    t_graph, o_g = timed(g, steps)
-    t_ag, o_a = timed(autograd, max(1, steps // 2))
+    t_graph, o_g, _ = timed_steps(g, steps)
+    t_ag, o_a, _ = timed_steps(autograd, max(1, steps // 2))
     ferr = float(torch.linalg.norm(o_a["forces"] - o_f["forces"]) / torch.linalg.norm(o_f["forces"]))
     geq = bool(torch.equal(o_g["forces"], o_f["forces"]))
     # per-kernel durations, each launched back to back on the same inputs
@@ -627,6 +626,7 @@ def main():
                    "adjoint_over_plain": adj_rate / plain_rate, "force_rel_diff_adjoint_vs_plain": r["ferr"],
                    "adjoint_autograd_ms_per_step": r["t_autograd"] * 1e3,
                    "force_rel_diff_autograd_vs_fused": r["ferr_autograd"],
+                   "host_ms_per_step": {"adjoint": r["host_adj"], "plain": r["host_plain"]},
                    "nlist_ms": r["t_nlist"] * 1e3, "kernel_ms_isolated": kt, "tuned": r["tuned"], **extra},
         "roofline": {"bound": "valu", "kernel": KERNEL_SYMBOL[dom],
                      "achieved": achieved / 1e12 if achieved else None, "peak": PEAK_FP64 / 1e12,
