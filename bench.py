@@ -116,12 +116,13 @@ class Timers:
 
 ADJ_KERNELS = ("ui", "z", "bi", "network", "yi", "deidrj", "gather")
 PLAIN_KERNELS = ("dbdr", "rows", "dxdr_contract")
-# Python wrapper -> the one kernel it launches (rocprof names)
-KERNEL_SYMBOL = {"ui": "so4_accum_kernel", "z": "so4_z_tile_kernel", "bi": "so4_b_kernel",
+# Python wrapper -> the kernels it launches at 4096 atoms (rocprof names)
+KERNEL_SYMBOL = {"ui": "so4_stage_kernel+so4_utot_group_kernel", "z": "so4_z_tile_kernel", "bi": "so4_b_kernel",
                  "zb": "so4_z_tile_kernel+so4_brow_sum_kernel",
-                 "network": "mlp_energy_grad_kernel", "yi": "so4_yi_kernel",
+                 "network": "mlp_mfma_kernel", "yi": "so4_yi_kernel",
                  "deidrj": "so4_deidrj_kernel", "gather": "so4_gather_kernel",
-                 "dbdr": "so4_dbdr_centre_kernel", "dbdr_atom_major_z": "so4_z_atom_major_kernel+so4_dbdr_centre_kernel",
+                 "dbdr": "so4_dbdr_centre_kernel+so4_dbdr_rest_kernel",
+                 "dbdr_atom_major_z": "so4_z_atom_major_kernel+so4_dbdr_centre_kernel+so4_dbdr_rest_kernel",
                  "rows": "so4_rows_kernel", "dxdr_contract": "dxdr_contract_kernel"}
 
 
@@ -389,19 +390,24 @@ def so3_flops(nmax, lmax):
 
 
 def so3_expansion_bytes(nimg, natoms, nmax, lmax):
-    """Algorithmic HBM bytes of the SO3 expansion with the radial store: the
-    (lmax + 1) 2 nmax doubles of every image's radial row written once and
-    read once, the separations read by both kernels, the neighbour index and
-    the reverse image (int64 each), and the per-centre expansion written
-    (nmax (lmax + 1) (2 lmax + 1) complex doubles per centre)."""
+    """Algorithmic HBM bytes of the SO3 expansion with the radial store and
+    the power spectrum: the (lmax + 1) 2 nmax doubles of every image's radial
+    row written once, the integrals (half of them) read once, the separations
+    read by both kernels, the neighbour index and the reverse image (int64
+    each), and per centre the m >= 0 half of the expansion (nmax (lmax + 1)
+    (lmax + 2) / 2 complex doubles) and the power spectrum written."""
     nf = (lmax + 1) * 2 * nmax
-    return nimg * (2 * nf * 8 + 2 * 3 * 8 + 2 * 8) + natoms * nmax * (lmax + 1) * (2 * lmax + 1) * 16
+    ncoef = nmax * (nmax + 1) // 2 * (lmax + 1)
+    return (nimg * (nf * 8 + nf * 4 + 2 * 3 * 8 + 2 * 8) +
+            natoms * (nmax * (lmax + 1) * (lmax + 2) // 2 * 16 + ncoef * 8))
 
 
+# the kernels of the fused step, as rocprof names them (12,000 atoms: the
+# sorted form of the radial store)
 SO3_KERNELS = {"expansion": "so3_rbin_hist_kernel+so3_rbin_scan_kernel+so3_rbin_fill_kernel+"
-                            "so3_radial_tab_kernel+so3_ctot_lm_kernel",
-               "power": "so3_power_kernel", "network": "mlp_mfma_kernel", "adjoint_a": "so3_adj_a_kernel",
-               "deidrj": "so3_deidrj_lm_kernel", "forces_energy": "so4_gather_kernel"}
+                            "so3_radial_tab_kernel+so3_expand_kernel",
+               "network": "mlp_mfma_kernel", "adjoint_a": "so3_adj_a_half_kernel",
+               "deidrj": "so3_deidrj_half_kernel", "forces_energy": "so4_gather_kernel"}
 
 
 def committed_traffic_sum(symbols):
@@ -465,16 +471,16 @@ def run_so3_sio2(steps=5):
         return gpu_time_ms(fn, reps)
 
     kt = {}
-    x, ct, rad = dso3.forward(nl, cfg, z, radial=True)
-    # the expansion: radial integrals once per image pair, then the per-centre sums
-    kt["expansion"] = t(lambda: dso3.ctot(nl, cfg, z, radial=True))
-    kt["power"] = t(lambda: dso3.power(nl, cfg, ct))
+    x, ct, rad = dso3.forward_half(nl, cfg, z)
+    # the expansion: radial integrals once per image pair, then the per-centre
+    # sums with the power spectrum
+    kt["expansion"] = t(lambda: dso3.forward_half(nl, cfg, z))
     e, beta = model.energy_grad(x, spa)
     kt["network"] = t(lambda: model.energy_grad(x, spa))
-    A = dso3.adjoint_a(nl, cfg, ct, beta)
-    kt["adjoint_a"] = t(lambda: dso3.adjoint_a(nl, cfg, ct, beta))
-    kt["deidrj"] = t(lambda: dso3.deidrj(nl, cfg, z, A, radial=rad))
-    dedr = dso3.deidrj(nl, cfg, z, A, radial=rad)
+    kt["adjoint_a"] = t(lambda: dso3.adjoint_half(nl, cfg, z, ct, beta, rad))
+    sweep = dso3.adjoint_half(nl, cfg, z, ct, beta, rad)
+    kt["deidrj"] = t(sweep)
+    dedr = sweep()
     kt["forces_energy"] = t(lambda: dso4.forces_energy(nl, dedr, e))
     fl = so3_flops(6, 6)
     # the expansion (tabulated radial integrals, then the per-centre sums) is
@@ -631,7 +637,7 @@ def main():
         "roofline": {"bound": "valu", "kernel": KERNEL_SYMBOL[dom],
                      "achieved": achieved / 1e12 if achieved else None, "peak": PEAK_FP64 / 1e12,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP64 if achieved else None,
-                     "traffic": committed_traffic(KERNEL_SYMBOL[dom]),
+                     "traffic": committed_traffic_sum(KERNEL_SYMBOL[dom]),
                      "kernel_ms_timed_region": r["dom_ms"],
                      "flops_per_launch": alg,
                      "note": "FP64 vector ALU roof (no MFMA; MI355X FP64 vector peak = FP64 matrix peak)"},
