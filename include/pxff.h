@@ -34,8 +34,8 @@ extern "C" {
 #define PXFF_ENOTIMPL -3 /* unsupported parameter (e.g. odd 2J) */
 
 /* Launch-parameter knobs (process-wide), set by the autotuner:
- *   PXFF_TUNE_Z_CHUNKS              Z rows split into at least this many wavefront chunks per 64-atom tile
- *                                   (1..256; the launch takes more by a rule on 2J and the atoms)
+ *   PXFF_TUNE_Z_CHUNKS              Z rows split into this many wavefront chunks per 64-atom tile (1..256),
+ *                                   0 (default) by a rule on 2J and the atoms (pxff_so4_z_chunks)
  *   PXFF_TUNE_ACCUM_WAVES_PER_CU    persistent grid of the per-centre kernels = CUs x this (1..256)
  *   PXFF_TUNE_IMAGE_WAVES_PER_BLOCK wavefronts per workgroup of the per-image adjoint kernel (1, 2, 4)
  *   PXFF_TUNE_ACCUM_LDSADD          per-centre U_tot sums: 0 = per-group LDS partials, 1 = one LDS array
@@ -249,6 +249,10 @@ int pxff_so4_ui_staged(const pxff_so4_params *p, int64_t natoms, const int64_t *
  * NULL). */
 int pxff_so4_zb(const pxff_so4_params *p, int64_t natoms, const double *d_utot, double *d_z, double *d_b,
                 void *stream);
+
+/* Chunks per 64-atom tile that pxff_so4_zb takes for natoms atoms as the knob
+ * stands (a host-side query; at most one per row group of the 2J). */
+int pxff_so4_z_chunks(const pxff_so4_params *p, int64_t natoms, int *chunks);
 
 /* Length in doubles of the d_z buffer of pxff_so4_zb for natoms atoms. */
 int pxff_so4_zlen(int twol, int64_t natoms, int64_t *len);

@@ -1,7 +1,8 @@
 """Autotuner for the launch parameters of the hot kernels.
 
 Knobs (``pxff_tune_set``, include/pxff.h):
-  * least Z-row chunks per 64-atom tile of the Z kernel (wavefronts per tile),
+  * Z-row chunks per 64-atom tile of the Z kernel (wavefronts per tile; 0: the
+    launch's own rule),
   * persistent-grid size of the per-centre kernels (wavefronts per CU),
   * how the per-centre kernels sum over images (register sums reduced once
     per centre, per-group LDS partials, LDS atomic adds, or LDS partials
@@ -21,8 +22,7 @@ from . import _native as nat
 from . import so4 as dso4
 
 Z_CHUNKS, ACCUM_WAVES_PER_CU, IMAGE_WAVES_PER_BLOCK, ACCUM_LDSADD = 0, 1, 2, 3
-# (the Z kernel takes at least its own rule's chunks: 16 stands for the rule)
-CANDIDATES = {Z_CHUNKS: (16, 64, 112), ACCUM_WAVES_PER_CU: (4, 8, 16, 32, 64),
+CANDIDATES = {Z_CHUNKS: (0, 16, 48, 64, 112), ACCUM_WAVES_PER_CU: (4, 8, 16, 32, 64),
               IMAGE_WAVES_PER_BLOCK: (1, 2, 4), ACCUM_LDSADD: (4, 0, 1, 2, 3)}
 CACHE = os.path.join(os.path.expanduser("~"), ".cache", "pyxtal_ff_amd", "tune.json")
 
@@ -73,7 +73,8 @@ def _save_cache(c):
 
 def tune_so4(nl, cfg, atom_w, site_w, work_order=None, use_cache=True, verbose=False):
     """Pick the three knobs for this SO4 workload; returns {knob: value}."""
-    key = "so4:2J=%d:atoms=%d:images=%d" % (cfg.twol, _bucket(nl.natoms), _bucket(nl.nimg))
+    # (z0: entries from before Z_CHUNKS 0 stood for the rule are not used)
+    key = "so4:z0:2J=%d:atoms=%d:images=%d" % (cfg.twol, _bucket(nl.natoms), _bucket(nl.nimg))
     cache = _load_cache() if use_cache else {}
     if key in cache:
         best = {int(k): v for k, v in cache[key].items()}

@@ -2405,8 +2405,8 @@ namespace pxff {
 // Atomic: a call reads each knob once when it launches, so calls from
 // several host threads and streams never race with a concurrent set (a set
 // affects the launches that start after it).
-static std::atomic<int> g_tune[PXFF_TUNE_COUNT] = {16, 16, 4, 4};
-static const int g_tune_lo[PXFF_TUNE_COUNT] = {1, 1, 1, 0};
+static std::atomic<int> g_tune[PXFF_TUNE_COUNT] = {0, 16, 4, 4};
+static const int g_tune_lo[PXFF_TUNE_COUNT] = {0, 1, 1, 0};
 static const int g_tune_hi[PXFF_TUNE_COUNT] = {256, 256, 4, 4};
 int tune_value(int knob) { return g_tune[knob].load(std::memory_order_relaxed); }
 

@@ -25,12 +25,16 @@ namespace pxff {
 // 80 (48 is the one resident round of 12 wavefronts per CU there), 512 tiles
 // 584 / 476 / 500; 2J = 6, 16 tiles 38 / 20 / 20, 64 tiles 48 / 28 / 31.  At
 // 2J = 10 the groups are four times as long: 128 chunks at every size (64
-// tiles 345 / 272 / 236, 1 tile 306 / 144 / 74).  The tuning knob can raise
-// the count, not lower it.
+// tiles 345 / 272 / 236, 1 tile 306 / 144 / 74).  The tuning knob, where
+// set, gives the count instead.
 constexpr int ZCH_SMALL_TILES = 24;
 static int zchunk_rule(int twol, int ntiles) {
     if (twol >= 10) return 128;
     return ntiles <= ZCH_SMALL_TILES ? 112 : 48;
+}
+static int zchunks(int twol, int ntiles, int nzgroups) {
+    const int set = tune_value(PXFF_TUNE_Z_CHUNKS);
+    return std::min(set > 0 ? set : zchunk_rule(twol, ntiles), nzgroups);
 }
 
 // Z-group chunk tables per (device, 2J, normalisation, nchunks).  The first
@@ -369,7 +373,7 @@ extern "C" int pxff_so4_zb(const pxff_so4_params *p, int64_t natoms, const doubl
     if ((rc = get_so4_tables(p->twol, p->normalize_u, &T))) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int ntiles = (int)((natoms + 63) / 64);
-    const int nch = std::min(std::max(tune_value(PXFF_TUNE_Z_CHUNKS), zchunk_rule(p->twol, ntiles)), T->nzgroups);
+    const int nch = zchunks(p->twol, ntiles, T->nzgroups);
     const int *zch = nullptr;
     if ((rc = get_zchunks(p->twol, p->normalize_u, nch, T->nzgroups, &zch))) return rc;
     const int grid = 8 * ((ntiles + 7) / 8) * ((nch + 3) / 4);
@@ -405,3 +409,15 @@ extern "C" int pxff_so4_zlen(int twol, int64_t natoms, int64_t *len) {
     return 0;
 }
 
+extern "C" int pxff_so4_z_chunks(const pxff_so4_params *p, int64_t natoms, int *chunks) {
+    int rc = so4_check_params(p);
+    if (rc) return rc;
+    PXFF_REQUIRE(natoms >= 0 && chunks != nullptr, "null output or negative size");
+    So4HostTables t;
+    if (!build_so4_tables(p->twol, p->normalize_u, t)) {
+        set_error("unsupported 2J");
+        return PXFF_ENOTIMPL;
+    }
+    *chunks = zchunks(p->twol, (int)std::min<int64_t>((natoms + 63) / 64, 1 << 30), t.nzgroups);
+    return 0;
+}

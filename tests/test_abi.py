@@ -94,3 +94,31 @@ def test_workspace_sizes_without_gpu():
     assert b.value == 1000 * 6 * 8
     assert L.pxff_workspace_size(9, None, 0, 0, ctypes.byref(b)) != 0
     assert "workspace kind" in _native.last_error()
+
+
+def test_z_chunk_knob_is_taken_as_set():
+    """Z chunks per tile: 0 (the default) leaves them to the rule, any other
+    value is what the Z kernel takes, up to one chunk per row group."""
+    from pyxtal_ff_amd import _native
+    L = _native.load()
+    c = ctypes.c_int()
+
+    def chunks(twol, natoms):
+        p = _native.So4Params(twol, 4.9, 0.99363, 1, 0)
+        assert L.pxff_so4_z_chunks(ctypes.byref(p), natoms, ctypes.byref(c)) == 0
+        return c.value
+
+    old = L.pxff_tune_get(0)
+    assert old == 0
+    rule = {(t, n): chunks(t, n) for t in (2, 6, 8, 10) for n in (1, 64, 1000, 4096, 136000)}
+    assert all(v >= 1 for v in rule.values())
+    try:
+        for v in (1, 16, 48, 112, 256):
+            assert L.pxff_tune_set(0, v) == 0
+            for n in (1, 1000, 136000):
+                assert chunks(8, n) == min(v, 175)  # 175 row groups
+            assert chunks(2, 64) <= v
+        assert L.pxff_tune_set(0, 257) != 0 and L.pxff_tune_set(0, -1) != 0
+    finally:
+        L.pxff_tune_set(0, old)
+    assert rule == {(t, n): chunks(t, n) for t, n in rule}
