@@ -125,7 +125,8 @@ class PyXtalFFCalculator(_Base):
         host = torch.cat([o["energy"].view(1), o["virial"].view(9), o["atom_energies"],
                           o["forces"].reshape(-1)]).cpu().numpy()
         w = host[1:10].reshape(1, 3, 3)
-        sv = (-w[:, bt.VOIGT[0], bt.VOIGT[1]] * (1.0 / self._sb.volumes)[:, None])[0]  # eV/A^3, (xx, yy, zz, xy, xz, yz)
+        with np.errstate(divide="ignore", invalid="ignore"):  # a cluster's zero cell has no stress
+            sv = (-w[:, bt.VOIGT[0], bt.VOIGT[1]] * (1.0 / self._sb.volumes)[:, None])[0]  # eV/A^3, (xx, yy, zz, xy, xz, yz)
         stress_ml = sv * EV2GPA
         self.results["energies"] = host[10: 10 + n].copy()
         self.results["energy"] = float(host[0])

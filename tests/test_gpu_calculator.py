@@ -81,3 +81,25 @@ def test_calculator_reuses_metadata_and_tracks_positions():
             es.append(calc.get_potential_energy(s2))
         assert calc._key == key
         assert abs(-(es[0] - es[1]) / (2 * h) - f[a, c]) < 1e-6 * max(1.0, abs(f[a, c]))
+
+
+def test_cluster_without_a_cell_computes_silently():
+    """Energies and forces of a cluster whose cell is zero; its stress has no
+    volume (not finite), which a later call does not warn about."""
+    import warnings
+    from pyxtal_ff_amd import potential
+    from pyxtal_ff_amd.calculator import PyXtalFFCalculator
+    from pyxtal_ff_amd.structure import Structure
+    pos = np.random.default_rng(1).uniform(0.0, 5.0, (9, 3))
+    s = Structure(pos, np.zeros((3, 3)), symbols=["Si"] * 9, pbc=False)
+    f = {"type": "SO4", "Rc": 4.2, "parameters": {"lmax": 2}, "cutoff": "cosine"}
+    calc = PyXtalFFCalculator(f, potential.NNPotential(["Si"], 14, (7, 5), seed=2))
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # the structure's own inverse volume
+        calc.calculate(s)
+    s.positions = pos + 0.01
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        calc.calculate(s)
+    assert np.isfinite(calc.results["energy"]) and np.isfinite(calc.results["forces"]).all()
+    assert not np.isfinite(calc.results["stress"]).any()
