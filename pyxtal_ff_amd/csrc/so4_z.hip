@@ -16,18 +16,19 @@
 
 namespace pxff {
 
-// Row-group chunks per 64-atom tile (one wavefront each).  A wavefront runs
-// its chunk alone, so few chunks leave one long serial chain per wavefront
-// and, below some thousand atoms, most of the chip idle; more chunks than
-// keep the wavefronts resident only add partly filled rounds.  Measured, us
-// for Z and the B row partials, at 16 / 48 / 112 chunks: 2J = 8, 1 tile 107 /
-// 39 / 29, 13 tiles 123 / 46 / 37, 27 tiles 128 / 50 / 47, 64 tiles 129 / 66 /
-// 80 (48 is the one resident round of 12 wavefronts per CU there), 512 tiles
-// 584 / 476 / 500; 2J = 6, 16 tiles 38 / 20 / 20, 64 tiles 48 / 28 / 31.  At
+// Row-group chunks per 64-atom tile (one wavefront each), where the tuning
+// knob does not give them.  A wavefront runs its chunk alone, so few chunks
+// leave one long serial chain per wavefront and, below some thousand atoms,
+// most of the chip idle; more chunks than keep the wavefronts resident only
+// add partly filled rounds.  Measured, us for Z and the B row sums, at 16 / 48
+// / 112 chunks: 2J = 8, 8 tiles 107 / 47 / 33, 16 121 / 57 / 39, 24 125 / 60 /
+// 42, 27 126 / 60 / 51, 30 125 / 60 / 52, 34 125 / 60 / 61, 40 125 / 61 / 64,
+// 64 126 / 69 / 80 (48 is the one resident round of 12 wavefronts per CU
+// there), 96 140 / 107 / 106; 2J = 6, 16 tiles 38 / 20 / 20, 30 41 / 23 / 22,
+// 64 48 / 26 / 30.  The line is at four tiles to each of the eight XCDs.  At
 // 2J = 10 the groups are four times as long: 128 chunks at every size (64
-// tiles 345 / 272 / 236, 1 tile 306 / 144 / 74).  The tuning knob, where
-// set, gives the count instead.
-constexpr int ZCH_SMALL_TILES = 24;
+// tiles 345 / 272 / 236, 1 tile 306 / 144 / 74).
+constexpr int ZCH_SMALL_TILES = 32;
 static int zchunk_rule(int twol, int ntiles) {
     if (twol >= 10) return 128;
     return ntiles <= ZCH_SMALL_TILES ? 112 : 48;
