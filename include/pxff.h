@@ -68,6 +68,9 @@ int pxff_tune_get(int knob); /* -1 for an unknown knob */
  *   PXFF_WS_SO4_UI       d_stage of pxff_so4_ui_staged, n1 = image capacity
  *   PXFF_WS_NLIST_SLOTS  the slot arrays of pxff_nlist_count_slots / _fill_slots
  *                        (44 bytes per slot entry), n0 = natoms, n1 = slot
+ *   PXFF_WS_SO4_TANGENT_STAGE  d_stage of pxff_so4_tangent_staged, n1 = image capacity
+ *   PXFF_WS_NLIST_BINNED d_bin_pos and d_bin_tag of pxff_nlist_count_binned
+ *                        (24 and 16 bytes per atom), n0 = natoms
  * The launch knobs below are the only other state: process-wide atomics
  * read once per launch, so calls on several threads and streams are
  * reentrant. */
@@ -78,6 +81,8 @@ int pxff_tune_get(int knob); /* -1 for an unknown knob */
 #define PXFF_WS_SO3_TABLE 4
 #define PXFF_WS_SO4_UI 5
 #define PXFF_WS_NLIST_SLOTS 6
+#define PXFF_WS_SO4_TANGENT_STAGE 7
+#define PXFF_WS_NLIST_BINNED 8
 int pxff_workspace_size(int kind, const void *params, int64_t n0, int64_t n1, int64_t *bytes);
 
 /* Copy the calling thread's last error message into buf (NUL-terminated). */
@@ -223,7 +228,8 @@ int pxff_so4_sizes(int twol, int *nu, int *nhalf, int *nz, int *nb);
  *   d_img_start [natoms+1], d_img_j [nimg], d_img_r [nimg*3]; d_atom_w
  *   [natoms] = neighbour weight of each atom (pair weight of image = w[j]);
  *   d_site_w [natoms] = self weight.  d_work_order [natoms] int64 or NULL:
- *   centres in the order they are scheduled (neighbour-count sorted). */
+ *   centres in the order they are scheduled (neighbour-count sorted); it
+ *   changes no value. */
 int pxff_so4_ui(const pxff_so4_params *p, int64_t natoms, const int64_t *d_img_start, const int64_t *d_img_j,
                 const double *d_img_r, const double *d_atom_w, const double *d_site_w,
                 const int64_t *d_work_order, double *d_utot, void *stream);
@@ -236,7 +242,10 @@ int pxff_so4_ui(const pxff_so4_params *p, int64_t natoms, const int64_t *d_img_s
  * between its sweeps (same construction as pxff_so4_ui, SNAP.py:1480-1500;
  * equal to it to rounding).  cap must be at least the image count.  With
  * a summation mode other than the register sums (pxff_tune_set
- * PXFF_TUNE_ACCUM_LDSADD != 4) or 2J > 8 it is pxff_so4_ui. */
+ * PXFF_TUNE_ACCUM_LDSADD != 4) or 2J > 8 it is pxff_so4_ui.  Long lists (four
+ * centres per SIMD and more: 4096 atoms on 256 CUs) take several centres per
+ * wavefront, in their own order: d_work_order and
+ * PXFF_TUNE_ACCUM_WAVES_PER_CU have no effect there. */
 int pxff_so4_ui_staged(const pxff_so4_params *p, int64_t natoms, const int64_t *d_img_start, const int64_t *d_img_j,
                        const double *d_img_r, const double *d_atom_w, const double *d_site_w,
                        const int64_t *d_work_order, int64_t cap, double *d_stage, double *d_utot, void *stream);

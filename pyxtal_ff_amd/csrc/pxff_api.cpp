@@ -57,6 +57,13 @@ extern "C" int pxff_workspace_size(int kind, const void *params, int64_t n0, int
     case PXFF_WS_SO4_UI:
         *bytes = 8 * 6 * n1;
         return 0;
+    case PXFF_WS_SO4_TANGENT_STAGE:
+        *bytes = 8 * 10 * n1;
+        return 0;
+    case PXFF_WS_NLIST_BINNED:
+        // d_bin_pos 3 x double, d_bin_tag 4 x int32 per atom
+        *bytes = (24 + 16) * n0;
+        return 0;
     case PXFF_WS_SO3_TABLE: {
         PXFF_REQUIRE(params != nullptr, "null params");
         int nk = 0;

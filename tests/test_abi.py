@@ -122,3 +122,15 @@ def test_z_chunk_knob_is_taken_as_set():
     finally:
         L.pxff_tune_set(0, old)
     assert rule == {(t, n): chunks(t, n) for t, n in rule}
+
+
+def test_workspace_sizes_of_staged_tangent_and_binned_count():
+    from pyxtal_ff_amd import _native
+    L = _native.load()
+    b = ctypes.c_int64()
+    # ten doubles per image of the capacity
+    assert L.pxff_workspace_size(7, None, 0, 1001, ctypes.byref(b)) == 0
+    assert b.value == 1001 * 10 * 8
+    # position 3 x double, index and wrap 4 x int32 per atom
+    assert L.pxff_workspace_size(8, None, 4097, 0, ctypes.byref(b)) == 0
+    assert b.value == 4097 * (3 * 8 + 4 * 4)
