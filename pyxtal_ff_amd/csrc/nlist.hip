@@ -513,7 +513,7 @@ __global__ void nl_row_rev_kernel(int64_t nrows, const int64_t *__restrict__ seq
 // fill pass ranks the list by (j, T) (rank = number of smaller keys) and
 // writes it in order.  Centres with more than NL_KMAX images are filled by
 // one lane of their wavefront (nl_fill_serial).
-constexpr int NL_KMAX = 128;  // 7 KB of LDS per centre: many resident wavefronts
+constexpr int NL_KMAX = 128;  // 6.4 KB of LDS per centre: many resident wavefronts
 
 struct NlHit {
     int32_t j, T[3];

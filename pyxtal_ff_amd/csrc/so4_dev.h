@@ -27,7 +27,6 @@ struct So4Dev {
     int *zgroups;
     int nbrow;        // B row partials per atom
     int *b_brow0;     // [nb] first B row partial of b
-    int zlevel_max;   // largest level of Z blocks: sum of its blocks' half-row entries
     // matrix-core dB/dr: levels of each tile and component of each slot
     // (tile * 4 + row), LDS row and factor per (level,
     // slot), generator coefficients, Z elements in level order, first Z
@@ -55,21 +54,6 @@ __host__ __device__ constexpr int nhalf_of(int twoj) {
     for (int l = 0; l <= twoj; l++) s += (l / 2 + 1) * (l + 1);
     return s;
 }
-// Half-row entries of the largest level of Z blocks: sum over the blocks
-// (l1, l2, l) of level l (l1 >= l2, |l1 - l2| <= l <= l1 + l2, l1 + l2 - l
-// even) of (l/2 + 1)(l + 1), maximised over l.
-__host__ __device__ constexpr int zlevel_max_of(int twoj) {
-    int best = 0;
-    for (int l = 0; l <= twoj; l++) {
-        int nbl = 0;
-        for (int l1 = 0; l1 <= twoj; l1++)
-            for (int l2 = 0; l2 <= l1; l2++)
-                if (l >= l1 - l2 && l <= l1 + l2 && ((l1 + l2 - l) & 1) == 0) nbl++;
-        const int n = nbl * (l / 2 + 1) * (l + 1);
-        if (n > best) best = n;
-    }
-    return best;
-}
 // Compile-time loop: f(std::integral_constant<int, 0>) ... f(<N-1>).
 template <typename F, int... I>
 __device__ inline void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
@@ -80,18 +64,13 @@ __device__ inline void static_for(F &&f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// Blocks of level l, and the most of one level.
+// Blocks (l1, l2, l) of level l.
 __host__ __device__ constexpr int nblk_level(int twoj, int l) {
     int nbl = 0;
     for (int l1 = 0; l1 <= twoj; l1++)
         for (int l2 = 0; l2 <= l1; l2++)
             if (l >= l1 - l2 && l <= l1 + l2 && ((l1 + l2 - l) & 1) == 0) nbl++;
     return nbl;
-}
-__host__ __device__ constexpr int nblk_level_max(int twoj) {
-    int best = 0;
-    for (int l = 0; l <= twoj; l++) best = nblk_level(twoj, l) > best ? nblk_level(twoj, l) : best;
-    return best;
 }
 // Matrix-core dB/dr.  Wavefronts per workgroup: four, so that two workgroups
 // share a CU; eight at 2J = 10, where six tiles per wavefront would not fit

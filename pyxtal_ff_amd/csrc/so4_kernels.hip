@@ -54,6 +54,14 @@ int upload(const std::vector<T> &v, T **dst) {
 
 // Tables of the matrix-core dB/dr kernel (so4_dbdr_centre_kernel).
 static int db_tables(const So4HostTables &t, So4Dev &d) {
+    // the kernel's LDS is sized at compile time by these counts
+    bool as_compiled = t.nb == nb_of(t.twol);
+    for (int l = 0; l < t.ldim; l++)
+        as_compiled = as_compiled && t.blk_level_start[l + 1] - t.blk_level_start[l] == nblk_level(t.twol, l);
+    if (!as_compiled) {
+        set_error("block counts of the 2J tables differ from those the dB/dr kernel is built for");
+        return PXFF_EINVAL;
+    }
     const int nw = db_waves(t.twol), tw = ((t.nb + 3) / 4 + nw - 1) / nw, nslot = nw * tw * 4;
     // stages: runs of levels whose values share a W row
     std::vector<int> stage(t.ldim, 0);
@@ -291,10 +299,6 @@ int get_so4_tables(int twol, int norm, const So4Dev **out) {
     if ((rc = upload(t.idxu_block, &d.idxu_block))) return rc;
     d.nbrow = t.nbrow;
     if ((rc = upload(t.b_brow0, &d.b_brow0))) return rc;
-    d.zlevel_max = 0;
-    for (int l = 0; l + 1 < (int)t.blk_level_start.size(); l++)
-        d.zlevel_max = std::max(d.zlevel_max,
-                                (t.blk_level_start[l + 1] - t.blk_level_start[l]) * (l / 2 + 1) * (l + 1));
     d.nzgroups = t.nzgroups;
     if ((rc = upload(t.zgroups, &d.zgroups))) return rc;
     // inverse of the block targets: the (block, factor) pairs of each b
@@ -1960,8 +1964,10 @@ __global__ __launch_bounds__(DbDim<TWOJ>::T) __attribute__((amdgpu_waves_per_eu(
     if (n > 0) so4_dbdr_pass<TWOJ>(A, c, s0, (int)(n < NI ? n : NI), dbdr);
 }
 
-// The images past NI of the centres that have more (none in a solid at the
-// usual cutoffs), a persistent grid over the centres, strided so that the
+// The images past NI of the centres that have more (at 2J <= 8, NI = 48, none
+// in a solid at the usual cutoffs; at 2J = 10, NI = 32, those of a dense one:
+// 1728 atoms of 33 images take 735 us where 28 images take 375, which is still
+// below the 1280 of the vector kernel), a persistent grid over the centres, strided so that the
 // centres of a list whose every centre has more are shared out evenly.  The
 // threads look at a centre each before the workgroup goes through them, and
 // one workgroup per CU has the registers to itself: with two, the kernel's
@@ -2806,8 +2812,6 @@ extern "C" int pxff_so4_dbdr_centres(const pxff_so4_params *p, int64_t natoms, c
     if (natoms <= 0) return 0;
     const So4Dev *T = nullptr;
     if ((rc = get_so4_tables(p->twol, p->normalize_u, &T))) return rc;
-    PXFF_REQUIRE(T->zlevel_max <= zlevel_max_of(p->twol) && T->nb <= nb_of(p->twol),
-                 "Z level staging exceeds its LDS bound");
     PXFF_REQUIRE(natoms <= ((int64_t)1 << 31) - 64, "too many atoms for one launch");
     hipStream_t s = (hipStream_t)stream;
     // one workgroup per centre, rounded up to whole 64-centre tiles (the
