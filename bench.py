@@ -120,7 +120,7 @@ PLAIN_KERNELS = ("dbdr", "rows", "dxdr_contract")
 KERNEL_SYMBOL = {"ui": "so4_stage_kernel+so4_utot_group_kernel", "z": "so4_z_tile_kernel", "bi": "so4_b_kernel",
                  "zb": "so4_z_tile_kernel+so4_brow_sum_kernel",
                  "network": "mlp_mfma_kernel", "yi": "so4_yi_kernel",
-                 "deidrj": "so4_deidrj_kernel", "gather": "so4_gather_kernel",
+                 "deidrj": "so4_deidrj_kernel", "gather": "so4_gather_kernel<false>",
                  "dbdr": "so4_dbdr_centre_kernel+so4_dbdr_rest_kernel",
                  "dbdr_atom_major_z": "so4_z_atom_major_kernel+so4_dbdr_centre_kernel+so4_dbdr_rest_kernel",
                  "rows": "so4_rows_kernel", "dxdr_contract": "dxdr_contract_kernel"}
@@ -407,15 +407,15 @@ def so3_expansion_bytes(nimg, natoms, nmax, lmax):
 SO3_KERNELS = {"expansion": "so3_rbin_hist_kernel+so3_rbin_scan_kernel+so3_rbin_fill_kernel+"
                             "so3_radial_tab_kernel+so3_expand_kernel",
                "network": "mlp_mfma_kernel", "adjoint_a": "so3_adj_a_half_kernel",
-               "deidrj": "so3_deidrj_half_kernel", "forces_energy": "so4_gather_kernel"}
+               "deidrj": "so3_deidrj_half_kernel<6,true>", "forces_energy": "so4_gather_kernel<true>"}
 
 
-def committed_traffic_sum(symbols):
+def committed_traffic_sum(symbols, workload):
     """Sum of committed_traffic over '+'-joined kernel names (None if any is
     missing)."""
     tot = 0
     for k in symbols.split("+"):
-        v = committed_traffic(k)
+        v = committed_traffic(k, workload)
         if v is None:
             return None
         tot += v
@@ -497,7 +497,7 @@ def run_so3_sio2(steps=5):
             "force_rel_diff_autograd_vs_fused": ferr, "kernel_ms_isolated": kt,
             "roofline": {"bound": bound, "kernel": SO3_KERNELS[dom], "achieved": ach / scale, "peak": peak / scale,
                          "unit": unit, "frac": ach / peak, "work_per_launch": work,
-                         "traffic": committed_traffic_sum(SO3_KERNELS[dom]),
+                         "traffic": committed_traffic_sum(SO3_KERNELS[dom], "so3"),
                          "kernel_ms_isolated": kt[dom],
                          "reference_work_tflops": ref_flops / (kt["expansion"] * 1e-3) / 1e12,
                          "note": "expansion: algorithmic bytes (bench.so3_expansion_bytes); deidrj: algorithmic "
@@ -553,13 +553,15 @@ def run_cpu_baseline(reps_one=3, reps_all=5):
                           "sample": "same, median of %d runs of %.2f s on 1 thread" % (reps_one, t_one)})
 
 
-def committed_traffic(symbol):
-    """HBM bytes per launch of a kernel on this workload, from the committed
-    rocprofv3 --pmc summary (profiles/*traffic*.md lines
-    'TRAFFIC <kernel> fetch=<bytes> write=<bytes>'), or None."""
+def committed_traffic(symbol, workload):
+    """HBM bytes per launch of a kernel on the workload ("so4": the headline,
+    "so3": the SO3 one), from its committed rocprofv3 --pmc summary
+    (profiles/<workload>*traffic*.md lines
+    'TRAFFIC <kernel> fetch=<bytes> write=<bytes>', with the template
+    arguments where a kernel has several forms), or None."""
     import glob
     import re
-    for path in sorted(glob.glob(os.path.join(ROOT, "profiles", "*traffic*.md"))):
+    for path in sorted(glob.glob(os.path.join(ROOT, "profiles", workload + "*traffic*.md"))):
         with open(path) as f:
             for line in f:
                 m = re.match(r"\s*TRAFFIC\s+(\S+)\s+fetch=(\d+)\s+write=(\d+)", line)
@@ -637,7 +639,7 @@ def main():
         "roofline": {"bound": "valu", "kernel": KERNEL_SYMBOL[dom],
                      "achieved": achieved / 1e12 if achieved else None, "peak": PEAK_FP64 / 1e12,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP64 if achieved else None,
-                     "traffic": committed_traffic_sum(KERNEL_SYMBOL[dom]),
+                     "traffic": committed_traffic_sum(KERNEL_SYMBOL[dom], "so4"),
                      "kernel_ms_timed_region": r["dom_ms"],
                      "flops_per_launch": alg,
                      "note": "FP64 vector ALU roof (no MFMA; MI355X FP64 vector peak = FP64 matrix peak)"},

@@ -1502,15 +1502,15 @@ __device__ __forceinline__ double so3_dpp(double v) {
 // several of them.  One batch per wavefront: in a loop over batches the
 // constants of the cutoff and the exponential are held in registers across
 // it (256 of them and one wavefront per SIMD).
-// 407k images at 6/6: 101 us, 2.7 TB/s of radial rows, two wavefronts per
-// SIMD (120 with a branch around the loads of the second order); 5.8k images
-// at 3/4: 11 us (its forerunner with a lane per (l, m), a Y
+// 407k images at 6/6: 90 us in the step, 3.0 TB/s of radial rows, two
+// wavefronts per SIMD (112 with a branch around the loads of the second
+// order); 5.8k images at 3/4: 11 us (its forerunner with a lane per (l, m), a Y
 // table and 64-lane sums: 215 and 56 us).
 // HALF: A is the m >= 0 half and stands for a full A with the symmetry of the
 // expansion.  Else A is full and any: only A_m + (-1)^m conj(A_-m) enters the
 // sums (A_0's real part), which a lane forms as it loads its orders, without
-// branches around the loads (407k images at 6/6: 104 us, 166 with them).  For
-// an A with the symmetry that is 2 A_m exactly, the same bits.
+// branches around the loads (407k images at 6/6, alone: 104 us, 166 with
+// them).  For an A with the symmetry that is 2 A_m exactly, the same bits.
 constexpr int SO3_AB = 32;  // images per batch, SO3_AB / 4 per row of lanes
 template <int NMAX, bool HALF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NMAX <= 4 ? 3 : 2))) void so3_deidrj_half_kernel(
